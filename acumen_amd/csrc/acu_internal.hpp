@@ -180,21 +180,27 @@ enum RampVariant { RAMP_FP64 = 0, RAMP_FP32 = 1, RAMP_BF16X3 = 2, RAMP_BF16X6 = 
 void launch_ramp(const RFTask* d_tasks, int ntasks, int base, int tiles, int variant, hipStream_t s);
 
 // ---- ramp filter by FFT convolution (fft.hip) ----
-constexpr int FFT_MAX_L = 8192;  // transform length limit (LDS: 8 B per point)
+constexpr int FFT_MAX_L = 8192;  // real transform length limit (LDS: 9 bytes per value)
 struct FFTTask {
-  int N, T, L, lg;     // L = 2^lg = fft_len(N)
-  int block_begin;     // one block per pair of angle rows
+  int N, T, lg;        // transform length L = 2^lg = fft_len(N), M = L/2 complex points
+  int block_begin;     // first global block of this slice (fft_blocks of them)
   int alias;           // L == 2N-2: outputs 0 and N-1 get the correction
   float g_edge;        // tap at distance N-1
-  const float* G;      // L: spectrum of the wrapped kernel, times 1/L
-  const float2* tw;    // L/2: exp(-2 pi i k / L)
+  const float* h;      // 2N+1 taps
+  const double* G;     // M+1: spectrum of the wrapped kernel, times 1/M
+  const double2* tw;   // M/2: exp(-2 pi i k / M), then M/2+1: exp(-2 pi i k / L)
   const float* sino;   // (T, N) in
   float* out;          // (T, N) out
 };
 int fft_len(int N);
 bool fft_supported(int N);
-void fft_tables(int N, const float* taps, float* G, float2* tw);
-void launch_ramp_fft(const FFTTask* d_tasks, int ntasks, int base, int blocks, int maxL, hipStream_t s);
+// threads per workgroup of a launch whose largest slice has side maxN, and
+// the blocks of one slice at that size
+int fft_threads(int maxN);
+int fft_blocks(int N, int T, int threads);
+// G and tw: M + 1 values each, M = fft_len(N) / 2
+void fft_tables(int N, const float* taps, double* G, double2* tw);
+void launch_ramp_fft(const FFTTask* d_tasks, int ntasks, int base, int blocks, int threads, hipStream_t s);
 // refpos: positions in the reference's FP32 arithmetic (default); false:
 // tile-relative positions (closer to FP64, two VALU fewer per update)
 // XCD shares of a backprojection launch over `tiles` tiles: XCD k runs the

@@ -207,8 +207,10 @@ struct Slice {
         *gx_gs = nullptr, *gx_hs = nullptr;
   double *gx_pd = nullptr, *gx_pt = nullptr, *gx_loss = nullptr;
   // global block ranges in the batched launches
-  float* fftG = nullptr;   // FFT ramp: spectrum of the wrapped kernel / L (fft_len(N))
-  float2* fftW = nullptr;  // FFT ramp: twiddles (fft_len(N) / 2)
+  // FFT ramp (fft_tables), null when N is past its limit: spectrum of the
+  // wrapped kernel and twiddles, fft_len(N) / 2 + 1 each
+  double* fftG = nullptr;
+  double2* fftW = nullptr;
   int ff_begin = 0, ff_n = 0;
   float ff_edge = 0.0f;    // FFT ramp: the tap at distance N-1 (h(2N-1), 0-based)
   int rf_begin = 0, rf_n = 0, bp_begin = 0, bp_n = 0, cl_begin = 0, cl_n = 0,
@@ -250,7 +252,7 @@ struct acu_batch {
   void* ops_mem = nullptr;
   void* tv_mem = nullptr;
   int tv_delta_cap = 0;
-  int ff_total = 0, ff_maxL = 0;  // FFT ramp blocks and the largest transform
+  int ff_total = 0, ff_threads = 64;  // FFT ramp blocks (slices within its limit) and threads per workgroup
   int rf_total = 0, bp_total = 0, cl_total = 0, fp_total = 0, fs_total = 0, ew_total = 0,
       sw_total = 0;
   int fl_total[acu::FL_GROUPS] = {0, 0, 0, 0};  // LDS projector blocks per variant group (lds1, lds2, lds4, cell16)
@@ -349,8 +351,9 @@ void layout_ops(acu_batch* b, Carver& cv) {
     s.fpart = cv.take<float>((size_t)fp_chunks(s.N, s.fp_clen) * NT);
     for (int g = 0; g < 3; ++g) s.pcls[g] = cv.take<uint8_t>((size_t)(s.T + (4 << g) - 1) / (4 << g));
     if (fft_supported(s.N)) {
-      s.fftG = cv.take<float>((size_t)fft_len(s.N));
-      s.fftW = cv.take<float2>((size_t)fft_len(s.N) / 2);
+      const size_t M1 = (size_t)fft_len(s.N) / 2 + 1;
+      s.fftG = cv.take<double>(M1);
+      s.fftW = cv.take<double2>(M1);
     }
   }
 }
@@ -387,13 +390,13 @@ void upload_tables(acu_batch* b, int i) {
   ACU_HIP_CHECK(hipMemcpyAsync(s.h, h.data(), h.size() * 4, hipMemcpyHostToDevice, st));
   s.ff_edge = h[2 * s.N - 1];
   if (s.fftG) {
-    const int L = fft_len(s.N);
-    std::vector<float> G(L);
-    std::vector<float2> W(L / 2);
+    const size_t M1 = (size_t)fft_len(s.N) / 2 + 1;
+    std::vector<double> G(M1);
+    std::vector<double2> W(M1);
     fft_tables(s.N, h.data(), G.data(), W.data());
-    ACU_HIP_CHECK(hipMemcpyAsync(s.fftG, G.data(), G.size() * 4, hipMemcpyHostToDevice, st));
-    ACU_HIP_CHECK(hipMemcpyAsync(s.fftW, W.data(), W.size() * sizeof(float2), hipMemcpyHostToDevice, st));
-    ACU_HIP_CHECK(hipStreamSynchronize(st));  // G and W end here
+    ACU_HIP_CHECK(hipMemcpyAsync(s.fftG, G.data(), M1 * sizeof(double), hipMemcpyHostToDevice, st));
+    ACU_HIP_CHECK(hipMemcpyAsync(s.fftW, W.data(), M1 * sizeof(double2), hipMemcpyHostToDevice, st));
+    ACU_HIP_CHECK(hipStreamSynchronize(st));  // the tables end here
   }
   ACU_HIP_CHECK(hipMemcpyAsync(s.cmask, cm.data(), cm.size() * 4, hipMemcpyHostToDevice, st));
   ACU_HIP_CHECK(hipMemcpyAsync(s.tact, act.data(), act.size(), hipMemcpyHostToDevice, st));
@@ -413,9 +416,9 @@ void copy_tables(acu_batch* b, int j, int i) {
   s.tact_h = a.tact_h;
   s.ff_edge = a.ff_edge;
   if (s.fftG) {
-    const size_t L = (size_t)fft_len(s.N);
-    ACU_HIP_CHECK(hipMemcpyAsync(s.fftG, a.fftG, L * 4, hipMemcpyDeviceToDevice, st));
-    ACU_HIP_CHECK(hipMemcpyAsync(s.fftW, a.fftW, L / 2 * sizeof(float2), hipMemcpyDeviceToDevice, st));
+    const size_t M1 = (size_t)fft_len(s.N) / 2 + 1;
+    ACU_HIP_CHECK(hipMemcpyAsync(s.fftG, a.fftG, M1 * sizeof(double), hipMemcpyDeviceToDevice, st));
+    ACU_HIP_CHECK(hipMemcpyAsync(s.fftW, a.fftW, M1 * sizeof(double2), hipMemcpyDeviceToDevice, st));
   }
 }
 
@@ -463,7 +466,7 @@ FFTTask ff_task(const Slice& s, const float* in, float* out) {
   const int L = fft_len(s.N);
   int lg = 0;
   while ((1 << lg) < L) ++lg;
-  return FFTTask{s.N, s.T, L, lg, s.ff_begin, L == 2 * s.N - 2 ? 1 : 0, s.ff_edge, s.fftG, s.fftW, in, out};
+  return FFTTask{s.N, s.T, lg, s.ff_begin, L == 2 * s.N - 2 ? 1 : 0, s.ff_edge, s.h, s.fftG, s.fftW, in, out};
 }
 BPTask bp_task(const Slice& s, const float* in, float* out) {
   return BPTask{s.N, s.T, s.mid, s.bp_begin, s.ntx, s.nty, s.nsub, in, s.cmask, s.scbp, s.tact, s.rowterm, out};
@@ -700,15 +703,28 @@ const BPShares& bp_shares(const acu_batch* b, int sl) { return sl < 0 ? b->bp_sh
 Range ew_range(acu_batch* b, int sl) { return sl < 0 ? Range{0, b->ew_total} : Range{b->s[sl].ew_begin, b->s[sl].ew_n}; }
 Range sw_range(acu_batch* b, int sl) { return sl < 0 ? Range{0, b->sw_total} : Range{b->s[sl].sw_begin, b->s[sl].sw_n}; }
 
-void ramp_seq(acu_batch* b, const RFSet& rf, int sl) {
-  acu_ctx* c = b->ctx;
-  if (b->ramp_variant == RAMP_FFT) {
-    const Range r = sl < 0 ? Range{0, b->ff_total} : Range{b->s[sl].ff_begin, b->s[sl].ff_n};
-    timed(c, K_RF, [&] { launch_ramp_fft(rf.ff.d, rf.ff.n, r.base, r.n, b->ff_maxL, c->stream); });
-  } else {
-    const Range r = rf_range(b, sl);
-    timed(c, K_RF, [&] { launch_ramp(rf.rf.d, rf.rf.n, r.base, r.n, b->ramp_variant, c->stream); });
+// The ramp filter of all slices (sl < 0) or one, in one arithmetic.  FP64
+// goes by FFT for every slice within its length limit (N <= 4097: a row's
+// points fit LDS twice over) and by the Toeplitz product on the FP64 matrix
+// cores beyond.  The FFT is faster at every size within it: ms by FFT and as
+// a product, 0.008 and 0.033 at 257^2 x 180, 0.032 and 0.27 at 2049^2 x 1500.
+void launch_ramp_any(acu_batch* b, const RFSet& rf, int sl, int variant) {
+  hipStream_t st = b->ctx->stream;
+  const bool all = sl < 0;
+  if (variant == RAMP_FFT || variant == RAMP_FP64) {
+    launch_ramp_fft(rf.ff.d, rf.ff.n, all ? 0 : b->s[sl].ff_begin, all ? b->ff_total : b->s[sl].ff_n, b->ff_threads,
+                    st);
+    if (variant == RAMP_FP64)
+      for (int i = all ? 0 : sl; i < (all ? (int)b->s.size() : sl + 1); ++i)
+        if (!b->s[i].fftG) launch_ramp(rf.rf.d, rf.rf.n, b->s[i].rf_begin, b->s[i].rf_n, variant, st);
+    return;
   }
+  const Range r = rf_range(b, sl);
+  launch_ramp(rf.rf.d, rf.rf.n, r.base, r.n, variant, st);
+}
+
+void ramp_seq(acu_batch* b, const RFSet& rf, int sl) {
+  timed(b->ctx, K_RF, [&] { launch_ramp_any(b, rf, sl, b->ramp_variant); });
 }
 
 // refpos: the backprojection positions (the batch's FBP positions, or
@@ -988,11 +1004,11 @@ void radon_dev(acu_batch* b, int sl, float* sino, const float* img) {
 void ramp_dev(acu_batch* b, int sl, float* out, const float* in) {
   Slice& s = slice_of(b, sl);
   acu_ctx* c = b->ctx;
-  if (b->ramp_variant == RAMP_FFT) {
+  if (b->ramp_variant == RAMP_FFT || (b->ramp_variant == RAMP_FP64 && s.fftG)) {
     FFTTask t = ff_task(s, in, out);
     t.block_begin = 0;
     FFTTask* d = put_adhoc(b, t);
-    timed(c, K_RF, [&] { launch_ramp_fft(d, 1, 0, s.ff_n, fft_len(s.N), c->stream); });
+    timed(c, K_RF, [&] { launch_ramp_fft(d, 1, 0, s.ff_n, b->ff_threads, c->stream); });
     check_launch();
     return;
   }
@@ -1116,12 +1132,7 @@ const char* ramp_name(int v) {
 // Average ms of one ramp filter of every slice (f -> sinoCS) with variant v.
 double time_ramp(acu_batch* b, int v, int reps) {
   acu_ctx* c = b->ctx;
-  const int saved = b->ramp_variant;
-  b->ramp_variant = v;
-  auto run = [&] {
-    if (v == RAMP_FFT) launch_ramp_fft(b->rf_f.ff.d, b->rf_f.ff.n, 0, b->ff_total, b->ff_maxL, c->stream);
-    else launch_ramp(b->rf_f.rf.d, b->rf_f.rf.n, 0, b->rf_total, v, c->stream);
-  };
+  auto run = [&] { launch_ramp_any(b, b->rf_f, -1, v); };
   hipEvent_t e0 = c->ev(), e1 = c->ev();
   run();
   ACU_HIP_CHECK(hipEventRecord(e0, c->stream));
@@ -1133,7 +1144,6 @@ double time_ramp(acu_batch* b, int v, int reps) {
   ACU_HIP_CHECK(hipEventElapsedTime(&ms, e0, e1));
   c->pool.push_back(e0);
   c->pool.push_back(e1);
-  b->ramp_variant = saved;
   return (double)ms / reps;
 }
 
@@ -1501,8 +1511,7 @@ int acu_batch_create(acu_ctx* ctx, int nslices, const int* nimage, const int* nt
       s.ntx = acu::bp_tiles_x(s.N); s.nsub = (s.N + acu::BP_SUB - 1) / acu::BP_SUB;
       s.theta.assign(s.T, 0.0f);
       s.rf_begin = rf; s.rf_n = acu::rf_tiles_m(s.N) * acu::rf_tiles_n(s.T); rf += s.rf_n;
-      s.ff_begin = b->ff_total; s.ff_n = (s.T + 1) / 2; b->ff_total += s.ff_n;
-      b->ff_maxL = std::max(b->ff_maxL, acu::fft_len(s.N));
+      if (acu::fft_supported(s.N)) b->ff_threads = std::max(b->ff_threads, acu::fft_threads(s.N));
       s.fp_clen = fp_clen_env > 0 ? fp_clen_env : acu::FP_CHUNK_DEFAULT;
       s.fpv = gather ? 0
                      : (al_env > 0 && acu::fpv_valid(al_env)) ? al_env
@@ -1511,6 +1520,10 @@ int acu_batch_create(acu_ctx* ctx, int nslices, const int* nimage, const int* nt
       s.sw_begin = sw; s.sw_n = acu::ew_blocks((size_t)s.N * s.T); sw += s.sw_n;
     }
     b->rf_total = rf;
+    for (auto& s : b->s)
+      if (acu::fft_supported(s.N)) {
+        s.ff_begin = b->ff_total; s.ff_n = acu::fft_blocks(s.N, s.T, b->ff_threads); b->ff_total += s.ff_n;
+      }
     acu::assign_bp(b.get());
     b->ew_total = ew; b->sw_total = sw;
     acu::Carver dry;

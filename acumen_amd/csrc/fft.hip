@@ -1,5 +1,5 @@
 // fft.hip -- the ramp filter (tomography/tv_hpc.F90:93-105) by FFT
-// convolution, the RAMP_FFT variant of the filter's precision study.
+// convolution in FP64: RAMP_FP64 of slices up to N = 4097, and RAMP_FFT.
 //
 //   sinoCS(i, t) = sum_{j=0..N-1} g(i - j) sino(j, t),   g(m) = h[m + N],
 //
@@ -8,28 +8,118 @@
 // with gw(r) = sum_{m = r mod L} g(m), except when L = 2N-2, where m = N-1
 // and m = -(N-1) share a residue: then outputs 0 and N-1 pick up one extra
 // term each, g(N-1) s(N-1) and g(N-1) s(0), which are subtracted.  G =
-// DFT(gw) is real and even (g is symmetric), so two real rows a, b ride in
-// one complex FFT: IDFT(G * DFT(a + i b)) = (a * g) + i (b * g).
+// DFT(gw) is real and even (g is symmetric).
 //
-// gfx950 mapping: one workgroup per pair of angle rows; the L complex
-// values live in LDS (L <= 8192, 64 KB).  The forward transform is a
-// radix-2 decimation in time over bit-reversed input (natural-order
-// output); after the multiplication by G the inverse is a radix-2
-// decimation in frequency (bit-reversed output), read back through the bit
-// reversal, so no permutation pass is needed.  G and the twiddles are
-// computed on the host in FP64 from the reference's FP32 taps; the
-// transforms run in FP32.
+// A real row of L values is one complex transform of M = L/2 points z(n) =
+// x(2n) + i x(2n+1), so rows never mix (a row of NaN or of huge values
+// leaves its neighbours alone).  The spectrum X of the row, its product with
+// G and the packing of the result back into M points are one pass over the
+// pairs (k, M-k).
+//
+// gfx950 mapping: M/8 threads per row, rows packed into workgroups of NT =
+// 64..512 threads (the largest row of the batch sets NT); the M points live
+// in LDS, padded by one in eight against bank conflicts.  Forward: radix-8
+// decimation in frequency, in place, the first pass straight from global
+// memory, the last of radix 1, 2 or 4; the pair pass works on the
+// digit-reversed order that leaves; the inverse runs the same passes
+// backwards (decimation in time), the last one straight to global memory.
+// A butterfly's twiddles are three table loads (w, w^2, w^4) and four
+// products.  G and the twiddles come from the host in FP64 (the reference's
+// FP32 taps).
+//
+// Bound by its LDS passes (about 16 of 16 bytes per point) and their
+// barriers.  A 2049^2 x 1500 slice is 12.6 GFLOP as a Toeplitz product and
+// 0.45 GFLOP this way.  The result is the exact one but for its rounding to
+// FP32, as the Toeplitz product's on the FP64 matrix cores is (filter.hip):
+// both are 2.5e-8 from FP64 on noise at N = 6..4097.  Measured on MI355X, ms
+// per launch: 8 x 2049^2 x 1500 0.207 (product 2.18; the radix-2 FP32
+// transform of row pairs this replaces 0.406), 4 x 1025^2 x 720 0.030
+// (product 0.21), 257^2 x 180 0.008 (product 0.033).  The same passes in
+// FP32 took 0.144 with products of FP32 twiddles, but 1.2x the error of that
+// radix-2 transform; without the extra error they took 0.202, so there is no
+// FP32 form.
 #include "acu_internal.hpp"
 
+#include <algorithm>
 #include <cmath>
 #include <complex>
+#include <type_traits>
 #include <vector>
 
 namespace acu {
 namespace {
 
-constexpr int FFT_THREADS = 256;
 constexpr double kPi = 3.14159265358979323846;
+
+typedef double2 C;
+
+__device__ __forceinline__ C mk(double x, double y) { return make_double2(x, y); }
+__device__ __forceinline__ C cadd(C a, C b) { return mk(a.x + b.x, a.y + b.y); }
+__device__ __forceinline__ C csub(C a, C b) { return mk(a.x - b.x, a.y - b.y); }
+__device__ __forceinline__ C cmul(C a, C b) { return mk(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x); }
+__device__ __forceinline__ C cconj(C a) { return mk(a.x, -a.y); }
+// a * (-i) (forward) or a * i (inverse)
+template <bool INV> __device__ __forceinline__ C rot(C a) { return INV ? mk(-a.y, a.x) : mk(a.y, -a.x); }
+
+template <bool INV>
+__device__ __forceinline__ void dft4(C a0, C a1, C a2, C a3, C& y0, C& y1, C& y2, C& y3) {
+  const C s02 = cadd(a0, a2), d02 = csub(a0, a2), s13 = cadd(a1, a3), r13 = rot<INV>(csub(a1, a3));
+  y0 = cadd(s02, s13);
+  y2 = csub(s02, s13);
+  y1 = cadd(d02, r13);
+  y3 = csub(d02, r13);
+}
+
+// x <- DFT of x (natural order both sides); INV: unnormalised inverse
+template <int R, bool INV>
+__device__ __forceinline__ void dft(C (&x)[R]) {
+  if constexpr (R == 2) {
+    const C a = x[0];
+    x[0] = cadd(a, x[1]);
+    x[1] = csub(a, x[1]);
+  } else if constexpr (R == 4) {
+    C y0, y1, y2, y3;
+    dft4<INV>(x[0], x[1], x[2], x[3], y0, y1, y2, y3);
+    x[0] = y0; x[1] = y1; x[2] = y2; x[3] = y3;
+  } else {
+    const double h = 0.70710678118654752440;
+    const C e0 = cadd(x[0], x[4]), e1 = cadd(x[1], x[5]), e2 = cadd(x[2], x[6]), e3 = cadd(x[3], x[7]);
+    const C o0 = csub(x[0], x[4]), d1 = csub(x[1], x[5]), d2 = csub(x[2], x[6]), d3 = csub(x[3], x[7]);
+    // o_j = d_j exp(-+ i pi j / 4)
+    const C r1 = rot<INV>(d1), r3 = rot<INV>(d3);
+    const C o1 = mk((d1.x + r1.x) * h, (d1.y + r1.y) * h), o2 = rot<INV>(d2),
+            o3 = mk((r3.x - d3.x) * h, (r3.y - d3.y) * h);
+    dft4<INV>(e0, e1, e2, e3, x[0], x[2], x[4], x[6]);
+    dft4<INV>(o0, o1, o2, o3, x[1], x[3], x[5], x[7]);
+  }
+}
+
+__device__ __forceinline__ int pad(int i) { return i + (i >> 3); }
+
+// the twiddles w^1..w^7 of one radix-8 butterfly, w = W_M^e (e < M/8); conj for the inverse
+template <bool INV>
+__device__ __forceinline__ void twiddles(const C* __restrict__ tw, int e, C (&w)[8]) {
+  w[1] = tw[e];
+  w[2] = tw[2 * e];
+  w[4] = tw[4 * e];
+  if (INV) { w[1] = cconj(w[1]); w[2] = cconj(w[2]); w[4] = cconj(w[4]); }
+  w[3] = cmul(w[1], w[2]);
+  w[5] = cmul(w[1], w[4]);
+  w[6] = cmul(w[2], w[4]);
+  w[7] = cmul(w[3], w[4]);
+}
+
+// position of frequency k after the forward passes: `q` base-8 digits of k
+// from the top of the m-bit position down, the rest below
+__device__ __forceinline__ int freq_pos(int k, int m, int q) {
+  int pos = 0, sh = m;
+  for (int i = 0; i < q; ++i) {
+    sh -= 3;
+    pos |= (k & 7) << sh;
+    k >>= 3;
+  }
+  return pos | k;
+}
 
 __device__ __forceinline__ int find_task(const FFTTask* tasks, int ntasks, int gb) {
   int lo = 0, hi = ntasks - 1;
@@ -40,72 +130,164 @@ __device__ __forceinline__ int find_task(const FFTTask* tasks, int ntasks, int g
   return lo;
 }
 
-__device__ __forceinline__ int bitrev(int i, int lg) { return (int)(__brev((unsigned)i) >> (32 - lg)); }
+// Outputs lt, lt + step, ... of one row as the plain sum in FP64: rows of
+// fewer than 8 points, and FP64 rows that hold an infinity or NaN (every tap
+// is nonzero, so each output is then the sum's own infinity or NaN).
+__device__ void direct_row(const float* __restrict__ h, const float* __restrict__ s, float* __restrict__ out, int N,
+                           int lt, int step) {
+  for (int i = lt; i < N; i += step) {
+    double a = 0.0;
+    for (int j = 0; j < N; ++j) a += (double)h[i - j + N] * (double)s[j];
+    out[i] = (float)a;
+  }
+}
 
-__global__ __launch_bounds__(FFT_THREADS) void fft_ramp_kernel(const FFTTask* __restrict__ tasks, int ntasks,
-                                                               int base, int nblocks) {
-  extern __shared__ float2 X[];
+template <int NT>
+__global__ __launch_bounds__(NT) void fft_ramp_kernel(const FFTTask* __restrict__ tasks, int ntasks, int base,
+                                                      int nblocks) {
+  __shared__ C lds[NT * 9];
+  __shared__ unsigned long long bad_s[NT / 64];
   const int lbk = xcd_remap(blockIdx.x, gridDim.x);
   if (lbk >= nblocks) return;  // uniform per workgroup
   const int gb = base + lbk;
   const FFTTask& tk = tasks[find_task(tasks, ntasks, gb)];
-  const int N = tk.N, T = tk.T, L = tk.L, lg = tk.lg;
-  const int ra = 2 * (gb - tk.block_begin), rb = ra + 1;
-  const bool hasb = rb < T;
-  const float* sa = tk.sino + (size_t)ra * N;
-  const float* sb = tk.sino + (size_t)(hasb ? rb : ra) * N;
-  const float2* __restrict__ W = tk.tw;  // exp(-2 pi i k / L), k < L/2
+  const int N = tk.N, m = tk.lg - 1, M = 1 << m;
+  const int local = gb - tk.block_begin;
+  const int tid = threadIdx.x;
+  if (m < 3) {
+    direct_row(tk.h, tk.sino + (size_t)local * N, tk.out + (size_t)local * N, N, tid, NT);
+    return;
+  }
+  const int lt = tid & (M / 8 - 1), g = tid >> (m - 3);  // thread of its row, row of the workgroup
+  const int row = local * (NT >> (m - 3)) + g;
+  const bool act = row < tk.T;
+  const float* __restrict__ s = tk.sino + (size_t)(act ? row : 0) * N;
+  float* __restrict__ out = tk.out + (size_t)(act ? row : 0) * N;
+  const C* __restrict__ tw = tk.tw;
+  const C* __restrict__ twl = tw + M / 2;  // exp(-2 pi i k / L), k <= M/2
+  const double* __restrict__ G = tk.G;
+  C* X = lds + g * (M + M / 8);
+  const int q = m / 3, tail = m - 3 * q;
 
-  // bit-reversed load: X[bitrev(j)] = a(j) + i b(j), zero beyond N
-  for (int j = threadIdx.x; j < L; j += FFT_THREADS) {
-    float2 v = make_float2(0.0f, 0.0f);
-    if (j < N) v = make_float2(sa[j], hasb ? sb[j] : 0.0f);
-    X[bitrev(j, lg)] = v;
+  // forward pass 1 from global memory: points beyond the row are zero
+  C x[8], w[8];
+  bool bad = false;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    const int n = 2 * (lt + j * (M / 8));
+    const float a = act && n < N ? s[n] : 0.0f, b = act && n + 1 < N ? s[n + 1] : 0.0f;
+    bad = bad || !(fabsf(a) <= 3.40282347e38f) || !(fabsf(b) <= 3.40282347e38f);
+    x[j] = mk((double)a, (double)b);
   }
+  const float s0 = s[0], s1 = s[N - 1];  // for the alias correction
+  const unsigned long long bm = __ballot(bad);
+  if ((tid & 63) == 0) bad_s[tid >> 6] = bm;
+  dft<8, false>(x);
+  twiddles<false>(tw, lt, w);
+  X[pad(lt)] = x[0];
+#pragma unroll
+  for (int j = 1; j < 8; ++j) X[pad(lt + j * (M / 8))] = cmul(x[j], w[j]);
   __syncthreads();
-  // forward: decimation in time
-  for (int m = 1, ts = L / 2; m < L; m <<= 1, ts >>= 1) {
-    for (int k = threadIdx.x; k < L / 2; k += FFT_THREADS) {
-      const int pos = k & (m - 1);
-      const int i0 = ((k - pos) << 1) + pos, i1 = i0 + m;
-      const float2 w = W[pos * ts];
-      const float2 x1 = X[i1], x0 = X[i0];
-      const float2 t = make_float2(w.x * x1.x - w.y * x1.y, w.x * x1.y + w.y * x1.x);
-      X[i0] = make_float2(x0.x + t.x, x0.y + t.y);
-      X[i1] = make_float2(x0.x - t.x, x0.y - t.y);
-    }
+  const int rt = M / 8;  // does this thread's row hold an infinity or NaN
+  if (rt >= 64) for (int v = 0; v < rt / 64; ++v) bad = bad || bad_s[g * (rt / 64) + v] != 0;
+  else bad = ((bad_s[tid >> 6] >> ((tid & 63) & ~(rt - 1))) & ((1ull << rt) - 1)) != 0;
+  for (int ls = m - 6; ls >= tail; ls -= 3) {  // sub-transforms of 8 << ls points
+    const int p = lt & ((1 << ls) - 1), i0 = ((lt >> ls) << (ls + 3)) + p;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) x[j] = X[pad(i0 + (j << ls))];
+    dft<8, false>(x);
+    twiddles<false>(tw, p << (m - 3 - ls), w);
+    X[pad(i0)] = x[0];
+#pragma unroll
+    for (int j = 1; j < 8; ++j) X[pad(i0 + (j << ls))] = cmul(x[j], w[j]);
     __syncthreads();
   }
-  // filter: the spectrum of the kernel is real; 1/L folded in
-  for (int k = threadIdx.x; k < L; k += FFT_THREADS) {
-    const float g = tk.G[k];
-    const float2 v = X[k];
-    X[k] = make_float2(v.x * g, v.y * g);
-  }
-  __syncthreads();
-  // inverse: decimation in frequency with conjugate twiddles
-  for (int m = L / 2, ts = 1; m >= 1; m >>= 1, ts <<= 1) {
-    for (int k = threadIdx.x; k < L / 2; k += FFT_THREADS) {
-      const int pos = k & (m - 1);
-      const int i0 = ((k - pos) << 1) + pos, i1 = i0 + m;
-      const float2 w = W[pos * ts];
-      const float2 x0 = X[i0], x1 = X[i1];
-      const float2 d = make_float2(x0.x - x1.x, x0.y - x1.y);
-      X[i0] = make_float2(x0.x + x1.x, x0.y + x1.y);
-      X[i1] = make_float2(w.x * d.x + w.y * d.y, w.x * d.y - w.y * d.x);
+  auto small = [&](auto inv) {  // the tail: sub-transforms of 2 or 4 points, no twiddles
+    constexpr bool INV = decltype(inv)::value;
+    if (tail == 1) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int i0 = 2 * (lt + j * (M / 8));
+        C y[2] = {X[pad(i0)], X[pad(i0 + 1)]};
+        dft<2, INV>(y);
+        X[pad(i0)] = y[0];
+        X[pad(i0 + 1)] = y[1];
+      }
+    } else {
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        const int i0 = 4 * (lt + j * (M / 8));
+        C y[4];
+#pragma unroll
+        for (int v = 0; v < 4; ++v) y[v] = X[pad(i0 + v)];
+        dft<4, INV>(y);
+#pragma unroll
+        for (int v = 0; v < 4; ++v) X[pad(i0 + v)] = y[v];
+      }
     }
     __syncthreads();
-  }
-  float* oa = tk.out + (size_t)ra * N;
-  float* ob = tk.out + (size_t)rb * N;
-  for (int i = threadIdx.x; i < N; i += FFT_THREADS) {
-    float2 c = X[bitrev(i, lg)];
-    if (tk.alias) {  // L = 2N-2: remove the wrapped term of the shared residue
-      if (i == N - 1) { c.x -= tk.g_edge * sa[0]; c.y -= hasb ? tk.g_edge * sb[0] : 0.0f; }
-      if (i == 0) { c.x -= tk.g_edge * sa[N - 1]; c.y -= hasb ? tk.g_edge * sb[N - 1] : 0.0f; }
+  };
+  if (tail) small(std::false_type{});
+
+  // pairs (k, M-k): X_k = E + w^k O, conj(X_{M-k}) = E - w^k O from Z_k and
+  // Z_{M-k}; times the real G; packed back (G carries the 1/M of the inverse)
+  for (int k = lt; k <= M / 2; k += M / 8) {
+    const int ia = pad(freq_pos(k, m, q));
+    const C za = X[ia];
+    if (k == 0) {
+      const double a = G[0] * (za.x + za.y), b = G[M] * (za.x - za.y);
+      X[ia] = mk(0.5 * (a + b), 0.5 * (a - b));
+    } else if (k == M / 2) {
+      X[ia] = mk(G[k] * za.x, G[k] * za.y);
+    } else {
+      const int ib = pad(freq_pos(M - k, m, q));
+      const C zb = cconj(X[ib]);
+      const C e = mk(0.5 * (za.x + zb.x), 0.5 * (za.y + zb.y));
+      const C o = mk(0.5 * (za.y - zb.y), 0.5 * (zb.x - za.x));  // -i (za - zb) / 2
+      const C wk = twl[k], t = cmul(wk, o);
+      const double ga = G[k], gm = G[M - k];
+      const C a = mk(ga * (e.x + t.x), ga * (e.y + t.y)), b = mk(gm * (e.x - t.x), gm * (e.y - t.y));
+      const C e2 = mk(0.5 * (a.x + b.x), 0.5 * (a.y + b.y));
+      const C o2 = cmul(cconj(wk), mk(0.5 * (a.x - b.x), 0.5 * (a.y - b.y)));
+      X[ia] = mk(e2.x - o2.y, e2.y + o2.x);  // E' + i O'
+      X[ib] = mk(e2.x + o2.y, o2.x - e2.y);  // conj(E' - i O')
     }
-    oa[i] = c.x;
-    if (hasb) ob[i] = c.y;
+  }
+  __syncthreads();
+
+  if (tail) small(std::true_type{});
+  for (int ls = tail; ls <= m - 6; ls += 3) {
+    const int p = lt & ((1 << ls) - 1), i0 = ((lt >> ls) << (ls + 3)) + p;
+    twiddles<true>(tw, p << (m - 3 - ls), w);
+    x[0] = X[pad(i0)];
+#pragma unroll
+    for (int j = 1; j < 8; ++j) x[j] = cmul(X[pad(i0 + (j << ls))], w[j]);
+    dft<8, true>(x);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) X[pad(i0 + (j << ls))] = x[j];
+    __syncthreads();
+  }
+  // inverse pass over all M points, to global memory (no barrier below)
+  if (!act) return;
+  if (bad) {
+    direct_row(tk.h, s, out, N, lt, M / 8);
+    return;
+  }
+  twiddles<true>(tw, lt, w);
+  x[0] = X[pad(lt)];
+#pragma unroll
+  for (int j = 1; j < 8; ++j) x[j] = cmul(X[pad(lt + j * (M / 8))], w[j]);
+  dft<8, true>(x);
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    const int n = 2 * (lt + j * (M / 8));
+    double a = x[j].x;
+    if (tk.alias) {  // L = 2N-2: remove the wrapped term of the shared residue (N - 1 is even)
+      if (n == 0) a -= (double)tk.g_edge * (double)s1;
+      if (n == N - 1) a -= (double)tk.g_edge * (double)s0;
+    }
+    if (n < N) out[n] = (float)a;
+    if (n + 1 < N) out[n + 1] = (float)x[j].y;
   }
 }
 
@@ -139,22 +321,37 @@ int fft_len(int N) {
 
 bool fft_supported(int N) { return N >= 3 && fft_len(N) <= FFT_MAX_L; }
 
-void fft_tables(int N, const float* taps, float* G, float2* tw) {
-  const int L = fft_len(N);
+int fft_threads(int maxN) { return std::max(64, std::min(512, fft_len(maxN) / 16)); }
+
+int fft_blocks(int N, int T, int threads) {
+  const int rows = std::max(1, 16 * threads / std::max(16, fft_len(N)));
+  return fft_len(N) < 16 ? T : (T + rows - 1) / rows;
+}
+
+void fft_tables(int N, const float* taps, double* G, double2* tw) {
+  const int L = fft_len(N), M = L / 2;
   std::vector<std::complex<double>> a(L, 0.0);
   for (int m = -(N - 1); m <= N - 1; ++m) a[((m % L) + L) % L] += (double)taps[m + N];
   fft_host(a);
-  for (int k = 0; k < L; ++k) G[k] = (float)(a[k].real() / (double)L);
-  for (int k = 0; k < L / 2; ++k) {
-    const double ang = -2.0 * kPi * (double)k / (double)L;
-    tw[k] = make_float2((float)std::cos(ang), (float)std::sin(ang));
-  }
+  for (int k = 0; k <= M; ++k) G[k] = a[k].real() / (double)M;
+  auto unit = [](int k, int n) {
+    const double ang = -2.0 * kPi * (double)k / (double)n;
+    return make_double2(std::cos(ang), std::sin(ang));
+  };
+  for (int k = 0; k < M / 2; ++k) tw[k] = unit(k, M);
+  for (int k = 0; k <= M / 2; ++k) tw[M / 2 + k] = unit(k, L);
 }
 
-void launch_ramp_fft(const FFTTask* d_tasks, int ntasks, int base, int blocks, int maxL, hipStream_t s) {
+void launch_ramp_fft(const FFTTask* d_tasks, int ntasks, int base, int blocks, int threads, hipStream_t s) {
   if (blocks <= 0) return;
-  hipLaunchKernelGGL(fft_ramp_kernel, dim3(xcd_grid(blocks)), dim3(FFT_THREADS), (size_t)maxL * sizeof(float2), s,
-                     d_tasks, ntasks, base, blocks);
+  const dim3 g(xcd_grid(blocks)), t(threads);
+  switch (threads) {
+    case 64: hipLaunchKernelGGL(fft_ramp_kernel<64>, g, t, 0, s, d_tasks, ntasks, base, blocks); break;
+    case 128: hipLaunchKernelGGL(fft_ramp_kernel<128>, g, t, 0, s, d_tasks, ntasks, base, blocks); break;
+    case 256: hipLaunchKernelGGL(fft_ramp_kernel<256>, g, t, 0, s, d_tasks, ntasks, base, blocks); break;
+    case 512: hipLaunchKernelGGL(fft_ramp_kernel<512>, g, t, 0, s, d_tasks, ntasks, base, blocks); break;
+    default: throw Error("FFT ramp: workgroups of 64, 128, 256 or 512 threads");
+  }
 }
 
 }  // namespace acu

@@ -1,5 +1,6 @@
-// filter.hip -- ramp filtering of sinograms as a Toeplitz GEMM on the
-// FP64 matrix cores.
+// filter.hip -- ramp filtering of sinograms as a Toeplitz GEMM on the matrix
+// cores: the FP64 form for slices past the FFT's length limit (N > 4097, see
+// fft.hip) and the FP32 and BF16 variants at every size.
 //
 // Restates the first half of iradon (tomography/tv_hpc.F90:93-105):
 //   sinoCS(i, t) = sum_{j=0..N-1} h[i - j + N] * sino(j, t)
@@ -17,8 +18,7 @@
 // v_mfma_f64_16x16x4_f64 (78.6 TF dense on MI355X), so the only rounding is
 // the final conversion of each output to FP32.
 //
-// Variants (RAMP_*, for the precision study of the filter; FP64 is the
-// default): FP32 MFMA (v_mfma_f32_16x16x4_f32, FP32 products and sums),
+// Variants (RAMP_*, for the precision study of the filter): FP32 MFMA (v_mfma_f32_16x16x4_f32, FP32 products and sums),
 // BF16x3 (each FP32 operand split into bf16 hi + lo, products hi*hi + hi*lo
 // + lo*hi on v_mfma_f32_16x16x32_bf16, FP32 sums) and BF16x6 (hi + mid + lo,
 // the six products down to 2^-16 relative, FP32 sums).  The splits are
