@@ -44,6 +44,19 @@ __device__ __forceinline__ float4 global_f4(const ACU_GLOBAL float4* tab, unsign
   return make_float4(v.x, v.y, v.z, v.w);
 }
 
+// LDS offsets in float arithmetic.  On gfx950 v_fma/add/sub/mul_f32 issue at
+// twice the rate of v_cvt, v_lshl_add, v_dot2 and v_mad_u24 (about 100 and 56
+// lanes per CU and clock in a probe), and a denormal float's bits are its
+// value in units of 2^-149.  So byte offsets k * n of integer-valued floats n
+// are formed as fma(n, lds_units(k), base) and read back as bits, with no
+// conversion or integer operation.  Exact while the offset is in [0, 2^23)
+// (FP32 denormals are on, HIP's default).
+__device__ constexpr float lds_units(int k) { return (float)k * 0x1p-149f; }
+// an integer in (-2^23, 2^23) as a float in those units
+__device__ __forceinline__ float lds_base(int v) {
+  return __uint_as_float(v < 0 ? 0x80000000u | (unsigned)-v : (unsigned)v);
+}
+
 // The dispatcher deals workgroups round-robin over the 8 XCDs of MI355X,
 // each with its own L2.  xcd_remap turns the hardware block index of a grid
 // of xcd_grid(n) blocks into a logical index in [0, xcd_grid(n)) such that

@@ -32,6 +32,11 @@
 //    K = s*(x0+1-m) + c*(y0+1-m) + m-1-lo formed in FP64 once per angle and
 //    tile, so a position is rounded at magnitude below ~100: closer to FP64,
 //    farther from the reference, two VALU fewer per update;
+//    in both, y1 = floor(yr) and the pair's LDS offset come from v_fract and
+//    full-rate float arithmetic (lds_units) instead of v_cvt and
+//    v_lshl_add: 551 against 575 us per 4 x 1025^2 x 720 launch, 6.23
+//    against 6.34 ms per 8 x 2049^2 x 1500 (0.79 ms a slice; the kernel is
+//    bound by its VALU issue, 1.4-1.5 wave-instructions per CU and clock);
 //  * each 32-angle block is summed separately and then added;
 //  * tiles whose mask is identically zero (by 64 x 16 sub-tiles) only store
 //    zeros.
@@ -163,17 +168,15 @@ __global__ __launch_bounds__(64 * bp_waves(TY)) void bp_kernel(const BPTask* __r
 #pragma clang fp contract(off)
         const float sa = const_f2(sc, a0 + a).x;
         const float A = sa * ux;  // sin(c)*(jx-midpoint), tv_hpc.F90:114
-        // byte offset of P[a*W - 1 - lo] (wave-uniform): the pair of the
-        // 1-based tap y1 is at Pb + 8*y1
-        const char* Pb = (const char*)P + __builtin_amdgcn_readfirstlane(8 * (a * W - 1 - lo_s[a]));
+        // offset of P[a*W - 1 - lo] (wave-uniform): the pair of the 1-based
+        // tap y1 is 8*y1 bytes on
+        const float base = lds_base(__builtin_amdgcn_readfirstlane(8 * (a * W - 1 - lo_s[a])));
 #pragma unroll
         for (int r = 0; r < PY; ++r) {
           const float yr = (A + rt[r]) + m;  // (sin(c)*(jx-m) + cos(c)*(jy-m)) + m
-          // y1 = floor(yr); truncation differs only for yr < 0, whose pairs
-          // (taps below 2) are staged as zeros either way
-          const int y1 = (int)yr;
-          const float fr = __builtin_amdgcn_fractf(yr);  // yr - floor(yr) = yr - y1, exact
-          const float2 pv = *(const float2*)(Pb + (y1 << 3));
+          const float fr = __builtin_amdgcn_fractf(yr);  // yr - y1, y1 = floor(yr) = yr - fr, both exact
+          const unsigned o = __float_as_uint(fmaf(yr - fr, lds_units(8), base));
+          const float2 pv = *(const float2*)((const char*)P + o);
           blk[r] += fmaf(fr, pv.y, pv.x);
         }
       }
@@ -181,13 +184,13 @@ __global__ __launch_bounds__(64 * bp_waves(TY)) void bp_kernel(const BPTask* __r
       for (int a = 0; a < na; ++a) {
         const float2 v = const_f2(sc, a0 + a);
         const float base = fmaf(v.x, xl, k_s[a]);
-        const float2* Pa = P + a * W;
+        const float Pa = lds_base(8 * a * W);
 #pragma unroll
         for (int r = 0; r < PY; ++r) {
           const float yr = fmaf(v.y, yl[r], base);  // detector position - 1 - lo, in (0, W - 1)
-          const int t = (int)yr;
           const float fr = __builtin_amdgcn_fractf(yr);
-          const float2 pv = Pa[t];
+          const unsigned o = __float_as_uint(fmaf(yr - fr, lds_units(8), Pa));
+          const float2 pv = *(const float2*)((const char*)P + o);
           blk[r] += fmaf(fr, pv.y, pv.x);
         }
       }
