@@ -132,6 +132,7 @@ struct BPTask {
   int tile_begin;        // first global tile index of this slice
   int ntx, nty;          // tiles along x and y (at the launch's tile height)
   int nsub;              // 16-row sub-tiles along y, ceil(N / 16)
+  int split_begin;       // first global 64 x 8 tile of this slice (launch_backproject_split)
   const float* sino;     // filtered sinogram (N*T)
   const float* cmask;    // N*N
   const float2* sc;      // per-angle (sin, cos) for backprojection
@@ -224,6 +225,12 @@ struct BPShares { int b[XCDS + 1]; int C; };
 BPShares bp_xcd_shares(const std::vector<float>& w);
 void launch_backproject(const BPTask* d_tasks, int ntasks, int base, int tiles, int ty, bool refpos,
                         const BPShares& sh, hipStream_t s);
+// The same, with the reference's positions, for launches of few tiles
+// (bp_use_split): small tiles, their angle blocks over the waves of a
+// workgroup.  Counted in 64 x 8 tiles, bp_split_tiles(N) (even) per slice.
+int bp_split_tiles(int N);
+bool bp_use_split(int tiles);
+void launch_backproject_split(const BPTask* d_tasks, int ntasks, int base, int tiles, hipStream_t s);
 void launch_cells(const CellTask* d_tasks, int ntasks, int base, int blocks, hipStream_t s);
 // rowterm[t*N + y] = cos(c_t) * ((y+1) - mid), one FP32 product each (the
 // backprojector's row term of tv_hpc.F90:114), for t < T, y < N

@@ -213,7 +213,7 @@ struct Slice {
   double2* fftW = nullptr;
   int ff_begin = 0, ff_n = 0;
   float ff_edge = 0.0f;    // FFT ramp: the tap at distance N-1 (h(2N-1), 0-based)
-  int rf_begin = 0, rf_n = 0, bp_begin = 0, bp_n = 0, cl_begin = 0, cl_n = 0,
+  int rf_begin = 0, rf_n = 0, bp_begin = 0, bp_n = 0, bps_begin = 0, bps_n = 0, cl_begin = 0, cl_n = 0,
       fp_begin = 0, fp_n = 0, fs_begin = 0, fs_n = 0, fl_begin = 0, fl_n = 0, ew_begin = 0, ew_n = 0, sw_begin = 0, sw_n = 0;
 };
 
@@ -253,7 +253,7 @@ struct acu_batch {
   void* tv_mem = nullptr;
   int tv_delta_cap = 0;
   int ff_total = 0, ff_threads = 64;  // FFT ramp blocks (slices within its limit) and threads per workgroup
-  int rf_total = 0, bp_total = 0, cl_total = 0, fp_total = 0, fs_total = 0, ew_total = 0,
+  int rf_total = 0, bp_total = 0, bps_total = 0, cl_total = 0, fp_total = 0, fs_total = 0, ew_total = 0,
       sw_total = 0;
   int fl_total[acu::FL_GROUPS] = {0, 0, 0, 0};  // LDS projector blocks per variant group (lds1, lds2, lds4, cell16)
   // dispatch orders of the LDS projector (fpl_dispatch_order) per variant
@@ -469,7 +469,7 @@ FFTTask ff_task(const Slice& s, const float* in, float* out) {
   return FFTTask{s.N, s.T, lg, s.ff_begin, L == 2 * s.N - 2 ? 1 : 0, s.ff_edge, s.h, s.fftG, s.fftW, in, out};
 }
 BPTask bp_task(const Slice& s, const float* in, float* out) {
-  return BPTask{s.N, s.T, s.mid, s.bp_begin, s.ntx, s.nty, s.nsub, in, s.cmask, s.scbp, s.tact, s.rowterm, out};
+  return BPTask{s.N, s.T, s.mid, s.bp_begin, s.ntx, s.nty, s.nsub, s.bps_begin, in, s.cmask, s.scbp, s.tact, s.rowterm, out};
 }
 FPLTask fpl_task(const Slice& s, const float* img, float* out) {
   static const bool fixed_pitch = [] {
@@ -612,14 +612,16 @@ void assign_bp_shares(acu_batch* b) {
 // Backprojection tile ranges at the batch's tile height (and their XCD
 // shares once the slices' tables exist).
 void assign_bp(acu_batch* b) {
-  int bp = 0;
+  int bp = 0, bps = 0;
   bool tables = true;
   for (auto& s : b->s) {
     s.nty = bp_tiles_y(s.N, b->bp_ty);
     s.bp_begin = bp; s.bp_n = s.ntx * s.nty; bp += s.bp_n;
+    s.bps_begin = bps; s.bps_n = bp_split_tiles(s.N); bps += s.bps_n;
     tables = tables && !s.tact_h.empty();
   }
   b->bp_total = bp;
+  b->bps_total = bps;
   if (tables) assign_bp_shares(b);
 }
 
@@ -727,13 +729,20 @@ void ramp_seq(acu_batch* b, const RFSet& rf, int sl) {
   timed(b->ctx, K_RF, [&] { launch_ramp_any(b, rf, sl, b->ramp_variant); });
 }
 
+// One backprojection launch: of all slices (sl < 0) or one with a task array
+// of all, or of slice sl with a task of its own (own).
+void backproject(acu_batch* b, const BPTask* d, int n, int sl, bool own, bool refpos) {
+  hipStream_t st = b->ctx->stream;
+  const Range r = bp_range(b, sl), rs = sl < 0 ? Range{0, b->bps_total} : Range{b->s[sl].bps_begin, b->s[sl].bps_n};
+  if (refpos && bp_use_split(rs.n)) launch_backproject_split(d, n, own ? 0 : rs.base, rs.n, st);
+  else launch_backproject(d, n, own ? 0 : r.base, r.n, b->bp_ty, refpos, bp_shares(b, sl), st);
+}
+
 // refpos: the backprojection positions (the batch's FBP positions, or
 // tvopt's inside its iteration)
 void iradon_seq(acu_batch* b, const RFSet& rf, const DevArray<BPTask>& bp, int sl, bool refpos) {
-  acu_ctx* c = b->ctx;
-  const Range r2 = bp_range(b, sl);
   ramp_seq(b, rf, sl);
-  timed(c, K_BP, [&] { launch_backproject(bp.d, bp.n, r2.base, r2.n, b->bp_ty, refpos, bp_shares(b, sl), c->stream); });
+  timed(b->ctx, K_BP, [&] { backproject(b, bp.d, bp.n, sl, false, refpos); });
   check_launch();
 }
 
@@ -851,9 +860,7 @@ void fbp_all(acu_batch* b, int sl) {
 
 // the backprojection alone (its ramp-filtered input is already in place)
 void bp_seq(acu_batch* b, const DevArray<BPTask>& bp, int sl, bool refpos) {
-  acu_ctx* c = b->ctx;
-  const Range r2 = bp_range(b, sl);
-  timed(c, K_BP, [&] { launch_backproject(bp.d, bp.n, r2.base, r2.n, b->bp_ty, refpos, bp_shares(b, sl), c->stream); });
+  timed(b->ctx, K_BP, [&] { backproject(b, bp.d, bp.n, sl, false, refpos); });
   check_launch();
 }
 
@@ -1023,9 +1030,9 @@ void bp_dev(acu_batch* b, int sl, float* img, const float* filt) {
   Slice& s = slice_of(b, sl);
   acu_ctx* c = b->ctx;
   BPTask t = bp_task(s, filt, img);
-  t.tile_begin = 0;
+  t.tile_begin = t.split_begin = 0;
   BPTask* d = put_adhoc(b, t);
-  timed(c, K_BP, [&] { launch_backproject(d, 1, 0, s.bp_n, b->bp_ty, b->bp_refpos, s.bp_sh, c->stream); });
+  timed(c, K_BP, [&] { backproject(b, d, 1, sl, true, b->bp_refpos); });
   check_launch();
 }
 

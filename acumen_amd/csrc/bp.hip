@@ -212,7 +212,145 @@ __global__ __launch_bounds__(64 * bp_waves(TY)) void bp_kernel(const BPTask* __r
   }
 }
 
+// Backprojection of small launches, with the reference's positions.  A tile
+// of the kernel above walks its angles serially: 4 waves of 8 rows, so a
+// 257^2 x 180 slice is 45 workgroups on 256 CUs, each a chain of 6 blocks of
+// staging and 32 angles.  Here a workgroup of 8 waves takes a 64 x ROWS tile
+// and every wave another block of 32 angles: each stages its own window in
+// its own part of LDS (BPS_AB angles at a time, no barrier), and the blocks'
+// sums are then added in block order, so the result is the other kernel's
+// bit for bit (but for the sign of the zeros it stores off the mask, as
+// between that kernel's tile heights).  A staged pair serves 8 or 16 rows
+// instead of 32, so a full GPU is better off with the other kernel.
+constexpr int BPS_WAVES = 8;  // waves of a workgroup, one angle block each
+constexpr int BPS_AB = 8;     // angles staged at a time, 8 lanes each
+constexpr int BPS_W = 72;     // window of up to 64 x 16 pixels: hypot(63, 15) + 3.01 = 67.8
+
+__device__ __forceinline__ int find_split_task(const BPTask* tasks, int ntasks, int gtile, int per) {
+  int lo = 0, hi = ntasks - 1;
+  while (lo < hi) {
+    int mid = (lo + hi + 1) >> 1;
+    if (tasks[mid].split_begin / per <= gtile) lo = mid; else hi = mid - 1;
+  }
+  return lo;
+}
+
+template <int ROWS>
+__global__ __launch_bounds__(64 * BPS_WAVES) void bp_split_kernel(const BPTask* __restrict__ tasks, int ntasks,
+                                                                  int base, int ntiles) {
+  constexpr int W = BPS_W, NST = W / 8, OWN = ROWS / BPS_WAVES;  // OWN: rows whose block sums a wave adds
+  static_assert(AB % BPS_AB == 0 && W % 8 == 0 && ROWS % BPS_WAVES == 0 && ROWS <= BP_SUB, "tile shape");
+  static_assert(ROWS * 64 <= 2 * BPS_AB * W, "a wave's block sums fit its pairs' space");
+  __shared__ float2 Ps[BPS_WAVES][BPS_AB * W];
+  const int l = xcd_remap(blockIdx.x, gridDim.x);
+  if (l >= ntiles) return;  // uniform per workgroup
+  const BPTask& tk = tasks[find_split_task(tasks, ntasks, base + l, ROWS / 8)];
+  const int N = tk.N, T = tk.T;
+  const float m = tk.mid;
+  const int local = base + l - tk.split_begin / (ROWS / 8);
+  const int tx = local % tk.ntx, ty = local / tk.ntx;
+  const int x0 = tx * TX, y0 = ty * ROWS;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int x = x0 + lane, yo = y0 + wave * OWN;  // the pixels this thread stores: x, rows yo .. yo + OWN - 1
+  // y0 / BP_SUB < nsub but for the tiles past the image's last rows, which store nothing
+  if (y0 >= N) return;
+  if (!tk.tile_active[(y0 / BP_SUB) * tk.ntx + tx]) {
+#pragma unroll
+    for (int r = 0; r < OWN; ++r)
+      if (x < N && yo + r < N) tk.img[(size_t)(yo + r) * N + x] = 0.0f;
+    return;
+  }
+  const float ux = (float)(x + 1) - m;
+  const float cx0 = (float)(x0 + 1) - m, cx1 = (float)(x0 + TX) - m;
+  const float cy0 = (float)(y0 + 1) - m, cy1 = (float)(y0 + ROWS) - m;
+  float2* P = Ps[wave];
+  float* part = (float*)P;  // the wave's 8 x 64 block sums, once its pairs are read
+  const ACU_GLOBAL float* __restrict__ S = as_global(tk.sino);
+  const ACU_GLOBAL float* __restrict__ sc = as_global((const float*)tk.sc);
+  const int nblk = (T + AB - 1) / AB;
+
+  float acc[OWN];
+#pragma unroll
+  for (int r = 0; r < OWN; ++r) acc[r] = 0.0f;
+  for (int b0 = 0; b0 < nblk; b0 += BPS_WAVES) {
+    const int b = b0 + wave;
+    float blk[ROWS];
+#pragma unroll
+    for (int r = 0; r < ROWS; ++r) blk[r] = 0.0f;
+    for (int a0 = b * AB; a0 < min(T, (b + 1) * AB); a0 += BPS_AB) {
+      const int na = min(BPS_AB, T - a0);
+      // lane l (mod 16) holds angle a0 + l: sine, cosine and window start
+      const int t = min(a0 + (lane & (BPS_AB - 1)), T - 1);
+      const float hs = sc[2 * t], hc = sc[2 * t + 1];
+      const int hlo = (int)floorf(fminf(hs * cx0, hs * cx1) + fminf(hc * cy0, hc * cy1) + m - 1.0f) - 1;
+      // staging: 8 lanes per angle, their loads issued before the first is used
+      const int q = lane >> 3, j = lane & 7, lo = __shfl(hlo, q) + j;
+      const ACU_GLOBAL float* row = S + (size_t)min(a0 + q, T - 1) * N;
+      float2 v[NST];
+#pragma unroll
+      for (int k = 0; k < NST; ++k) {
+        const int dc = min(max(lo + 8 * k, 1), N - 2);  // N >= 3: row[dc + 1] is in the row
+        v[k] = make_float2(row[dc], row[dc + 1]);
+      }
+#pragma unroll
+      for (int k = 0; k < NST; ++k) {
+        const int d = lo + 8 * k;
+        P[q * W + j + 8 * k] = (d >= 1 && d <= N - 2) ? make_float2(v[k].x, v[k].y - v[k].x) : make_float2(0.0f, 0.0f);
+      }
+      __builtin_amdgcn_wave_barrier();  // one wave: its LDS operations are in order
+      for (int a = 0; a < na; ++a) {
+#pragma clang fp contract(off)
+        const float sn = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(hs), a));
+        const float cs = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(hc), a));
+        const float A = sn * ux;
+        const float ob = lds_base(8 * (a * W - 1 - __builtin_amdgcn_readlane(hlo, a)));
+#pragma unroll
+        for (int r = 0; r < ROWS; ++r) {
+          const float yr = (A + cs * ((float)(y0 + r + 1) - m)) + m;
+          const float fr = __builtin_amdgcn_fractf(yr);
+          const unsigned o = __float_as_uint(fmaf(yr - fr, lds_units(8), ob));
+          const float2 pv = *(const float2*)((const char*)P + o);
+          blk[r] += fmaf(fr, pv.y, pv.x);
+        }
+      }
+      __builtin_amdgcn_wave_barrier();
+    }
+#pragma unroll
+    for (int r = 0; r < ROWS; ++r) part[r * 64 + lane] = blk[r];
+    __syncthreads();
+    for (int k = 0; k < min(BPS_WAVES, nblk - b0); ++k)
+#pragma unroll
+      for (int r = 0; r < OWN; ++r) acc[r] += ((const float*)Ps[k])[(wave * OWN + r) * 64 + lane];
+    __syncthreads();
+  }
+#pragma unroll
+  for (int r = 0; r < OWN; ++r)
+    if (x < N && yo + r < N) {
+      const size_t o = (size_t)(yo + r) * N + x;
+      tk.img[o] = tk.cmask[o] * acc[r];
+    }
+}
+
 }  // namespace
+
+int bp_split_tiles(int N) { return bp_tiles_x(N) * ((N + 15) / 16) * 2; }
+
+// us per launch, MI355X: 64 x 8 and 64 x 16 tiles here | 64 x 32 tiles of
+// bp_kernel, by the launch's 64 x 8 tiles:
+//   180 (257^2 x 180) 17, 22 | 65;      612 (513^2 x 360) 56, 55 | 126;
+//   1300 (769^2 x 600) 133, 129 | 207;  2244 (1025^2 x 720) 244, 218 | 269;
+//   2880 (16 x 257^2 x 180) 73, 68 | 75;  4900 (1537^2 x 900) 613, 520 | 469
+bool bp_use_split(int tiles) { return tiles <= 3200; }
+
+void launch_backproject_split(const BPTask* d_tasks, int ntasks, int base, int tiles, hipStream_t s) {
+  if (tiles <= 0) return;
+  if (tiles <= 800)
+    hipLaunchKernelGGL(bp_split_kernel<8>, dim3(xcd_grid(tiles)), dim3(64 * BPS_WAVES), 0, s, d_tasks, ntasks, base,
+                       tiles);
+  else
+    hipLaunchKernelGGL(bp_split_kernel<16>, dim3(xcd_grid(tiles / 2)), dim3(64 * BPS_WAVES), 0, s, d_tasks, ntasks,
+                       base / 2, tiles / 2);
+}
 
 __global__ __launch_bounds__(256) void rowterm_kernel(const float2* __restrict__ sc, int N, int T, float mid,
                                                       float* __restrict__ out) {
