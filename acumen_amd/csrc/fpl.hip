@@ -36,6 +36,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <type_traits>
 
 namespace acu {
 namespace {
@@ -175,113 +176,112 @@ __device__ __forceinline__ void fpl_body(const FPLTask& tk, int gb, float* __res
         }
       }
     } else {
-      const bool xin = cok && gx >= 1 && gx <= N;
-      for (int ly0 = rp; ly0 < bh; ly0 += 2 * FPL_SB) {
-        float v[FPL_SB];
+      // a box that crosses the image's edge: every load at a position clamped
+      // into the image, then zero where the pixel is outside it
+      if (cok) {
+        const bool xin = gx >= 1 && gx <= N;
+        const ACU_GLOBAL float* col0 = img + (min(max(gx, 1), N) - 1);
+        for (int ly0 = rp; ly0 < bh; ly0 += 2 * FPL_SB) {
+          float v[FPL_SB];
 #pragma unroll
-        for (int k = 0; k < FPL_SB; ++k) {
-          const int gy = by0 + ly0 + 2 * k;
-          v[k] = 0.0f;
-          if (xin && ly0 + 2 * k < bh && gy >= 1 && gy <= N)
-            v[k] = *(const ACU_GLOBAL float*)(ib + (goff + (unsigned)k * gstep));
-        }
+          for (int k = 0; k < FPL_SB; ++k)
+            v[k] = col0[(unsigned)(min(max(by0 + ly0 + 2 * k, 1), N) - 1) * (unsigned)N];
 #pragma unroll
-        for (int k = 0; k < FPL_SB; ++k) {
-          if (cok && ly0 + 2 * k < bh) lrow[2 * k * PITCH] = v[k];
-          nzb |= __float_as_uint(v[k]) << 1;
+          for (int k = 0; k < FPL_SB; ++k) {
+            const int gy = by0 + ly0 + 2 * k;
+            const float w = xin && gy >= 1 && gy <= N ? v[k] : 0.0f;
+            if (ly0 + 2 * k < bh) lrow[2 * k * PITCH] = w;
+            nzb |= __float_as_uint(w) << 1;
+          }
+          lrow += 2 * FPL_SB * PITCH;
         }
-        goff += (unsigned)FPL_SB * gstep;
-        lrow += 2 * FPL_SB * PITCH;
       }
     }
     return nzb != 0u;
   };
-  // this wave's samples of the chunk from the staged box B
-  auto compute = [&](const FplBox& B) {
-    const int bx0 = B.x0, by0 = B.y0, bw = B.w, bh = B.h;
-    const bool interior = bx0 >= 2 && by0 >= 2 && bx0 + bw - 1 <= N && by0 + bh - 1 <= N;
-    if (interior) {
-      // every cell in the box passes the bounds test: fast positions, no
-      // branches; an inactive (ray, angle) reads a fixed in-box pixel and
-      // its sum is never stored
-      float bxl[AL], byl[AL], cj[AL], sj[AL];
+  // this wave's samples of the chunk from the staged box B.  EXACT (border
+  // chunks): the reference's positions and bounds test; a sample that fails
+  // the test adds +0, which changes no sum that started at +0.  Else
+  // (interior chunks: every cell in the box passes the test) fast positions
+  // and no test.  An inactive (ray, angle) reads a fixed in-box pixel and its
+  // sum is never stored, so there are no branches.
+  auto compute = [&](const FplBox& B, auto exact) {
+    constexpr bool EXACT = decltype(exact)::value;
+    const int bx0 = B.x0, by0 = B.y0;
+    float bxl[AL], byl[AL], cj[AL], sj[AL];
 #pragma unroll
-      for (int j = 0; j < AL; ++j) {
-        cj[j] = act[j] ? c[j] : 0.0f;
-        sj[j] = act[j] ? s[j] : 0.0f;
+    for (int j = 0; j < AL; ++j) {
+      cj[j] = act[j] ? c[j] : 0.0f;
+      sj[j] = act[j] ? s[j] : 0.0f;
+      if (EXACT) {
+        bxl[j] = act[j] ? sy[j] : m - (float)(bx0 + 1);
+        byl[j] = act[j] ? cyv[j] : (float)(by0 + 1) - m;
+      } else {
         bxl[j] = act[j] ? (m - sy[j]) - (float)bx0 : 1.0f;
         byl[j] = act[j] ? (m + cyv[j]) - (float)by0 : 1.0f;
       }
-      // Software-pipelined over two groups of the lane's angles: a group's
-      // taps for the next step are read from LDS right after its lerps of
-      // this step, so they are in flight while the other group's lerps run
-      // (a scheduling barrier keeps the compiler from merging the groups
-      // back into one wait).  Each angle still adds its samples in step
-      // order.  u = x - m is an integer below 2^24 in magnitude, so
-      // stepping it by 1.0f gives exactly (float)x - m without a conversion.
-      constexpr int NG = AL < 2 ? AL : 2;  // angle groups
-      constexpr int H = AL / NG;           // angles per group
-      struct Taps { float fx, fy, v00, v10, v01, v11; };
-      Taps tp[NG][H];
-      auto fetch = [&](float uu, int g) {
+    }
+    // Software-pipelined over two groups of the lane's angles: a group's
+    // taps for the next step are read from LDS right after its lerps of
+    // this step, so they are in flight while the other group's lerps run
+    // (a scheduling barrier keeps the compiler from merging the groups
+    // back into one wait).  Each angle still adds its samples in step
+    // order.  u = x - m is an integer below 2^24 in magnitude, so
+    // stepping it by 1.0f gives exactly (float)x - m without a conversion.
+    constexpr int NG = AL < 2 ? AL : 2;  // angle groups
+    constexpr int H = AL / NG;           // angles per group
+    struct Taps { float fx, fy, v00, v10, v01, v11; bool ok; };
+    Taps tp[NG][H];
+    auto fetch = [&](float uu, int g) {
 #pragma unroll
-        for (int q = 0; q < H; ++q) {
-          const int j = g * H + q;
+      for (int q = 0; q < H; ++q) {
+        const int j = g * H + q;
+        const float* p0;
+        if (EXACT) {
+          const float xr = (cj[j] * uu - bxl[j]) + m;
+          const float yr = (sj[j] * uu + byl[j]) + m;
+          const float fxr = floorf(xr), fyr = floorf(yr);
+          const int x1 = (int)fxr, y1 = (int)fyr;
+          tp[g][q].ok = (unsigned)(x1 - 2) <= (unsigned)(N - 3) && (unsigned)(y1 - 2) <= (unsigned)(N - 3);
+          tp[g][q].fx = xr - fxr;
+          tp[g][q].fy = yr - fyr;
+          p0 = box + (__mul24(y1 - by0, PITCH) + (x1 - bx0));
+        } else {
           const float xl = fmaf(cj[j], uu, bxl[j]);
           const float yl = fmaf(sj[j], uu, byl[j]);
           tp[g][q].fx = __builtin_amdgcn_fractf(xl);
           tp[g][q].fy = __builtin_amdgcn_fractf(yl);
-          const float* p0 = (const float*)((const char*)box + fpl_cell_offset<PITCH>(xl, yl));
-          tp[g][q].v00 = p0[0];
-          tp[g][q].v10 = p0[1];
-          tp[g][q].v01 = p0[PITCH];
-          tp[g][q].v11 = p0[PITCH + 1];
+          p0 = (const float*)((const char*)box + fpl_cell_offset<PITCH>(xl, yl));
         }
-      };
-      auto sample = [&](int g) {
-#pragma unroll
-        for (int q = 0; q < H; ++q) {
-          const Taps& t = tp[g][q];
-          const float top = fmaf(t.fx, t.v10 - t.v00, t.v00);
-          const float bot = fmaf(t.fx, t.v11 - t.v01, t.v01);
-          acc[g * H + q] += fmaf(t.fy, bot - top, top);
-        }
-      };
-      float u = (float)c0 - m;
-#pragma unroll
-      for (int g = 0; g < NG; ++g) fetch(u, g);
-      for (int x = c0; x < c1; ++x, u += 1.0f) {
-#pragma unroll
-        for (int g = 0; g < NG; ++g) {
-          sample(g);
-          fetch(u + 1.0f, g);
-          __builtin_amdgcn_sched_barrier(0);
-        }
+        tp[g][q].v00 = p0[0];
+        tp[g][q].v10 = p0[1];
+        tp[g][q].v01 = p0[PITCH];
+        tp[g][q].v11 = p0[PITCH + 1];
       }
+    };
+    auto sample = [&](int g) {
 #pragma unroll
-      for (int g = 0; g < NG; ++g) sample(g);  // step c1
-    } else {
-      // border chunk: the reference's positions and bounds test
-      for (int x = c0; x <= c1; ++x) {
-        const float u = (float)x - m;
+      for (int q = 0; q < H; ++q) {
+        const Taps& t = tp[g][q];
+        const float top = fmaf(t.fx, t.v10 - t.v00, t.v00);
+        const float bot = fmaf(t.fx, t.v11 - t.v01, t.v01);
+        const float v = fmaf(t.fy, bot - top, top);
+        acc[g * H + q] += EXACT && !t.ok ? 0.0f : v;
+      }
+    };
+    float u = (float)c0 - m;
 #pragma unroll
-        for (int j = 0; j < AL; ++j) {
-          if (!act[j]) continue;
-          const float xr = (c[j] * u - sy[j]) + m;
-          const float yr = (s[j] * u + cyv[j]) + m;
-          const float fxr = floorf(xr), fyr = floorf(yr);
-          const int x1 = (int)fxr, y1 = (int)fyr;
-          if (x1 >= 2 && x1 <= N - 1 && y1 >= 2 && y1 <= N - 1) {
-            const float fx = xr - fxr, fy = yr - fyr;
-            const float* p0 = box + (__mul24(y1 - by0, PITCH) + (x1 - bx0));
-            const float v00 = p0[0], v10 = p0[1], v01 = p0[PITCH], v11 = p0[PITCH + 1];
-            const float top = fmaf(fx, v10 - v00, v00);
-            const float bot = fmaf(fx, v11 - v01, v01);
-            acc[j] += fmaf(fy, bot - top, top);
-          }
-        }
+    for (int g = 0; g < NG; ++g) fetch(u, g);
+    for (int x = c0; x < c1; ++x, u += 1.0f) {
+#pragma unroll
+      for (int g = 0; g < NG; ++g) {
+        sample(g);
+        fetch(u + 1.0f, g);
+        __builtin_amdgcn_sched_barrier(0);
       }
     }
+#pragma unroll
+    for (int g = 0; g < NG; ++g) sample(g);  // step c1
   };
   // this wave's samples of the chunk, bilinear cells from global memory
   auto gather = [&]() {
@@ -326,7 +326,10 @@ __device__ __forceinline__ void fpl_body(const FPLTask& tk, int gb, float* __res
       __syncthreads();
       const bool nonzero = *flag != 0.0f;
       if (threadIdx.x == 0) red[0][2 + ((kst + 1) & 1)] = 0.0f;
-      if (nonzero) compute(B);
+      if (nonzero) {
+        if (B.x0 >= 2 && B.y0 >= 2 && B.x0 + B.w - 1 <= N && B.y0 + B.h - 1 <= N) compute(B, std::false_type{});
+        else compute(B, std::true_type{});
+      }
       __syncthreads();
       ++kst;
     } else {
