@@ -30,8 +30,11 @@
 //  * border chunks: positions are the reference's FP32 values (c*u, s*u,
 //    s*ym, c*ym rounded once, summed in its order, no contraction) and the
 //    bounds test is applied, so every edge decision is the reference's own;
+//    the same loop without branches (a sample that fails the test adds +0);
 //  * a chunk whose box does not fit the LDS budget falls back to gathering
 //    the bilinear cells of fp.hip from global memory (exact positions).
+// Small launches split a block's angles over workgroups and stage a chunk
+// ahead through registers (launch_forward_lds).
 #include "fpl_common.hpp"
 
 #include <algorithm>
@@ -41,12 +44,22 @@
 namespace acu {
 namespace {
 
-constexpr int FPL_THREADS = 256;
 #ifndef ACUMEN_FPL_AMAX
 #define ACUMEN_FPL_AMAX 2
 #endif
 constexpr int AMAX = ACUMEN_FPL_AMAX;  // max angles per lane (1, 2 or 4)
 constexpr int FPL_SB = 8;  // staging loads in flight per lane
+constexpr int FPL_THREADS = 256;
+// rows of a box that a thread stages, two rows apart, and the LDS floats
+// that every pitch's boxes then take
+constexpr int fpl_pre_rows(int pitch) { return (FPL_CAP / pitch + 1) / 2; }
+constexpr int fpl_pre_cap() {
+  int c = 0;
+  for (int p : FPL_PITCHES) c = 2 * fpl_pre_rows(p) * p > c ? 2 * fpl_pre_rows(p) * p : c;
+  return c;
+}
+constexpr int FPL_PRE_CAP = fpl_pre_cap();
+constexpr int FPL_SPLIT_MAX = 1536;  // workgroups of a split launch: two rounds of 3 per CU (their LDS)
 constexpr int FPL_SLOTS = 1024;  // workgroups resident at once: 4 per CU x 256 CUs
 
 // Byte offset 4*(iy*PITCH + ix) of the box cell of a position (xl, yl) with
@@ -70,9 +83,16 @@ __device__ __forceinline__ unsigned fpl_cell_offset(float xl, float yl) {
 // One workgroup's work; PITCH is the LDS row pitch of its boxes (which of
 // a few pitches spreads the lanes' taps best over the banks depends on the
 // angles, see fpl_pitch_classes).
-template <int AL, int PITCH>
-__device__ __forceinline__ void fpl_body(const FPLTask& tk, int gb, float* __restrict__ box, float (*red)[4]) {
+// BLK: angles of a block (64 rays x BLK angles share boxes and chunks).  A
+// block is SPLIT workgroups, each with the angles of its share `sub`.  PRE
+// (small launches): a chunk's box is loaded into registers while the chunk
+// before it is sampled.
+template <int BLK, int SPLIT, bool PRE, int PITCH>
+__device__ __forceinline__ void fpl_body(const FPLTask& tk, int gb, int sub, float* __restrict__ box,
+                                         float (*red)[4]) {
 #pragma clang fp contract(off)
+  constexpr int AL = BLK / (4 * SPLIT);  // angles per lane
+  static_assert(BLK % (4 * SPLIT) == 0, "work split");
   static_assert(PITCH + 1 <= 255, "ds_read2 offsets");
   const int N = tk.N, T = tk.T;
   const float m = tk.mid;
@@ -80,8 +100,8 @@ __device__ __forceinline__ void fpl_body(const FPLTask& tk, int gb, float* __res
   const int rb = local / tk.nab, ab = local - rb * tk.nab;  // ray-block-major
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   // wave w: rays 16w..16w+15 (lane & 15) of the block; lane group g = lane >> 4
-  // takes angles g, g + 4, ... (so the 64 lanes of one instruction cover 16 rays
-  // at 4 consecutive angles)
+  // takes angles g, g + 4, ... of the workgroup's share (so the 64 lanes of
+  // one instruction cover 16 rays at 4 consecutive angles)
   const int ray = rb * 64 + wave * 16 + (lane & 15);
   const float ym = (float)(min(ray, N - 1) + 1) - m;
 
@@ -90,19 +110,26 @@ __device__ __forceinline__ void fpl_body(const FPLTask& tk, int gb, float* __res
   int ang[AL];
   float lu0 = 1e30f, lu1 = -1e30f;
 #pragma unroll
-  for (int j = 0; j < AL; ++j) {
-    ang[j] = ab * 4 * AL + (lane >> 4) + 4 * j;
-    act[j] = ang[j] < T && ray < N;
-    const float2 v = const_f2(tk.sc, min(ang[j], T - 1));
-    s[j] = v.x;
-    c[j] = v.y;
-    sy[j] = s[j] * ym;   // one rounding each (tv_hpc.F90:143-144)
-    cyv[j] = c[j] * ym;
-    acc[j] = 0.0f;
-    if (act[j]) {
+  for (int i = 0; i < BLK / 4; ++i) {  // every angle of the block: the step window is the block's
+    const int a = ab * BLK + (lane >> 4) + 4 * i;
+    const bool on = a < T && ray < N;
+    const float2 v = const_f2(tk.sc, min(a, T - 1));
+    const float sya = v.x * ym, cya = v.y * ym;  // one rounding each (tv_hpc.F90:143-144)
+#pragma unroll
+    for (int j = 0; j < AL; ++j)
+      if (SPLIT == 1 ? i == j : i == sub * AL + j) {
+        ang[j] = a;
+        act[j] = on;
+        s[j] = v.x;
+        c[j] = v.y;
+        sy[j] = sya;
+        cyv[j] = cya;
+        acc[j] = 0.0f;
+      }
+    if (on) {
       float ua, ub, va, vb;
-      fpl_urange(m - sy[j], c[j], 1.99f, (float)N + 0.01f, ua, ub);
-      fpl_urange(m + cyv[j], s[j], 1.99f, (float)N + 0.01f, va, vb);
+      fpl_urange(m - sya, v.y, 1.99f, (float)N + 0.01f, ua, ub);
+      fpl_urange(m + cya, v.x, 1.99f, (float)N + 0.01f, va, vb);
       const float u0 = fmaxf(ua, va), u1 = fminf(ub, vb);
       if (u0 <= u1) { lu0 = fminf(lu0, u0); lu1 = fmaxf(lu1, u1); }
     }
@@ -124,19 +151,20 @@ __device__ __forceinline__ void fpl_body(const FPLTask& tk, int gb, float* __res
 
   const ACU_GLOBAL float* __restrict__ img = as_global(tk.img);
   const int r1 = min(N - 1, rb * 64 + 63);
-  const FplBoxGeom bg = fpl_box_geom(tk, ab * 4 * AL, 4 * AL, rb * 64, r1, lane);
+  const FplBoxGeom bg = fpl_box_geom(tk, ab * BLK, BLK, rb * 64, r1, lane);
   int c0 = 0, c1 = -1;
 
-  // stage the box B of the chunk [c0, c1] into LDS (all four waves);
-  // returns whether this thread staged a value other than +-0
+  // row staging: lanes cover 128 columns, the wave pair (wave >> 1) picks the
+  // row parity
+  const int rp = __builtin_amdgcn_readfirstlane(wave >> 1);
+  const int col = lane + ((wave & 1) << 6);
+  // stage the box B of the chunk [c0, c1] into LDS (all waves); returns
+  // whether this thread staged a value other than +-0.  FPL_SB loads in
+  // flight per lane, 32-bit byte offsets from the image base and LDS stores
+  // at immediate offsets.
   auto stage = [&](const FplBox& B) {
     unsigned nzb = 0u;  // OR of the staged values' bits without the sign
     const int bx0 = B.x0, by0 = B.y0, bw = B.w, bh = B.h;
-    // row staging: lanes cover 128 columns, the wave pair (wave >> 1) picks
-    // the row parity, FPL_SB loads in flight per lane; 32-bit byte offsets
-    // from the image base and LDS stores at immediate offsets
-    const int rp = __builtin_amdgcn_readfirstlane(wave >> 1);
-    const int col = lane + ((wave & 1) << 6);
     const int gx = bx0 + col;
     const bool cok = col < bw;
     const ACU_GLOBAL char* ib = (const ACU_GLOBAL char*)img;
@@ -199,6 +227,37 @@ __device__ __forceinline__ void fpl_body(const FPLTask& tk, int gb, float* __res
     }
     return nzb != 0u;
   };
+  // The same a chunk ahead: load(B) issues every load of box B, store() puts
+  // them into LDS once the chunk before is sampled.  Buffer loads: a pixel
+  // outside the image is out of the buffer's range (or gets an offset that
+  // is) and loads as zero.  Rows past the box's last are loaded and stored
+  // with the rest (the LDS array has room for them).
+  constexpr int NR = PRE ? fpl_pre_rows(PITCH) : 1;
+  float pv[NR];
+  const auto rsrc = __builtin_amdgcn_make_buffer_rsrc((void*)tk.img, 0, 4u * (unsigned)N * (unsigned)N, 0x00020000);
+  auto load = [&](const FplBox& B) {
+    const int gx = B.x0 + col;
+    unsigned off = 4u * (unsigned)((B.y0 + rp - 1) * N + (gx - 1));
+    // x outside the image: an offset past any row of the box; the last valid byte is below 2^30
+    if (gx < 1 || gx > N || col >= B.w) off = 0x80000000u;
+#pragma unroll
+    for (int k = 0; k < NR; ++k) {
+      pv[k] = __int_as_float(__builtin_amdgcn_raw_buffer_load_b32(rsrc, (int)off, 0, 0));
+      off += 8u * (unsigned)N;
+    }
+  };
+  auto store = [&](const FplBox& B) {
+    unsigned nzb = 0u;
+    if (col < B.w) {
+      float* lrow = box + (rp * PITCH + col);
+#pragma unroll
+      for (int k = 0; k < NR; ++k) {
+        lrow[2 * k * PITCH] = pv[k];
+        nzb |= __float_as_uint(pv[k]) << 1;
+      }
+    }
+    return nzb != 0u;
+  };
   // this wave's samples of the chunk from the staged box B.  EXACT (border
   // chunks): the reference's positions and bounds test; a sample that fails
   // the test adds +0, which changes no sum that started at +0.  Else
@@ -221,6 +280,73 @@ __device__ __forceinline__ void fpl_body(const FPLTask& tk, int gb, float* __res
         byl[j] = act[j] ? (m + cyv[j]) - (float)by0 : 1.0f;
       }
     }
+    struct Taps { float fx, fy, v00, v10, v01, v11; bool ok; };
+    auto fetch = [&](float uu, int j, Taps& t) {
+      const float* p0;
+      if (EXACT) {
+        const float xr = (cj[j] * uu - bxl[j]) + m;
+        const float yr = (sj[j] * uu + byl[j]) + m;
+        const float fxr = floorf(xr), fyr = floorf(yr);
+        const int x1 = (int)fxr, y1 = (int)fyr;
+        t.ok = (unsigned)(x1 - 2) <= (unsigned)(N - 3) && (unsigned)(y1 - 2) <= (unsigned)(N - 3);
+        t.fx = xr - fxr;
+        t.fy = yr - fyr;
+        p0 = box + (__mul24(y1 - by0, PITCH) + (x1 - bx0));
+      } else {
+        const float xl = fmaf(cj[j], uu, bxl[j]);
+        const float yl = fmaf(sj[j], uu, byl[j]);
+        t.fx = __builtin_amdgcn_fractf(xl);
+        t.fy = __builtin_amdgcn_fractf(yl);
+        p0 = (const float*)((const char*)box + fpl_cell_offset<PITCH>(xl, yl));
+      }
+      t.v00 = p0[0];
+      t.v10 = p0[1];
+      t.v01 = p0[PITCH];
+      t.v11 = p0[PITCH + 1];
+    };
+    auto sample = [&](const Taps& t) {
+      const float top = fmaf(t.fx, t.v10 - t.v00, t.v00);
+      const float bot = fmaf(t.fx, t.v11 - t.v01, t.v01);
+      const float v = fmaf(t.fy, bot - top, top);
+      return EXACT && !t.ok ? 0.0f : v;
+    };
+    if constexpr (PRE) {
+      // One to three waves per SIMD and one angle per lane: two groups of
+      // two steps in flight, then the steps left over one at a time.
+      static_assert(AL == 1, "one angle per lane");
+      Taps tp[2][2];
+      int x = c0;
+      float u = (float)c0 - m;
+      auto fetch2 = [&](float uu, int g) {
+        fetch(uu, 0, tp[g][0]);
+        fetch(uu + 1.0f, 0, tp[g][1]);
+      };
+      auto sample2 = [&](int g) {
+        acc[0] += sample(tp[g][0]);
+        acc[0] += sample(tp[g][1]);
+      };
+      if (c1 - c0 >= 3) {
+        fetch2(u, 0);
+        fetch2(u + 2.0f, 1);
+        for (; x + 7 <= c1; x += 4, u += 4.0f) {
+          sample2(0);
+          fetch2(u + 4.0f, 0);
+          __builtin_amdgcn_sched_barrier(0);
+          sample2(1);
+          fetch2(u + 6.0f, 1);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        sample2(0);
+        sample2(1);
+        x += 4;
+        u += 4.0f;
+      }
+      for (; x <= c1; ++x, u += 1.0f) {
+        fetch(u, 0, tp[0][0]);
+        acc[0] += sample(tp[0][0]);
+      }
+      return;
+    }
     // Software-pipelined over two groups of the lane's angles: a group's
     // taps for the next step are read from LDS right after its lerps of
     // this step, so they are in flight while the other group's lerps run
@@ -230,89 +356,90 @@ __device__ __forceinline__ void fpl_body(const FPLTask& tk, int gb, float* __res
     // stepping it by 1.0f gives exactly (float)x - m without a conversion.
     constexpr int NG = AL < 2 ? AL : 2;  // angle groups
     constexpr int H = AL / NG;           // angles per group
-    struct Taps { float fx, fy, v00, v10, v01, v11; bool ok; };
     Taps tp[NG][H];
-    auto fetch = [&](float uu, int g) {
-#pragma unroll
-      for (int q = 0; q < H; ++q) {
-        const int j = g * H + q;
-        const float* p0;
-        if (EXACT) {
-          const float xr = (cj[j] * uu - bxl[j]) + m;
-          const float yr = (sj[j] * uu + byl[j]) + m;
-          const float fxr = floorf(xr), fyr = floorf(yr);
-          const int x1 = (int)fxr, y1 = (int)fyr;
-          tp[g][q].ok = (unsigned)(x1 - 2) <= (unsigned)(N - 3) && (unsigned)(y1 - 2) <= (unsigned)(N - 3);
-          tp[g][q].fx = xr - fxr;
-          tp[g][q].fy = yr - fyr;
-          p0 = box + (__mul24(y1 - by0, PITCH) + (x1 - bx0));
-        } else {
-          const float xl = fmaf(cj[j], uu, bxl[j]);
-          const float yl = fmaf(sj[j], uu, byl[j]);
-          tp[g][q].fx = __builtin_amdgcn_fractf(xl);
-          tp[g][q].fy = __builtin_amdgcn_fractf(yl);
-          p0 = (const float*)((const char*)box + fpl_cell_offset<PITCH>(xl, yl));
-        }
-        tp[g][q].v00 = p0[0];
-        tp[g][q].v10 = p0[1];
-        tp[g][q].v01 = p0[PITCH];
-        tp[g][q].v11 = p0[PITCH + 1];
-      }
-    };
-    auto sample = [&](int g) {
-#pragma unroll
-      for (int q = 0; q < H; ++q) {
-        const Taps& t = tp[g][q];
-        const float top = fmaf(t.fx, t.v10 - t.v00, t.v00);
-        const float bot = fmaf(t.fx, t.v11 - t.v01, t.v01);
-        const float v = fmaf(t.fy, bot - top, top);
-        acc[g * H + q] += EXACT && !t.ok ? 0.0f : v;
-      }
-    };
     float u = (float)c0 - m;
 #pragma unroll
-    for (int g = 0; g < NG; ++g) fetch(u, g);
+    for (int j = 0; j < AL; ++j) fetch(u, j, tp[j / H][j % H]);
     for (int x = c0; x < c1; ++x, u += 1.0f) {
 #pragma unroll
       for (int g = 0; g < NG; ++g) {
-        sample(g);
-        fetch(u + 1.0f, g);
+#pragma unroll
+        for (int q = 0; q < H; ++q) acc[g * H + q] += sample(tp[g][q]);
+#pragma unroll
+        for (int q = 0; q < H; ++q) fetch(u + 1.0f, g * H + q, tp[g][q]);
         __builtin_amdgcn_sched_barrier(0);
       }
     }
 #pragma unroll
-    for (int g = 0; g < NG; ++g) sample(g);  // step c1
+    for (int j = 0; j < AL; ++j) acc[j] += sample(tp[j / H][j % H]);  // step c1
   };
-  // this wave's samples of the chunk, bilinear cells from global memory
+  // this wave's samples of the chunk, bilinear cells from global memory, GL
+  // of them in flight per lane; an inactive (ray, angle) reads cell (0, 0).
+  // us per launch at 2049^2 x 48 (3.75 degrees between angles, nearly every
+  // chunk) with 1 (a branch per sample), 4, 8 and 16: 934, 812, 876, 1897
+  // (more lines in flight than the L1 holds); 2 x 2049^2 x 1500 inside TV
+  // (a tenth of the chunks): 4.73 ms with 1, 4.62 with 4.
+  constexpr int GL = 4, GU = GL / AL;  // GU steps at a time
   auto gather = [&]() {
     const int P = N + 1;
     const float fN = (float)N;
-    for (int x = c0; x <= c1; ++x) {
-      const float u = (float)x - m;
+    float cj[AL], sj[AL], sx[AL], cy[AL];
 #pragma unroll
-      for (int j = 0; j < AL; ++j) {
-        if (!act[j]) continue;
-        const float xr = (c[j] * u - sy[j]) + m;
-        const float yr = (s[j] * u + cyv[j]) + m;
-        const int cx = (int)__builtin_amdgcn_fmed3f(xr, 0.0f, fN);
-        const int cyi = (int)__builtin_amdgcn_fmed3f(yr, 0.0f, fN);
-        const float wx = __builtin_amdgcn_fractf(xr), wy = __builtin_amdgcn_fractf(yr);
-        const float4 q = global_f4(as_global(tk.cells), (unsigned)(__mul24(cyi, P) + cx));
-        const float t1 = fmaf(wx, q.w, q.z);
-        const float t2 = fmaf(wx, q.y, q.x);
-        acc[j] += fmaf(wy, t1, t2);
+    for (int j = 0; j < AL; ++j) {
+      cj[j] = act[j] ? c[j] : 0.0f;
+      sj[j] = act[j] ? s[j] : 0.0f;
+      sx[j] = act[j] ? sy[j] : m;
+      cy[j] = act[j] ? cyv[j] : -m;
+    }
+    for (int x = c0; x <= c1; x += GU) {
+      float4 q[GU][AL];
+      float wx[GU][AL], wy[GU][AL];
+#pragma unroll
+      for (int k = 0; k < GU; ++k) {
+        const float u = (float)min(x + k, c1) - m;
+#pragma unroll
+        for (int j = 0; j < AL; ++j) {
+          const float xr = (cj[j] * u - sx[j]) + m;
+          const float yr = (sj[j] * u + cy[j]) + m;
+          const int cx = (int)__builtin_amdgcn_fmed3f(xr, 0.0f, fN);
+          const int cyi = (int)__builtin_amdgcn_fmed3f(yr, 0.0f, fN);
+          wx[k][j] = __builtin_amdgcn_fractf(xr);
+          wy[k][j] = __builtin_amdgcn_fractf(yr);
+          q[k][j] = global_f4(as_global(tk.cells), (unsigned)(__mul24(cyi, P) + cx));
+        }
+      }
+#pragma unroll
+      for (int k = 0; k < GU; ++k) {
+        if (x + k > c1) break;
+#pragma unroll
+        for (int j = 0; j < AL; ++j) {
+          const float t1 = fmaf(wx[k][j], q[k][j].w, q[k][j].z);
+          const float t2 = fmaf(wx[k][j], q[k][j].y, q[k][j].x);
+          acc[j] += fmaf(wy[k][j], t1, t2);
+        }
       }
     }
   };
   auto fits = [](const FplBox& B) { return B.w > 0 && B.h > 0 && B.w <= PITCH && B.h * PITCH <= FPL_CAP; };
 
   int kst = 0;  // chunks staged so far
+  FplBox B, nx;
+  if (PRE && XS <= XE) {
+    nx = fpl_box(bg, m, XS, min(XE, XS + FPL_U - 1));
+    if (nx.any && fits(nx)) load(nx);
+  }
   for (c0 = XS; c0 <= XE; c0 += FPL_U) {
     c1 = min(XE, c0 + FPL_U - 1);
     // bounding box of the chunk's samples (fpl_box: wave-uniform, no LDS)
-    const FplBox B = fpl_box(bg, m, c0, c1);
-    if (!B.any) continue;  // no active lane in this workgroup (uniform)
-    if (fits(B)) {
+    B = PRE ? nx : fpl_box(bg, m, c0, c1);
+    const bool fit = B.any && fits(B);  // B.any: an active lane in this workgroup (uniform)
+    bool nz = false;
+    if (fit) nz = PRE ? store(B) : stage(B);
+    if (PRE && c1 < XE) {
+      nx = fpl_box(bg, m, c1 + 1, min(XE, c1 + FPL_U));
+      if (nx.any && fits(nx)) load(nx);
+    }
+    if (fit) {
       // A box of zeros (+-0) adds exactly +0 to every sum (with taps of
       // either sign, fma(fx, v10 - v00, v00) and the lerps after it are +0,
       // and a sum started at +0 never holds -0), so its samples are
@@ -322,7 +449,7 @@ __device__ __forceinline__ void fpl_body(const FPLTask& tk, int gb, float* __res
       // nobody reads after the previous chunk's last barrier and nobody sets
       // before this chunk's last barrier.
       float* flag = &red[0][2 + (kst & 1)];
-      if (stage(B)) *flag = 1.0f;
+      if (nz) *flag = 1.0f;
       __syncthreads();
       const bool nonzero = *flag != 0.0f;
       if (threadIdx.x == 0) red[0][2 + ((kst + 1) & 1)] = 0.0f;
@@ -332,7 +459,7 @@ __device__ __forceinline__ void fpl_body(const FPLTask& tk, int gb, float* __res
       }
       __syncthreads();
       ++kst;
-    } else {
+    } else if (B.any) {
       gather();  // box too large for LDS
     }
   }
@@ -341,26 +468,25 @@ __device__ __forceinline__ void fpl_body(const FPLTask& tk, int gb, float* __res
     if (act[j]) tk.sino[(size_t)ang[j] * N + ray] = acc[j] / (float)N;
 }
 
-template <int AL>
-__global__ __launch_bounds__(FPL_THREADS) void fpl_kernel(const FPLTask* __restrict__ tasks, int ntasks,
-                                                          int base, int nblocks,
-                                                          const int* __restrict__ order) {
-  __shared__ float box[FPL_CAP];
-  __shared__ float red[4][4];  // per-wave min x, min y, max x, max y (or step range)
-  const int lbk = xcd_remap(blockIdx.x, gridDim.x);
+template <int BLK, int SPLIT, bool PRE>
+__global__ __launch_bounds__(FPL_THREADS) void fpl_kernel(const FPLTask* __restrict__ tasks, int ntasks, int base,
+                                                          int nblocks, const int* __restrict__ order) {
+  __shared__ float box[PRE ? FPL_PRE_CAP : FPL_CAP];
+  __shared__ float red[4][4];  // per-wave step range, and (row 0) the flags of boxes that are not all zero
+  const int lwg = xcd_remap(blockIdx.x, gridDim.x), lbk = lwg / SPLIT, sub = lwg % SPLIT;
   if (lbk >= nblocks) return;
   const int gb = base + (order ? order[lbk] : lbk);
   const FPLTask& tk = tasks[fpl_find_task(tasks, ntasks, gb)];
   const int ab = (gb - tk.block_begin) % tk.nab;
   switch (tk.pclass ? (int)tk.pclass[ab] : FPL_PCLASS_DEFAULT) {
-    case 0: fpl_body<AL, FPL_PITCHES[0]>(tk, gb, box, red); break;
-    case 1: fpl_body<AL, FPL_PITCHES[1]>(tk, gb, box, red); break;
-    case 2: fpl_body<AL, FPL_PITCHES[2]>(tk, gb, box, red); break;
-    case 4: fpl_body<AL, FPL_PITCHES[4]>(tk, gb, box, red); break;
-    case 5: fpl_body<AL, FPL_PITCHES[5]>(tk, gb, box, red); break;
-    case 6: fpl_body<AL, FPL_PITCHES[6]>(tk, gb, box, red); break;
-    case 7: fpl_body<AL, FPL_PITCHES[7]>(tk, gb, box, red); break;
-    default: fpl_body<AL, FPL_PITCHES[FPL_PCLASS_DEFAULT]>(tk, gb, box, red); break;
+    case 0: fpl_body<BLK, SPLIT, PRE, FPL_PITCHES[0]>(tk, gb, sub, box, red); break;
+    case 1: fpl_body<BLK, SPLIT, PRE, FPL_PITCHES[1]>(tk, gb, sub, box, red); break;
+    case 2: fpl_body<BLK, SPLIT, PRE, FPL_PITCHES[2]>(tk, gb, sub, box, red); break;
+    case 4: fpl_body<BLK, SPLIT, PRE, FPL_PITCHES[4]>(tk, gb, sub, box, red); break;
+    case 5: fpl_body<BLK, SPLIT, PRE, FPL_PITCHES[5]>(tk, gb, sub, box, red); break;
+    case 6: fpl_body<BLK, SPLIT, PRE, FPL_PITCHES[6]>(tk, gb, sub, box, red); break;
+    case 7: fpl_body<BLK, SPLIT, PRE, FPL_PITCHES[7]>(tk, gb, sub, box, red); break;
+    default: fpl_body<BLK, SPLIT, PRE, FPL_PITCHES[FPL_PCLASS_DEFAULT]>(tk, gb, sub, box, red); break;
   }
 }
 
@@ -499,13 +625,25 @@ void launch_forward_lds(const FPLTask* d_tasks, int ntasks, int base, int blocks
                         const int* order, hipStream_t s) {
   if (blocks <= 0) return;
   if (al == FPV_CELL) { launch_forward_cell(d_tasks, ntasks, base, blocks, s); return; }
-  const dim3 g(xcd_grid(blocks)), t(FPL_THREADS);
-  if (al >= 4)
-    hipLaunchKernelGGL(fpl_kernel<4>, g, t, 0, s, d_tasks, ntasks, base, blocks, order);
-  else if (al == 2)
-    hipLaunchKernelGGL(fpl_kernel<2>, g, t, 0, s, d_tasks, ntasks, base, blocks, order);
-  else
-    hipLaunchKernelGGL(fpl_kernel<1>, g, t, 0, s, d_tasks, ntasks, base, blocks, order);
+  const dim3 t(FPL_THREADS);
+  // Launches of few workgroups: a block's angles over several of them, each
+  // staging the block's boxes (same boxes, chunks and sums, so the same bits).
+  // Staging a box more often costs a full GPU: us with al = 2, split and not,
+  // 16 and 24 at 65^2 x 48, 41 and 71 at 257^2 x 180 (115 blocks), 104 and
+  // 140 at 513^2 x 361 (414), 303 and 302 at 769^2 x 600 (975), 574 and 500
+  // at 1025^2 x 720 (1530); with al = 4 111 and 219 at 513^2 x 361 (207).
+  const int split = al >= 4 ? 4 : al;
+  if (blocks * split <= FPL_SPLIT_MAX) {
+    const dim3 g(xcd_grid(blocks * split));
+    if (al >= 4) hipLaunchKernelGGL((fpl_kernel<16, 4, true>), g, t, 0, s, d_tasks, ntasks, base, blocks, order);
+    else if (al == 2) hipLaunchKernelGGL((fpl_kernel<8, 2, true>), g, t, 0, s, d_tasks, ntasks, base, blocks, order);
+    else hipLaunchKernelGGL((fpl_kernel<4, 1, true>), g, t, 0, s, d_tasks, ntasks, base, blocks, order);
+    return;
+  }
+  const dim3 g(xcd_grid(blocks));
+  if (al >= 4) hipLaunchKernelGGL((fpl_kernel<16, 1, false>), g, t, 0, s, d_tasks, ntasks, base, blocks, order);
+  else if (al == 2) hipLaunchKernelGGL((fpl_kernel<8, 1, false>), g, t, 0, s, d_tasks, ntasks, base, blocks, order);
+  else hipLaunchKernelGGL((fpl_kernel<4, 1, false>), g, t, 0, s, d_tasks, ntasks, base, blocks, order);
 }
 
 namespace {
