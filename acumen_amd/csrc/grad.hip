@@ -12,6 +12,26 @@
 // 3 x 3 lattice points, and each is tested with the projector's own FP32
 // expressions (contraction off), so the weights are exactly the projector's
 // and the kernel is its transpose.
+//
+// The projector's weights (x1+1) - xr and xr - x1 are differences of floats
+// within a factor of two of each other (x1 >= 2), hence exact (Sterbenz), and
+// equal to 1 - |dx|, dx = xr - px, which is exact too; off the stencil 1 -
+// |dx| <= 0.  So a candidate's weight is the product of two differences
+// clamped to [0, 1] -- an output modifier, no comparison or select -- and
+// the rays of an angle (rows jy) each add (sum of their three candidates'
+// weights) x (their sinogram value).  That is 9 full-rate instructions per
+// candidate.  The bounds test only bites on the image's rim: pixel 1 is in no
+// valid cell, pixel 2 only in x1 = 2 (dx >= 0), pixel N only in x1 = N-1
+// (dx < 0); tiles that hold such pixels, and angles at which a tile's samples
+// reach jx < 1 or > N (or a window holds an infinity or NaN), take the same
+// loop with those tests.  The sinogram
+// values of a tile (a window of 32 rays per angle, zero off the detector) are
+// staged in LDS for 32 angles at a time.
+//
+// Bound by VALU issue (about 115 instructions per pixel and angle, 90 of them
+// the candidates).  On MI355X 6.7 ms per 16 x 513^2 x 720 launch (9.7 with
+// comparisons per candidate and three global loads per angle), 130 us at
+// 257^2 x 180 (344).
 #include "acu_grad.hpp"
 
 namespace acu {
@@ -47,103 +67,129 @@ __device__ double block_sum(double v, double* wsum) {
   return r;
 }
 
+constexpr int ADJ_W = 32;  // rays staged per angle and tile: 15 (|c| + |s|) + 4 <= 25.3, and one of margin on each side
+
+// One angle's contribution to one pixel.  (X, Y): the pixel relative to the
+// midpoint; w: LDS offset (lds_units) of the angle's ray jy = m in P.  CHECK: the rim's and the sweep's bounds (xlo, xhi, ylo, yhi: dx, dy
+// allowed in [lo, hi); u0, u1: jx - m allowed in [u0, u1]).
+struct AdjPixel {
+  float X, Y, px, py, xlo, xhi, ylo, yhi, u0, u1;
+};
+template <bool CHECK>
+__device__ __forceinline__ float adj_angle(const AdjPixel& g, float s, float c, float hw, float m, float w,
+                                           const float* P) {
+#pragma clang fp contract(off)
+  // first candidate, relative to the midpoint (integer valued): the margin in
+  // hw covers the rounding of this estimate and of the exact positions
+  const float ua = ceilf(fmaf(c, g.X, fmaf(s, g.Y, -hw)));
+  const float wa = ceilf(fmaf(c, g.Y, fmaf(-s, g.X, -hw)));
+  const float* r = (const float*)((const char*)P + __float_as_uint(fmaf(wa, lds_units(4), w)));
+  const float rv[3] = {r[0], r[1], r[2]};
+  float cu[3], su[3];
+  bool uok[3];
+#pragma unroll
+  for (int a = 0; a < 3; ++a) {
+    const float u = a == 0 ? ua : ua + (float)a;
+    cu[a] = c * u;
+    su[a] = s * u;
+    uok[a] = !CHECK || (u >= g.u0 && u <= g.u1);
+  }
+  float v = 0.0f;
+#pragma unroll
+  for (int b = 0; b < 3; ++b) {
+    const float wb = b == 0 ? wa : wa + (float)b;
+    const float sw = s * wb, cw = c * wb;
+    float sum = 0.0f;
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+      const float dx = ((cu[a] - sw) + m) - g.px;
+      const float dy = ((su[a] + cw) + m) - g.py;
+      float wx = __builtin_amdgcn_fmed3f(1.0f - fabsf(dx), 0.0f, 1.0f);
+      const float wy = __builtin_amdgcn_fmed3f(1.0f - fabsf(dy), 0.0f, 1.0f);
+      if (CHECK) wx = uok[a] && dx >= g.xlo && dx < g.xhi && dy >= g.ylo && dy < g.yhi ? wx : 0.0f;
+      sum = a == 0 ? wx * wy : fmaf(wx, wy, sum);
+    }
+    // CHECK: a ray of infinity or NaN stays out of the pixels it does not cover
+    if (!CHECK) v = b == 0 ? rv[b] * sum : fmaf(rv[b], sum, v);
+    else v = sum > 0.0f ? fmaf(rv[b], sum, v) : v;
+  }
+  return v;
+}
+
 __global__ __launch_bounds__(ADJ_T * ADJ_T) void adjoint_kernel(const AdjTask* __restrict__ tasks, int ntasks,
                                                                 int base, int nblocks) {
-#pragma clang fp contract(off)
+  __shared__ float P[ADJ_AB * ADJ_W];
   const int lbk = xcd_remap(blockIdx.x, gridDim.x);
-  if (lbk >= nblocks) return;
+  if (lbk >= nblocks) return;  // uniform per workgroup
   const int gb = base + lbk;
   const AdjTask& tk = tasks[find_by<AdjTask, &AdjTask::block_begin>(tasks, ntasks, gb)];
   const int N = tk.N, T = tk.T;
   const float m = tk.mid;
   const int local = gb - tk.block_begin;
   const int ty = local / tk.ntx, tx = local - ty * tk.ntx;
-  const int px = tx * ADJ_T + (int)(threadIdx.x % ADJ_T) + 1;  // 1-based pixel
-  const int py = ty * ADJ_T + (int)(threadIdx.x / ADJ_T) + 1;
-  if (px > N || py > N) return;  // no barrier below
-  const float X = (float)px - m, Y = (float)py - m;
+  const int tid = (int)threadIdx.x, lane = tid & 63;
+  const int px = tx * ADJ_T + tid % ADJ_T + 1;  // 1-based pixel; past the image in the last tiles (not stored)
+  const int py = ty * ADJ_T + tid / ADJ_T + 1;
+  AdjPixel g;
+  g.px = (float)px;
+  g.py = (float)py;
+  g.X = g.px - m;
+  g.Y = g.py - m;
+  g.xlo = px == 1 ? 4.0f : px == 2 ? 0.0f : -4.0f;
+  g.xhi = px >= N ? 0.0f : 4.0f;
+  g.ylo = py == 1 ? 4.0f : py == 2 ? 0.0f : -4.0f;
+  g.yhi = py >= N ? 0.0f : 4.0f;
+  g.u0 = 1.0f - m;
+  g.u1 = (float)N - m;
+  const bool rim = tx == 0 || ty == 0 || (tx + 1) * ADJ_T >= N || (ty + 1) * ADJ_T >= N;  // uniform
+  // tile corners relative to the midpoint
+  const float X0 = (float)(tx * ADJ_T + 1) - m, X1 = X0 + (float)(ADJ_T - 1);
+  const float Y0 = (float)(ty * ADJ_T + 1) - m, Y1 = Y0 + (float)(ADJ_T - 1);
+  const float margin = 1e-3f + 3e-7f * (float)N;
   const ACU_GLOBAL float* __restrict__ sino = as_global(tk.sino);
-  // Pixels with 3 <= px, py <= N-1: the cells x1 in {px-1, px} that can
-  // cover them always pass 2 <= x1 <= N-1, and the projector's weights
-  // (x1+1) - xr and xr - x1 are differences of floats within a factor of two
-  // of each other, hence exact (Sterbenz), and equal to 1 - |xr - px|, which
-  // is exact too (xr - px is, and 1 - d is a multiple of xr's ulp below 1).
-  // So the test and weights of those pixels reduce to the two weights being
-  // positive (a weight of 0 adds nothing) -- the same bits with no floor,
-  // conversion or select.  The rim keeps the projector's own test.
-  const bool inner = px >= 3 && px <= N - 1 && py >= 3 && py <= N - 1;
-  const float pxf = (float)px, pyf = (float)py;
+  const ACU_GLOBAL float* __restrict__ sc = as_global((const float*)tk.sc);
   float acc = 0.0f;
   for (int t0 = 0; t0 < T; t0 += ADJ_AB) {
-    const int t1 = min(T, t0 + ADJ_AB);
-    float blk = 0.0f;  // FP32 sum over one block of angles, then into acc
-    for (int t = t0; t < t1; ++t) {
-      const float2 v = const_f2(tk.sc, t);
-      const float s = v.x, c = v.y;
-      // inverse rotation of the pixel centre, lattice coordinates; the margin
-      // covers the rounding of both this estimate and the exact positions
-      const float qx = (c * X + s * Y) + m;
-      const float qy = (c * Y - s * X) + m;
-      const float hw = fabsf(c) + fabsf(s) + 1e-3f;
-      const int jx0 = (int)ceilf(qx - hw), jy0 = (int)ceilf(qy - hw);
-      const ACU_GLOBAL float* row = sino + (size_t)t * N;
-      if (inner) {
-        float sw[3], cw[3], rv[3];
-        bool yok[3];
+    const int na = min(ADJ_AB, T - t0);
+    // lane l (mod 32) of every wave holds angle t0 + l: sine, cosine, first
+    // ray of the tile's window, and whether a sample can leave 1 <= jx <= N
+    const int t = min(t0 + (lane & (ADJ_AB - 1)), T - 1);
+    const float hs = sc[2 * t], hc = sc[2 * t + 1];
+    const float hh = fabsf(hc) + fabsf(hs) + margin;
+    const float ymin = fminf(hc * Y0, hc * Y1) + fminf(-hs * X0, -hs * X1);
+    const float xmin = fminf(hc * X0, hc * X1) + fminf(hs * Y0, hs * Y1);
+    const float xmax = fmaxf(hc * X0, hc * X1) + fmaxf(hs * Y0, hs * Y1);
+    const int lo = (int)floorf((ymin - hh) + m) - 1;
+    const float hb = lds_base(4 * ((lane & (ADJ_AB - 1)) * ADJ_W + (int)m - lo));  // LDS offset of ray jy = m
+    unsigned long long chk = rim ? ~0ull : __ballot(xmin - hh < g.u0 + 1.0f || xmax + hh > g.u1 - 1.0f);
+    bool bad = false;
+    {
+      const int q = tid >> 3, j = tid & 7;  // 8 threads per angle
+      const int jy0 = __shfl(lo, q) + j;
+      const ACU_GLOBAL float* row = sino + (size_t)min(t0 + q, T - 1) * N;
+      float v[ADJ_W / 8];
 #pragma unroll
-        for (int bb = 0; bb < 3; ++bb) {
-          const int jy = jy0 + bb;
-          const float w = (float)jy - m;
-          sw[bb] = s * w;
-          cw[bb] = c * w;
-          yok[bb] = jy >= 1 && jy <= N;
-          rv[bb] = yok[bb] ? row[jy - 1] : 0.0f;
-        }
+      for (int k = 0; k < ADJ_W / 8; ++k) v[k] = row[min(max(jy0 + 8 * k, 1), N) - 1];
+      if (t0 > 0) __syncthreads();  // the last block's rays are read
 #pragma unroll
-        for (int a = 0; a < 3; ++a) {
-          const int jx = jx0 + a;
-          const float u = (float)jx - m;
-          const float cu = c * u, su = s * u;
-          const bool xok = jx >= 1 && jx <= N;
-#pragma unroll
-          for (int bb = 0; bb < 3; ++bb) {
-            const float xr = (cu - sw[bb]) + m;
-            const float yr = (su + cw[bb]) + m;
-            const float wx = 1.0f - fabsf(xr - pxf);
-            const float wy = 1.0f - fabsf(yr - pyf);
-            if (xok && yok[bb] && wx > 0.0f && wy > 0.0f) blk += (rv[bb] * wx) * wy;
-          }
-        }
-      } else {
-#pragma unroll
-        for (int a = 0; a < 3; ++a) {
-          const int jx = jx0 + a;
-          const float u = (float)jx - m;
-          const float cu = c * u, su = s * u;
-#pragma unroll
-          for (int bb = 0; bb < 3; ++bb) {
-            const int jy = jy0 + bb;
-            const float w = (float)jy - m;
-            const float xr = (cu - s * w) + m;
-            const float yr = (su + c * w) + m;
-            const float fx = floorf(xr), fy = floorf(yr);
-            const int x1 = (int)fx, y1 = (int)fy;
-            const int dx = px - x1, dy = py - y1;
-            const bool hit = jx >= 1 && jx <= N && jy >= 1 && jy <= N && (unsigned)dx <= 1u &&
-                             (unsigned)dy <= 1u && x1 >= 2 && x1 <= N - 1 && y1 >= 2 && y1 <= N - 1;
-            if (hit) {
-              // the projector's weights: (x2 - xr) for x1, (xr - x1) for x2
-              const float wx = dx == 0 ? (fx + 1.0f) - xr : xr - fx;
-              const float wy = dy == 0 ? (fy + 1.0f) - yr : yr - fy;
-              blk += (row[jy - 1] * wx) * wy;
-            }
-          }
-        }
+      for (int k = 0; k < ADJ_W / 8; ++k) {
+        P[q * ADJ_W + j + 8 * k] = jy0 + 8 * k >= 1 && jy0 + 8 * k <= N ? v[k] : 0.0f;
+        bad = bad || !(fabsf(v[k]) <= 3.40282347e38f);
       }
+    }
+    if (__syncthreads_or(bad)) chk = ~0ull;  // uniform
+    float blk = 0.0f;  // FP32 sum over one block of angles, then into acc
+    for (int a = 0; a < na; ++a) {
+      const float s = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(hs), a));
+      const float c = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(hc), a));
+      const float hw = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(hh), a));
+      const float w = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(hb), a));
+      if ((chk >> a) & 1) blk += adj_angle<true>(g, s, c, hw, m, w, P);
+      else blk += adj_angle<false>(g, s, c, hw, m, w, P);
     }
     acc += blk;
   }
-  tk.out[(size_t)(py - 1) * N + (px - 1)] = acc / (float)N;
+  if (px <= N && py <= N) tk.out[(size_t)(py - 1) * N + (px - 1)] = acc / (float)N;
 }
 
 __device__ __forceinline__ float at(const ACU_GLOBAL float* row, int N, int i) {
