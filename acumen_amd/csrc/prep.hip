@@ -16,8 +16,6 @@
 namespace acu {
 namespace {
 
-constexpr int MT = 16;  // median tile side (16 x 16 threads)
-
 __device__ __forceinline__ int clampi(int v, int lo, int hi) { return v < lo ? lo : v > hi ? hi : v; }
 __device__ __forceinline__ float clampf(float v, float lo, float hi) { return fminf(fmaxf(v, lo), hi); }
 
@@ -33,6 +31,25 @@ __device__ __forceinline__ float median27(float (&v)[27]) {
   return v[MEDIAN27_NET.out];
 }
 
+// the instructions themselves: fminf and fmaxf would quiet each operand first
+struct Float3Ops {
+  static __device__ __forceinline__ float min3(float a, float b, float c) {
+    float r;
+    asm("v_min3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+    return r;
+  }
+  static __device__ __forceinline__ float med3(float a, float b, float c) {
+    float r;
+    asm("v_med3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+    return r;
+  }
+  static __device__ __forceinline__ float max3(float a, float b, float c) {
+    float r;
+    asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+    return r;
+  }
+};
+
 // 3x3x3 median (:420-447): projections l, c, r; neighbours clamped into the
 // image; the 14th of 27 in descending order = the 14th in ascending order.
 // This is the median the reference's loop nest describes: its register
@@ -42,51 +59,97 @@ __device__ __forceinline__ float median27(float (&v)[27]) {
 // Values that compare equal but differ in bits (+0 and -0) or NaN are the
 // exception: the reference's exchange sort is not stable, so which of them
 // it leaves in the middle depends on its order of exchanges.
-__global__ __launch_bounds__(MT * MT) void median27_kernel(int n, const float* __restrict__ l,
-                                                           const float* __restrict__ c,
-                                                           const float* __restrict__ r, float* __restrict__ out,
-                                                           int tiles_x) {
-  constexpr int H = MT + 2, HH = H * H, NS = (3 * HH + MT * MT - 1) / (MT * MT);
-  __shared__ float t[3 * HH];  // [p][yy][xx]
+//
+// A wave takes 62 x K pixels: a lane loads its column of the K + 2 rows of
+// the three projections (all loads in flight, no LDS), gets its neighbours'
+// values by DPP and, walking down, sorts the nine values of the next row once
+// and selects the median of the last three sorted rows: 46 instructions a
+// pixel (and 27 for each of the rows above and below its K) instead of the
+// 306 of the network for 27 loose values.  That network stays for waves whose
+// values hold a NaN, where the result depends on the order of comparisons.
+// Bound by its traffic (three images in, one out: 67 MB, 3.5 TB/s) beside
+// about 80 instructions a pixel. us per 2048^2 image: 19, 21 with the rows
+// staged in LDS, 57 with the network in every pixel.
+constexpr int MED_X = 62;
+
+__device__ __forceinline__ float lane_prev(float v) {  // wave_shr:1: lane i reads lane i - 1
+  return __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(v), __float_as_int(v), 0x138, 0xF, 0xF, false));
+}
+__device__ __forceinline__ float lane_next(float v) {  // wave_shl:1: lane i reads lane i + 1
+  return __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(v), __float_as_int(v), 0x130, 0xF, 0xF, false));
+}
+
+template <int K>
+__global__ __launch_bounds__(256) void median27_kernel(int n, const float* __restrict__ l,
+                                                       const float* __restrict__ c, const float* __restrict__ r,
+                                                       float* __restrict__ out, int tiles_x) {
   const int bx = blockIdx.x % tiles_x, by = blockIdx.x / tiles_x;
-  const int x0 = bx * MT, y0 = by * MT;  // 0-based tile origin
-  // halo tiles of the three projections: every load issued before the first
-  // LDS store (element i = p*HH + yy*H + xx; the divisions are by constants)
-  float st[NS];
+  const int lane = threadIdx.x & 63;
+  const int y = __builtin_amdgcn_readfirstlane((by * 4 + (int)(threadIdx.x >> 6)) * K);  // 0-based first row
+  const int x = bx * MED_X + lane - 1;
+  if (y >= n) return;  // the whole wave
+  const unsigned gx = (unsigned)clampi(x, 0, n - 1);
+  const bool own = lane >= 1 && lane <= MED_X && x < n;
+  float raw[K + 2][3];
 #pragma unroll
-  for (int k = 0; k < NS; ++k) {
-    const int i = (int)threadIdx.x + k * MT * MT;
-    const int ic = i < 3 * HH ? i : 0;
-    const int p = ic / HH, q = ic - p * HH;
-    const int yy = q / H, xx = q - yy * H;
-    const int gx = clampi(x0 + xx - 1, 0, n - 1), gy = clampi(y0 + yy - 1, 0, n - 1);
-    const float* sp = p == 0 ? l : p == 1 ? c : r;  // no private-memory pointer table
-    st[k] = sp[(size_t)gy * n + gx];
+  for (int k = 0; k < K + 2; ++k) {
+    const size_t o = (size_t)clampi(y + k - 1, 0, n - 1) * n;
+    raw[k][0] = (l + o)[gx];
+    raw[k][1] = (c + o)[gx];
+    raw[k][2] = (r + o)[gx];
   }
+  bool nan = false;
 #pragma unroll
-  for (int k = 0; k < NS; ++k) {
-    const int i = (int)threadIdx.x + k * MT * MT;
-    if (i < 3 * HH) t[i] = st[k];
+  for (int k = 0; k < K + 2; ++k)
+#pragma unroll
+    for (int p = 0; p < 3; ++p) nan = nan || raw[k][p] != raw[k][p];
+  if (__ballot(nan)) {
+    if (!own) return;
+    for (int k = 0; k < K && y + k < n; ++k) {
+      float v[27];
+#pragma unroll
+      for (int p = 0; p < 3; ++p) {
+        const float* img = p == 0 ? l : p == 1 ? c : r;
+#pragma unroll
+        for (int dy = 0; dy < 3; ++dy)
+#pragma unroll
+          for (int dx = 0; dx < 3; ++dx)
+            v[p * 9 + dy * 3 + dx] =
+                img[(size_t)clampi(y + k + dy - 1, 0, n - 1) * n + clampi(x + dx - 1, 0, n - 1)];
+      }
+      out[(size_t)(y + k) * n + x] = median27(v);
+    }
+    return;
   }
-  __syncthreads();
-  const int tx = threadIdx.x % MT, ty = threadIdx.x / MT;
-  const int x = x0 + tx, y = y0 + ty;
-  if (x >= n || y >= n) return;  // after the only barrier
-  float v[27];
+  auto row = [&](int k, float (&v)[9]) {
 #pragma unroll
-  for (int p = 0; p < 3; ++p)
+    for (int p = 0; p < 3; ++p) {
+      v[3 * p] = lane_prev(raw[k][p]);
+      v[3 * p + 1] = raw[k][p];
+      v[3 * p + 2] = lane_next(raw[k][p]);
+    }
+    sort9<Float3Ops>(v);
+  };
+  float v[3][9];
+  row(0, v[0]);
+  row(1, v[1]);
 #pragma unroll
-    for (int dy = 0; dy < 3; ++dy)
-#pragma unroll
-      for (int dx = 0; dx < 3; ++dx) v[p * 9 + dy * 3 + dx] = t[p * HH + (ty + dy) * H + tx + dx];
-  out[(size_t)y * n + x] = median27(v);
+  for (int k = 0; k < K; ++k) {
+    row(k + 2, v[(k + 2) % 3]);
+    const float med = median27_of_sorted<Float3Ops>(v[0], v[1], v[2]);
+    if (own && y + k < n) out[(size_t)(y + k) * n + x] = med;
+  }
 }
 
 // The resampling of :449-464 at output (jx, jy), 1-based, in the
 // reference's FP32 order: u = (jx - mx) - S*shift, xr = clamp((c*u - s*(jy-my)) + mx),
 // yr = clamp((s*u + c*(jy-my)) + my), taps clamped into the image; a tap
 // pair clamped onto one pixel has both weights zero.
-__device__ __forceinline__ float prep_sample(const PrepGeom& g, const float* __restrict__ img, int jx, int jy) {
+struct PrepTaps {
+  size_t o11, o12, o21, o22;  // pixels (x1, y1), (x2, y1), (x1, y2), (x2, y2)
+  float ax, bx, ay, by;
+};
+__device__ __forceinline__ PrepTaps prep_taps(const PrepGeom& g, int jx, int jy) {
 #pragma clang fp contract(off)
   const int n = g.n;
   const float u = ((float)jx - g.mx) - g.S * g.shift;
@@ -95,28 +158,55 @@ __device__ __forceinline__ float prep_sample(const PrepGeom& g, const float* __r
   const float yr = clampf((g.s * u + g.c * w) + g.my, 1.0f, (float)n);
   const int y1 = clampi((int)floorf(yr), 1, n), y2 = clampi(y1 + 1, 1, n);
   const int x1 = clampi((int)floorf(xr), 1, n), x2 = clampi(x1 + 1, 1, n);
-  const float ax = (float)x2 - xr, bx = xr - (float)x1, ay = (float)y2 - yr, by = yr - (float)y1;
-  const float* r1 = img + (size_t)(y1 - 1) * n;
-  const float* r2 = img + (size_t)(y2 - 1) * n;
-  float v = (r1[x1 - 1] * ax) * ay;
-  v = v + (r1[x2 - 1] * bx) * ay;
-  v = v + (r2[x1 - 1] * ax) * by;
-  v = v + (r2[x2 - 1] * bx) * by;
+  PrepTaps q;
+  q.ax = (float)x2 - xr;
+  q.bx = xr - (float)x1;
+  q.ay = (float)y2 - yr;
+  q.by = yr - (float)y1;
+  const size_t r1 = (size_t)(y1 - 1) * n, r2 = (size_t)(y2 - 1) * n;
+  q.o11 = r1 + (x1 - 1);
+  q.o12 = r1 + (x2 - 1);
+  q.o21 = r2 + (x1 - 1);
+  q.o22 = r2 + (x2 - 1);
+  return q;
+}
+__device__ __forceinline__ float prep_lerp(const PrepTaps& q, const float* __restrict__ img) {
+#pragma clang fp contract(off)
+  float v = (img[q.o11] * q.ax) * q.ay;
+  v = v + (img[q.o12] * q.bx) * q.ay;
+  v = v + (img[q.o21] * q.ax) * q.by;
+  v = v + (img[q.o22] * q.bx) * q.by;
   return v;
+}
+__device__ __forceinline__ float prep_sample(const PrepGeom& g, const float* __restrict__ img, int jx, int jy) {
+  return prep_lerp(prep_taps(g, jx, jy), img);
 }
 
 // Corrected projections of a batch -> sinogram rows: projection k of the
 // batch (global index job0 + k) fills row job0 + k of every slice's
 // sinogram; sino is nslices(= n) x nfiles x Nw, slice-major.  Grid: x over
-// the Nw output columns, y = the detector row jy - 1 - row0, z = the projection.
-__global__ __launch_bounds__(256) void correct_kernel(PrepGeom g, const float* __restrict__ imgs, int job0,
+// the Nw output columns, y = the detector row jy - 1 - row0, z = groups of
+// COR_K projections: the positions and weights are the same for every
+// projection, so a thread forms them once for its group and has the group's
+// gathers in flight together.  Bound by its traffic: 8 projections of 2048^2
+// (268 MB) take 74 us (3.6 TB/s), 110 with one projection a thread.
+constexpr int COR_K = 4;
+__global__ __launch_bounds__(256) void correct_kernel(PrepGeom g, const float* __restrict__ imgs, int count, int job0,
                                                       int nfiles, int row0, float* __restrict__ sino) {
   const int nw = g.n + g.add_nx;
   const int jx = (int)(blockIdx.x * blockDim.x + threadIdx.x) + 1;
   if (jx > nw) return;
-  const int jy = row0 + (int)blockIdx.y + 1, k = (int)blockIdx.z;
-  const float v = prep_sample(g, imgs + (size_t)k * g.n * g.n, jx, jy);
-  sino[((size_t)(jy - 1) * nfiles + (size_t)(job0 + k)) * nw + (jx - 1)] = v;
+  const int jy = row0 + (int)blockIdx.y + 1, k0 = (int)blockIdx.z * COR_K;
+  const PrepTaps q = prep_taps(g, jx, jy);
+  const size_t nn = (size_t)g.n * g.n;
+  const float* img = imgs + (size_t)k0 * nn;
+  float* o = sino + ((size_t)(jy - 1) * nfiles + (size_t)(job0 + k0)) * nw + (jx - 1);
+  float v[COR_K];
+#pragma unroll
+  for (int k = 0; k < COR_K; ++k) v[k] = prep_lerp(q, img + (size_t)min(k, count - 1 - k0) * nn);
+#pragma unroll
+  for (int k = 0; k < COR_K; ++k)
+    if (k0 + k < count) o[(size_t)k * nw] = v[k];
 }
 
 // |V0(jx,jy) - V180(Nw-jx+1,jy)| summed per block in FP64 (:278-283).
@@ -151,9 +241,18 @@ __global__ __launch_bounds__(256) void sum_kernel(const double* __restrict__ par
 
 }  // namespace
 
+constexpr int MED_MIN = 512;  // workgroups of strips of 8 rows: two per CU
+
 void launch_median27(int n, const float* l, const float* c, const float* r, float* out, hipStream_t s) {
-  const int tx = (n + MT - 1) / MT;
-  hipLaunchKernelGGL(median27_kernel, dim3(tx * tx), dim3(MT * MT), 0, s, n, l, c, r, out, tx);
+  const int tx = (n + MED_X - 1) / MED_X;
+  auto rows = [&](int k) { return (n + 4 * k - 1) / (4 * k); };
+  // strips of 8 rows sort 10 rows for 8 pixels, of 2 rows 4 for 2, but keep
+  // the GPU busier on small images: us per image with 8 and with 2 rows, 6.5
+  // and 6.8 at 1024^2, 4.2 and 4.3 at 700^2, 4.1 and 4.0 at 512^2
+  if (tx * rows(8) >= MED_MIN)
+    hipLaunchKernelGGL(median27_kernel<8>, dim3(tx * rows(8)), dim3(256), 0, s, n, l, c, r, out, tx);
+  else
+    hipLaunchKernelGGL(median27_kernel<2>, dim3(tx * rows(2)), dim3(256), 0, s, n, l, c, r, out, tx);
 }
 
 void launch_correct(const PrepGeom& g, const float* imgs, int count, int job0, int nfiles, float* sino,
@@ -162,8 +261,8 @@ void launch_correct(const PrepGeom& g, const float* imgs, int count, int job0, i
   for (int k0 = 0; k0 < count; k0 += 65535)  // the grid's y and z extents are at most 65535
     for (int r0 = 0; r0 < g.n; r0 += 65535) {
       const int cnt = std::min(65535, count - k0), rows = std::min(65535, g.n - r0);
-      hipLaunchKernelGGL(correct_kernel, dim3(gx, (unsigned)rows, (unsigned)cnt), dim3(256), 0, s, g,
-                         imgs + (size_t)k0 * g.n * g.n, job0 + k0, nfiles, r0, sino);
+      hipLaunchKernelGGL(correct_kernel, dim3(gx, (unsigned)rows, (unsigned)((cnt + COR_K - 1) / COR_K)), dim3(256),
+                         0, s, g, imgs + (size_t)k0 * g.n * g.n, cnt, job0 + k0, nfiles, r0, sino);
     }
 }
 
