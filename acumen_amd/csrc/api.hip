@@ -374,7 +374,7 @@ void layout_tv(acu_batch* b, Carver& cv, int delta_cap) {
     s.iukt64 = cv.take<double>(NN);
     s.ruk64 = cv.take<double>(NT);
     s.scal = cv.take<double>(SCAL_STRIDE);
-    s.partials = cv.take<double>((size_t)s.ew_n);
+    s.partials = cv.take<double>(3 * (size_t)s.ew_n);
     s.delta = cv.take<float>((size_t)delta_cap);
     s.delta_cap = delta_cap;
   }
@@ -820,6 +820,8 @@ void outer_body(acu_batch* b, int sl, int ninner, int ncg, bool ruk_fresh, bool 
   const int nt = b->tv.n;
   const int first = sl < 0 ? 0 : sl, count = sl < 0 ? nt : 1;  // finalize: one block per slice
   const bool lin = b->tv_sched == ACU_TV_SCHED_LINEAR;
+  bool inl = !host_sync;
+  for (int i = first; i < first + count; ++i) inl = inl && b->s[i].ew_n <= TV_INLINE_BLOCKS;
   for (int ji = 0; ji < ninner; ++ji) {
     const bool exact = !lin || (refresh && ji == 0);
     const bool tp = b->tv_bp_refpos;
@@ -829,31 +831,30 @@ void outer_body(acu_batch* b, int sl, int ninner, int ncg, bool ruk_fresh, bool 
     if (exact) iradon_seq(b, b->rf_ruk, b->bp_iukt, sl, tp);       // :229
     if (lin && exact) launch_tv_linload(tv, nt, ew.base, ew.n, sw.base, sw.n, c->stream);
     launch_tv_residual(tv, nt, ew.base, ew.n, lin, c->stream);     // :207-249
-    launch_tv_finalize(tv, first, count, 0, c->stream);
+    if (!inl) launch_tv_finalize(tv, first, count, 0, c->stream);
     check_launch();
     if (host_sync) (void)read_scalar(b, sl, 0);
     for (int j = 0; j < ncg; ++j) {                                // :252-303
       radon_seq(b, b->fp_p, sl);
       iradon_seq(b, b->rf_rp, b->bp_irpt, sl, tp);
       launch_tv_apdot(tv, nt, ew.base, ew.n, j, c->stream);
-      launch_tv_finalize(tv, first, count, 64 + j, c->stream);
+      if (!inl) launch_tv_finalize(tv, first, count, 64 + j, c->stream);
       check_launch();
       if (host_sync) (void)read_scalar(b, sl, 64 + j);
-      launch_tv_axpy(tv, nt, ew.base, ew.n, j, lin, c->stream);
-      if (lin) launch_tv_sino_axpy(tv, nt, sw.base, sw.n, j, c->stream);
-      launch_tv_finalize(tv, first, count, j + 1, c->stream);
+      launch_tv_axpy(tv, nt, ew.base, ew.n, sw.base, sw.n, j, lin, inl, c->stream);
+      if (!inl) launch_tv_finalize(tv, first, count, j + 1, c->stream);
       check_launch();
       if (host_sync) (void)read_scalar(b, sl, j + 1);
-      launch_tv_pupdate(tv, nt, ew.base, ew.n, j, c->stream);
+      launch_tv_pupdate(tv, nt, ew.base, ew.n, j, inl, c->stream);
       check_launch();
     }
     launch_tv_shrink(tv, nt, ew.base, ew.n, lin && ji == ninner - 1, c->stream);  // :305-333
-    launch_tv_finalize(tv, first, count, 127, c->stream);
+    if (host_sync) launch_tv_finalize(tv, first, count, 127, c->stream);  // else summed by the add-back
     check_launch();
     if (host_sync) (void)read_scalar(b, sl, 127);
   }
   if (!lin) radon_seq(b, b->fp_uk, sl);                            // :339
-  launch_tv_addback(tv, nt, sw.base, sw.n, lin, c->stream);        // :341-346
+  launch_tv_addback(tv, nt, sw.base, sw.n, lin, !host_sync && ninner > 0, c->stream);  // :341-346
   check_launch();
 }
 

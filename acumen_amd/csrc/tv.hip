@@ -11,8 +11,11 @@
 // HIP graph.  All kernels are batched: blocks are flattened over slices.
 //
 // Scalar slots per slice (doubles): rs[j] at j (j = 0..ncg), pAp[j] at
-// 64+j, outer-iteration counter at 126, Err_diff at 127.  Every reduction
-// kernel writes block partials and is followed by finalize_kernel.
+// 64+j, outer-iteration counter at 126, Err_diff at 127.  A reduction kernel
+// writes block partials; for slices of up to TV_INLINE_BLOCKS blocks the
+// kernel that needs the sum adds them in each of its workgroups, otherwise
+// finalize_kernel (one workgroup per slice) does, in the same order, so both
+// give the same bits.
 #include "acu_tv.hpp"
 
 namespace acu {
@@ -45,8 +48,8 @@ __device__ __forceinline__ double wave_sum(double v) {
   return v;
 }
 
-// Block-reduce v and write this block's partial; finalize_kernel (launched
-// next on the same stream) sums a slice's partials in index order.  No
+// Block-reduce v and write this block's partial; a later kernel of the same
+// stream sums a slice's partials in index order.  No
 // device-scope fence per block: on a multi-XCD part each such fence writes
 // back the L2, which made these kernels ~10x slower than their traffic.
 __device__ void reduce_to_partial(double v, double* partials, int lblock) {
@@ -62,6 +65,32 @@ __device__ void reduce_to_partial(double v, double* partials, int lblock) {
     partials[lblock] = b;
   }
 }
+
+// Sum of a slice's block partials in a fixed order (thread t sums a contiguous
+// range, then a tree), known to every thread of the workgroup.
+__device__ double partials_total(const double* __restrict__ partials, int nb) {
+  __shared__ double wsum[NT_ / 64];
+  const int chunk = (nb + NT_ - 1) / NT_;
+  const int b0 = threadIdx.x * chunk;
+  double s = 0.0;
+  for (int b = b0; b < min(nb, b0 + chunk); ++b) s += partials[b];
+  s = wave_sum(s);
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  if (lane == 0) wsum[wave] = s;
+  __syncthreads();
+  double tot = 0.0;
+#pragma unroll
+  for (int w = 0; w < NT_ / 64; ++w) tot += wsum[w];
+  __syncthreads();
+  return tot;
+}
+
+// A slice's partials: rs of the CG's axpy and Err_diff, p.Ap, rs[0].  Each
+// consumer kernel may sum them itself (INL) before another producer writes
+// the same set.
+__device__ __forceinline__ double* part_rs(const TVTask& tk) { return tk.partials; }
+__device__ __forceinline__ double* part_pap(const TVTask& tk) { return tk.partials + tk.nb; }
+__device__ __forceinline__ double* part_rs0(const TVTask& tk) { return tk.partials + 2 * (size_t)tk.nb; }
 
 __device__ __forceinline__ float lap(const float* __restrict__ u, int x, int y, int N) {
   const int xl = x == 0 ? N - 1 : x - 1, xr = x == N - 1 ? 0 : x + 1;
@@ -109,7 +138,7 @@ __global__ __launch_bounds__(NT_) void residual_kernel(const TVTask* __restrict_
       acc += (double)rv * (double)rv;
     }
   }
-  reduce_to_partial(acc, tk.partials, lb);
+  reduce_to_partial(acc, part_rs0(tk), lb);
 }
 
 // K12 + K13 (tv_hpc.F90:257-274): Ap = mu*irpt + lambda*L(p); pAp[j] = p.Ap
@@ -130,7 +159,7 @@ __global__ __launch_bounds__(NT_) void apdot_kernel(const TVTask* __restrict__ t
       acc += (double)tk.p[e] * (double)a;
     }
   }
-  reduce_to_partial(acc, tk.partials, lb);
+  reduce_to_partial(acc, part_pap(tk), lb);
 }
 
 // K14 + K15 (tv_hpc.F90:277-292): alpha = rs[j]/pAp[j] (FP64);
@@ -140,18 +169,51 @@ __global__ __launch_bounds__(NT_) void apdot_kernel(const TVTask* __restrict__ t
 // LIN (linear schedule): iukt = F(R(uk)) is carried along by linearity in
 // FP64, iukt64 += alpha irpt with irpt = F(R(p)), instead of being
 // recomputed from uk by a projection and a backprojection.
-__device__ __forceinline__ float cg_alpha(const double* scal, int j) {
-  const double num = scal[64 + j];
-  return num != 0.0 ? (float)(scal[j] / num) : 0.0f;
+// INL (slices of few blocks): every workgroup sums the partials of p.Ap (and,
+// in the first step, of rs[0]) itself instead of a finalize launch before it.
+template <bool INL>
+__device__ __forceinline__ float cg_alpha(const TVTask& tk, int j, bool store) {
+  double num = tk.scal[64 + j], rs = tk.scal[j];
+  if (INL) {
+    num = partials_total(part_pap(tk), tk.nb);
+    if (j == 0) rs = partials_total(part_rs0(tk), tk.nb);
+    if (store && threadIdx.x == 0) {
+      tk.scal[64 + j] = num;
+      if (j == 0) tk.scal[0] = rs;
+    }
+  }
+  return num != 0.0 ? (float)(rs / num) : 0.0f;
 }
 
-template <bool LIN>
-__global__ __launch_bounds__(NT_) void axpy_kernel(const TVTask* __restrict__ tasks, int ntasks, int base, int j) {
+// Linear schedule, sinogram part of K14 (the blocks after the image's):
+// ruk = R(uk) is carried along by linearity in FP64, ruk64 += alpha rp with
+// rp = R(p), so the add-back of tv_hpc.F90:339-346 needs no projection of the
+// new uk.
+template <bool INL>
+__device__ __forceinline__ void sino_axpy(const TVTask* __restrict__ tasks, int ntasks, int gb, int j) {
+  const TVTask& tk = tasks[find_task_s(tasks, ntasks, gb)];
+  const int lb = gb - tk.sb_begin;
+  const size_t NT = (size_t)tk.N * tk.T;
+  const float alpha = cg_alpha<INL>(tk, j, false);
+#pragma unroll
+  for (int it = 0; it < IT; ++it) {
+    const size_t e = (size_t)lb * PER_BLOCK + it * NT_ + threadIdx.x;
+    if (e < NT) tk.ruk64[e] += (double)alpha * (double)tk.rp[e];
+  }
+}
+
+template <bool LIN, bool INL>
+__global__ __launch_bounds__(NT_) void axpy_kernel(const TVTask* __restrict__ tasks, int ntasks, int base, int blocks,
+                                                   int sbase, int j) {
+  if (LIN && (int)blockIdx.x >= blocks) {
+    sino_axpy<INL>(tasks, ntasks, sbase + (int)blockIdx.x - blocks, j);
+    return;
+  }
   const TVTask& tk = tasks[find_task_e(tasks, ntasks, base + blockIdx.x)];
   const int N = tk.N;
   const int lb = base + blockIdx.x - tk.eb_begin;
   const size_t NN = (size_t)N * N;
-  const float alpha = cg_alpha(tk.scal, j);
+  const float alpha = cg_alpha<INL>(tk, j, lb == 0);
   double acc = 0.0;
 #pragma unroll
   for (int it = 0; it < IT; ++it) {
@@ -164,33 +226,23 @@ __global__ __launch_bounds__(NT_) void axpy_kernel(const TVTask* __restrict__ ta
       acc += (double)rv * (double)rv;
     }
   }
-  reduce_to_partial(acc, tk.partials, lb);
-}
-
-// Linear schedule, sinogram part of K14: ruk = R(uk) is carried along by
-// linearity in FP64, ruk64 += alpha rp with rp = R(p), so the add-back of
-// tv_hpc.F90:339-346 needs no projection of the new uk.
-__global__ __launch_bounds__(NT_) void sino_axpy_kernel(const TVTask* __restrict__ tasks, int ntasks, int base,
-                                                        int j) {
-  const TVTask& tk = tasks[find_task_s(tasks, ntasks, base + blockIdx.x)];
-  const int lb = base + blockIdx.x - tk.sb_begin;
-  const size_t NT = (size_t)tk.N * tk.T;
-  const float alpha = cg_alpha(tk.scal, j);
-#pragma unroll
-  for (int it = 0; it < IT; ++it) {
-    const size_t e = (size_t)lb * PER_BLOCK + it * NT_ + threadIdx.x;
-    if (e < NT) tk.ruk64[e] += (double)alpha * (double)tk.rp[e];
-  }
+  reduce_to_partial(acc, part_rs(tk), lb);
 }
 
 // K16 (tv_hpc.F90:294-299): p = r + (rs[j+1]/rs[j]) p
+template <bool INL>
 __global__ __launch_bounds__(NT_) void pupdate_kernel(const TVTask* __restrict__ tasks, int ntasks, int base, int j) {
   const TVTask& tk = tasks[find_task_e(tasks, ntasks, base + blockIdx.x)];
   const int N = tk.N;
   const int lb = base + blockIdx.x - tk.eb_begin;
   const size_t NN = (size_t)N * N;
   const double rs = tk.scal[j];
-  const float beta = rs != 0.0 ? (float)(tk.scal[j + 1] / rs) : 0.0f;
+  double rn = tk.scal[j + 1];
+  if (INL) {
+    rn = partials_total(part_rs(tk), tk.nb);
+    if (lb == 0 && threadIdx.x == 0) tk.scal[j + 1] = rn;
+  }
+  const float beta = rs != 0.0 ? (float)(rn / rs) : 0.0f;
 #pragma unroll
   for (int it = 0; it < IT; ++it) {
     const size_t e = (size_t)lb * PER_BLOCK + it * NT_ + threadIdx.x;
@@ -198,27 +250,13 @@ __global__ __launch_bounds__(NT_) void pupdate_kernel(const TVTask* __restrict__
   }
 }
 
-// One workgroup per slice: scal[slot] = sum of the slice's block partials,
-// in a fixed order (thread t sums a contiguous range, then a tree).
+// One workgroup per slice: scal[slot] = sum of the slice's partials of that slot.
 __global__ __launch_bounds__(NT_) void finalize_kernel(const TVTask* __restrict__ tasks, int first,
                                                        int slot) {
   const TVTask& tk = tasks[first + blockIdx.x];
-  __shared__ double wsum[NT_ / 64];
-  const int nb = tk.nb;
-  const int chunk = (nb + NT_ - 1) / NT_;
-  const int b0 = threadIdx.x * chunk;
-  double s = 0.0;
-  for (int b = b0; b < min(nb, b0 + chunk); ++b) s += tk.partials[b];
-  s = wave_sum(s);
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  if (lane == 0) wsum[wave] = s;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    double tot = 0.0;
-#pragma unroll
-    for (int w = 0; w < NT_ / 64; ++w) tot += wsum[w];
-    tk.scal[slot] = tot;
-  }
+  const double* part = slot == 0 ? part_rs0(tk) : slot >= 64 && slot < 127 ? part_pap(tk) : part_rs(tk);
+  const double tot = partials_total(part, tk.nb);
+  if (threadIdx.x == 0) tk.scal[slot] = tot;
 }
 
 __device__ __forceinline__ void shrink(float t, float inv_lambda, float& d, float& b) {
@@ -264,13 +302,15 @@ __global__ __launch_bounds__(NT_) void shrink_kernel(const TVTask* __restrict__ 
       acc += (double)fabsf(u - tk.ukp[e]);
     }
   }
-  reduce_to_partial(acc, tk.partials, lb);
+  reduce_to_partial(acc, part_rs(tk), lb);
 }
 
 // K19 (tv_hpc.F90:341-346): fk = (fk + f) - ruk, plus the delta log entry.
-// LIN: ruk is the linear schedule's FP64 carried term.
+// LIN: ruk is the linear schedule's FP64 carried term.  sum: the slice's first
+// workgroup sums Err_diff's partials itself instead of a finalize launch.
 template <bool LIN>
-__global__ __launch_bounds__(NT_) void addback_kernel(const TVTask* __restrict__ tasks, int ntasks, int base) {
+__global__ __launch_bounds__(NT_) void addback_kernel(const TVTask* __restrict__ tasks, int ntasks, int base,
+                                                      bool sum) {
   const TVTask& tk = tasks[find_task_s(tasks, ntasks, base + blockIdx.x)];
   const int lb = base + blockIdx.x - tk.sb_begin;
   const size_t NT = (size_t)tk.N * tk.T;
@@ -282,10 +322,14 @@ __global__ __launch_bounds__(NT_) void addback_kernel(const TVTask* __restrict__
       else tk.fk[e] = (tk.fk[e] + tk.f[e]) - tk.ruk[e];
     }
   }
-  if (lb == 0 && threadIdx.x == 0) {
-    const int j = (int)tk.scal[126];
-    if (tk.delta_log != nullptr && j < tk.delta_cap) tk.delta_log[j] = (float)tk.scal[127];
-    tk.scal[126] = (double)(j + 1);
+  if (lb == 0) {  // uniform per workgroup
+    const double err = sum ? partials_total(part_rs(tk), tk.nb) : tk.scal[127];
+    if (threadIdx.x == 0) {
+      if (sum) tk.scal[127] = err;
+      const int j = (int)tk.scal[126];
+      if (tk.delta_log != nullptr && j < tk.delta_cap) tk.delta_log[j] = (float)err;
+      tk.scal[126] = (double)(j + 1);
+    }
   }
 }
 
@@ -356,23 +400,25 @@ void launch_tv_residual(const TVTask* t, int n, int base, int blocks, bool lin, 
 void launch_tv_apdot(const TVTask* t, int n, int base, int blocks, int j, hipStream_t s) {
   hipLaunchKernelGGL(apdot_kernel, dim3(blocks), dim3(NT_), 0, s, t, n, base, j);
 }
-void launch_tv_axpy(const TVTask* t, int n, int base, int blocks, int j, bool lin, hipStream_t s) {
-  if (lin) hipLaunchKernelGGL(axpy_kernel<true>, dim3(blocks), dim3(NT_), 0, s, t, n, base, j);
-  else hipLaunchKernelGGL(axpy_kernel<false>, dim3(blocks), dim3(NT_), 0, s, t, n, base, j);
+void launch_tv_axpy(const TVTask* t, int n, int base, int blocks, int sbase, int sblocks, int j, bool lin, bool inl,
+                    hipStream_t s) {
+  const dim3 g(blocks + (lin ? sblocks : 0));
+  if (lin && inl) hipLaunchKernelGGL((axpy_kernel<true, true>), g, dim3(NT_), 0, s, t, n, base, blocks, sbase, j);
+  else if (lin) hipLaunchKernelGGL((axpy_kernel<true, false>), g, dim3(NT_), 0, s, t, n, base, blocks, sbase, j);
+  else if (inl) hipLaunchKernelGGL((axpy_kernel<false, true>), g, dim3(NT_), 0, s, t, n, base, blocks, sbase, j);
+  else hipLaunchKernelGGL((axpy_kernel<false, false>), g, dim3(NT_), 0, s, t, n, base, blocks, sbase, j);
 }
-void launch_tv_sino_axpy(const TVTask* t, int n, int base, int sblocks, int j, hipStream_t s) {
-  hipLaunchKernelGGL(sino_axpy_kernel, dim3(sblocks), dim3(NT_), 0, s, t, n, base, j);
-}
-void launch_tv_pupdate(const TVTask* t, int n, int base, int blocks, int j, hipStream_t s) {
-  hipLaunchKernelGGL(pupdate_kernel, dim3(blocks), dim3(NT_), 0, s, t, n, base, j);
+void launch_tv_pupdate(const TVTask* t, int n, int base, int blocks, int j, bool inl, hipStream_t s) {
+  if (inl) hipLaunchKernelGGL(pupdate_kernel<true>, dim3(blocks), dim3(NT_), 0, s, t, n, base, j);
+  else hipLaunchKernelGGL(pupdate_kernel<false>, dim3(blocks), dim3(NT_), 0, s, t, n, base, j);
 }
 void launch_tv_shrink(const TVTask* t, int n, int base, int blocks, bool upd_ifkt, hipStream_t s) {
   if (upd_ifkt) hipLaunchKernelGGL(shrink_kernel<true>, dim3(blocks), dim3(NT_), 0, s, t, n, base);
   else hipLaunchKernelGGL(shrink_kernel<false>, dim3(blocks), dim3(NT_), 0, s, t, n, base);
 }
-void launch_tv_addback(const TVTask* t, int n, int base, int sblocks, bool lin, hipStream_t s) {
-  if (lin) hipLaunchKernelGGL(addback_kernel<true>, dim3(sblocks), dim3(NT_), 0, s, t, n, base);
-  else hipLaunchKernelGGL(addback_kernel<false>, dim3(sblocks), dim3(NT_), 0, s, t, n, base);
+void launch_tv_addback(const TVTask* t, int n, int base, int sblocks, bool lin, bool sum, hipStream_t s) {
+  if (lin) hipLaunchKernelGGL(addback_kernel<true>, dim3(sblocks), dim3(NT_), 0, s, t, n, base, sum);
+  else hipLaunchKernelGGL(addback_kernel<false>, dim3(sblocks), dim3(NT_), 0, s, t, n, base, sum);
 }
 void launch_tv_linload(const TVTask* t, int n, int base, int blocks, int sbase, int sblocks, hipStream_t s) {
   hipLaunchKernelGGL(linload_img_kernel, dim3(blocks), dim3(NT_), 0, s, t, n, base);
