@@ -139,6 +139,9 @@ struct BPTask {
   const uint8_t* tile_active;  // nsub*ntx: 1 if any cmask > 0 in the 64 x 16 sub-tile
   const float* rowterm;  // T*N (+ padding): cos(c_t) * (y - midpoint) in FP32, angle-major
   float* img;            // N*N out
+  // a pair's second slice, of the same geometry (the tables above); else null
+  const float* sino2;
+  float* img2;
 };
 
 struct FPTask {
@@ -225,6 +228,9 @@ struct BPShares { int b[XCDS + 1]; int C; };
 BPShares bp_xcd_shares(const std::vector<float>& w);
 void launch_backproject(const BPTask* d_tasks, int ntasks, int base, int tiles, int ty, bool refpos,
                         const BPShares& sh, hipStream_t s);
+// The same, with the reference's positions, for tasks of two slices each
+// (sino2, img2): the positions are computed once for both.
+void launch_backproject_pairs(const BPTask* d_tasks, int ntasks, int tiles, int ty, const BPShares& sh, hipStream_t s);
 // The same, with the reference's positions, for launches of few tiles
 // (bp_use_split): small tiles, their angle blocks over the waves of a
 // workgroup.  Counted in 64 x 8 tiles, bp_split_tiles(N) (even) per slice.

@@ -224,6 +224,14 @@ struct RFSet {
   void release() { rf.release(); ff.release(); }
 };
 
+// Backprojection tasks of one operand pair: of every slice, and, where slices
+// share their geometry, of a launch over all slices in two parts: pairs of
+// slices (pair) and the slices without a partner (rest).
+struct BPSet {
+  DevArray<BPTask> all, pair, rest;
+  void release() { all.release(); pair.release(); rest.release(); }
+};
+
 // Task arrays of one radon operand pair, one array per variant group; a
 // slice appears in the cells array only when its variant reads the cells.
 struct FPSet {
@@ -264,11 +272,15 @@ struct acu_batch {
   int ramp_variant = acu::RAMP_FP64;  // arithmetic of the ramp filter
   int bp_ty = acu::BP_TY_DEFAULT;     // backprojection tile height (16, 32 or 64)
   acu::BPShares bp_sh_all{};          // XCD shares of the backprojection over all slices
+  // slices of one geometry (N, T, wpu, angles) in pairs: each slice's partner
+  // or -1 (find_pairs), and the XCD shares of the two parts of a launch
+  std::vector<int> bp_partner;
+  acu::BPShares bp_sh_pair{}, bp_sh_rest{};
   bool bp_refpos = true;              // FBP backprojection positions in the reference's arithmetic
   bool tv_bp_refpos = true;           // the same inside tvopt's iteration
   // task sets for the fixed operand combinations of FBP / TV
   acu::RFSet rf_f, rf_fk, rf_ruk, rf_rp;  // ramp filter of f, fk, ruk, rp
-  acu::DevArray<acu::BPTask> bp_fbp, bp_ftv, bp_ifkt, bp_iukt, bp_irpt;
+  acu::BPSet bp_fbp, bp_ftv, bp_ifkt, bp_iukt, bp_irpt;
   acu::FPSet fp_uk, fp_p;  // radon(uk) -> ruk, radon(p) -> rp
   acu::DevArray<acu::TVTask> tv;
   float tv_mu = 0.f, tv_lambda = 0.f;
@@ -472,7 +484,8 @@ FFTTask ff_task(const Slice& s, const float* in, float* out) {
   return FFTTask{s.N, s.T, lg, s.ff_begin, L == 2 * s.N - 2 ? 1 : 0, s.ff_edge, s.h, s.fftG, s.fftW, in, out};
 }
 BPTask bp_task(const Slice& s, const float* in, float* out) {
-  return BPTask{s.N, s.T, s.mid, s.bp_begin, s.ntx, s.nty, s.nsub, s.bps_begin, in, s.cmask, s.scbp, s.tact, s.rowterm, out};
+  return BPTask{s.N, s.T, s.mid, s.bp_begin, s.ntx, s.nty, s.nsub, s.bps_begin, in, s.cmask, s.scbp, s.tact, s.rowterm, out,
+                nullptr, nullptr};
 }
 FPLTask fpl_task(const Slice& s, const float* img, float* out) {
   static const bool fixed_pitch = [] {
@@ -600,8 +613,74 @@ void bp_tile_work(const Slice& s, int ty, std::vector<float>& w) {
     }
 }
 
-// XCD shares of the all-slice and per-slice backprojection launches.
+// Pairs of slices with one geometry, in slice order.
+std::vector<int> find_pairs(const acu_batch* b) {
+  std::vector<int> partner(b->s.size(), -1);
+  std::map<std::tuple<int, int, int, uint64_t>, int> open;  // a slice that waits for a partner
+  for (int i = 0; i < (int)b->s.size(); ++i) {
+    const Slice& s = b->s[i];
+    if (!s.theta_set) continue;
+    const auto key = std::make_tuple(s.N, s.T, s.wpu, theta_hash(s.theta));
+    const auto it = open.find(key);
+    if (it == open.end()) {
+      open.emplace(key, i);
+    } else if (std::memcmp(b->s[it->second].theta.data(), s.theta.data(), sizeof(float) * s.T) == 0) {
+      partner[i] = it->second;
+      partner[it->second] = i;
+      open.erase(it);
+    }
+  }
+  return partner;
+}
+
+// The two parts of a backprojection launch over the first ns slices at tile
+// height ty (one part if not pairs): their tasks and the estimated work of
+// their tiles.
+struct BPParts {
+  std::vector<BPTask> pair, rest;
+  std::vector<float> pair_work, rest_work;
+};
+template <class InF, class OutF>
+BPParts bp_parts(acu_batch* b, int ns, int ty, bool pairs, InF in, OutF out) {
+  BPParts p;
+  for (int i = 0; i < ns; ++i) {
+    Slice& s = b->s[i];
+    const int j = b->bp_partner[i];
+    const bool two = pairs && j >= 0 && j < ns;
+    if (two && j < i) continue;  // with its partner's task
+    std::vector<float>& w = two ? p.pair_work : p.rest_work;
+    BPTask t = bp_task(s, in(s), out(s));
+    t.nty = bp_tiles_y(s.N, ty);
+    t.tile_begin = (int)w.size();
+    if (two) {
+      t.sino2 = in(b->s[j]);
+      t.img2 = out(b->s[j]);
+    }
+    bp_tile_work(s, ty, w);
+    (two ? p.pair : p.rest).push_back(t);
+  }
+  return p;
+}
+
+template <class InF, class OutF>
+void build_bpset(acu_batch* b, BPSet& set, InF in, OutF out) {
+  build(b, set.all, [&](Slice& s) { return bp_task(s, in(s), out(s)); });
+  set.pair.release();
+  set.rest.release();
+  const BPParts p = bp_parts(b, (int)b->s.size(), b->bp_ty, true, in, out);
+  if (p.pair.empty()) return;  // the launch is over set.all
+  set.pair.upload(p.pair, b->ctx->stream);
+  set.rest.upload(p.rest, b->ctx->stream);
+}
+
+// Pairs, and the XCD shares of the all-slice and per-slice backprojection
+// launches.
 void assign_bp_shares(acu_batch* b) {
+  b->bp_partner = find_pairs(b);
+  const auto none = [](Slice&) { return (float*)nullptr; };
+  const BPParts p = bp_parts(b, (int)b->s.size(), b->bp_ty, true, none, none);
+  b->bp_sh_pair = bp_xcd_shares(p.pair_work);
+  b->bp_sh_rest = bp_xcd_shares(p.rest_work);
   std::vector<float> all, one;
   for (auto& s : b->s) {
     one.clear();
@@ -642,17 +721,17 @@ void set_bp_tile(acu_batch* b, int ty) {
 
 void build_op_tasks(acu_batch* b) {
   build_rfset(b, b->rf_f, [](Slice& s) { return (const float*)s.f; }, [](Slice& s) { return s.sinoCS; });
-  build(b, b->bp_fbp, [](Slice& s) { return bp_task(s, s.sinoCS, s.fbp); });
+  build_bpset(b, b->bp_fbp, [](Slice& s) { return s.sinoCS; }, [](Slice& s) { return s.fbp; });
 }
 
 void build_tv_tasks(acu_batch* b) {
   build_rfset(b, b->rf_fk, [](Slice& s) { return (const float*)s.fk; }, [](Slice& s) { return s.sinoCS; });
   build_rfset(b, b->rf_ruk, [](Slice& s) { return (const float*)s.ruk; }, [](Slice& s) { return s.sinoCS; });
   build_rfset(b, b->rf_rp, [](Slice& s) { return (const float*)s.rp; }, [](Slice& s) { return s.sinoCS; });
-  build(b, b->bp_ftv, [](Slice& s) { return bp_task(s, s.sinoCS, s.ftv); });
-  build(b, b->bp_ifkt, [](Slice& s) { return bp_task(s, s.sinoCS, s.ifkt); });
-  build(b, b->bp_iukt, [](Slice& s) { return bp_task(s, s.sinoCS, s.iukt); });
-  build(b, b->bp_irpt, [](Slice& s) { return bp_task(s, s.sinoCS, s.irpt); });
+  build_bpset(b, b->bp_ftv, [](Slice& s) { return s.sinoCS; }, [](Slice& s) { return s.ftv; });
+  build_bpset(b, b->bp_ifkt, [](Slice& s) { return s.sinoCS; }, [](Slice& s) { return s.ifkt; });
+  build_bpset(b, b->bp_iukt, [](Slice& s) { return s.sinoCS; }, [](Slice& s) { return s.iukt; });
+  build_bpset(b, b->bp_irpt, [](Slice& s) { return s.sinoCS; }, [](Slice& s) { return s.irpt; });
   build_fpset(b, b->fp_uk, [](Slice& s) { return (const float*)s.uk; }, [](Slice& s) { return s.ruk; });
   build_fpset(b, b->fp_p, [](Slice& s) { return (const float*)s.p; }, [](Slice& s) { return s.rp; });
 }
@@ -703,8 +782,6 @@ void require_theta(acu_batch* b) {
 // ---- operator sequences (all slices at once, or one slice: sl >= 0) ----
 struct Range { int base, n; };
 Range rf_range(acu_batch* b, int sl) { return sl < 0 ? Range{0, b->rf_total} : Range{b->s[sl].rf_begin, b->s[sl].rf_n}; }
-Range bp_range(acu_batch* b, int sl) { return sl < 0 ? Range{0, b->bp_total} : Range{b->s[sl].bp_begin, b->s[sl].bp_n}; }
-const BPShares& bp_shares(const acu_batch* b, int sl) { return sl < 0 ? b->bp_sh_all : b->s[sl].bp_sh; }
 Range ew_range(acu_batch* b, int sl) { return sl < 0 ? Range{0, b->ew_total} : Range{b->s[sl].ew_begin, b->s[sl].ew_n}; }
 Range sw_range(acu_batch* b, int sl) { return sl < 0 ? Range{0, b->sw_total} : Range{b->s[sl].sw_begin, b->s[sl].sw_n}; }
 
@@ -732,20 +809,35 @@ void ramp_seq(acu_batch* b, const RFSet& rf, int sl) {
   timed(b->ctx, K_RF, [&] { launch_ramp_any(b, rf, sl, b->ramp_variant); });
 }
 
-// One backprojection launch: of all slices (sl < 0) or one with a task array
-// of all, or of slice sl with a task of its own (own).
-void backproject(acu_batch* b, const BPTask* d, int n, int sl, bool own, bool refpos) {
+// One backprojection of slice sl by a task array d of n slices, at its range
+// of the tiles of all slices, or at its first tiles (own).
+void backproject_one(acu_batch* b, const BPTask* d, int n, int sl, bool own, bool refpos) {
   hipStream_t st = b->ctx->stream;
-  const Range r = bp_range(b, sl), rs = sl < 0 ? Range{0, b->bps_total} : Range{b->s[sl].bps_begin, b->s[sl].bps_n};
-  if (refpos && bp_use_split(rs.n)) launch_backproject_split(d, n, own ? 0 : rs.base, rs.n, st);
-  else launch_backproject(d, n, own ? 0 : r.base, r.n, b->bp_ty, refpos, bp_shares(b, sl), st);
+  const Slice& s = b->s[sl];
+  if (refpos && bp_use_split(s.bps_n)) launch_backproject_split(d, n, own ? 0 : s.bps_begin, s.bps_n, st);
+  else launch_backproject(d, n, own ? 0 : s.bp_begin, s.bp_n, b->bp_ty, refpos, s.bp_sh, st);
+}
+
+// Backprojection of all slices (sl < 0) or one.  With the reference's
+// positions slices of one geometry go two to a workgroup (the same bits).
+void backproject(acu_batch* b, const BPSet& bp, int sl, bool refpos) {
+  if (sl >= 0) return backproject_one(b, bp.all.d, bp.all.n, sl, false, refpos);
+  hipStream_t st = b->ctx->stream;
+  if (refpos && bp_use_split(b->bps_total)) {
+    launch_backproject_split(bp.all.d, bp.all.n, 0, b->bps_total, st);
+  } else if (refpos && bp.pair.n > 0) {
+    launch_backproject_pairs(bp.pair.d, bp.pair.n, b->bp_sh_pair.b[XCDS], b->bp_ty, b->bp_sh_pair, st);
+    launch_backproject(bp.rest.d, bp.rest.n, 0, b->bp_sh_rest.b[XCDS], b->bp_ty, true, b->bp_sh_rest, st);
+  } else {
+    launch_backproject(bp.all.d, bp.all.n, 0, b->bp_total, b->bp_ty, refpos, b->bp_sh_all, st);
+  }
 }
 
 // refpos: the backprojection positions (the batch's FBP positions, or
 // tvopt's inside its iteration)
-void iradon_seq(acu_batch* b, const RFSet& rf, const DevArray<BPTask>& bp, int sl, bool refpos) {
+void iradon_seq(acu_batch* b, const RFSet& rf, const BPSet& bp, int sl, bool refpos) {
   ramp_seq(b, rf, sl);
-  timed(b->ctx, K_BP, [&] { backproject(b, bp.d, bp.n, sl, false, refpos); });
+  timed(b->ctx, K_BP, [&] { backproject(b, bp, sl, refpos); });
   check_launch();
 }
 
@@ -863,8 +955,8 @@ void fbp_all(acu_batch* b, int sl) {
 }
 
 // the backprojection alone (its ramp-filtered input is already in place)
-void bp_seq(acu_batch* b, const DevArray<BPTask>& bp, int sl, bool refpos) {
-  timed(b->ctx, K_BP, [&] { backproject(b, bp.d, bp.n, sl, false, refpos); });
+void bp_seq(acu_batch* b, const BPSet& bp, int sl, bool refpos) {
+  timed(b->ctx, K_BP, [&] { backproject(b, bp, sl, refpos); });
   check_launch();
 }
 
@@ -1050,7 +1142,7 @@ void bp_dev(acu_batch* b, int sl, float* img, const float* filt) {
   BPTask t = bp_task(s, filt, img);
   t.tile_begin = t.split_begin = 0;
   BPTask* d = put_adhoc(b, t);
-  timed(c, K_BP, [&] { backproject(b, d, 1, sl, true, b->bp_refpos); });
+  timed(c, K_BP, [&] { backproject_one(b, d, 1, sl, true, b->bp_refpos); });
   check_launch();
 }
 
@@ -1194,24 +1286,21 @@ double time_bp(acu_batch* b, int ty, int reps) {
   for (int i = 0; i < ns; ++i) total += (size_t)b->s[i].N * b->s[i].N;
   struct Scratch { float* p = nullptr; ~Scratch() { if (p) hipFree(p); } } sc;
   ACU_HIP_CHECK(hipMalloc(&sc.p, total * sizeof(float)));
-  std::vector<BPTask> tv;
-  int tiles = 0;
+  std::map<const Slice*, float*> img;
   size_t off = 0;
   for (int i = 0; i < ns; ++i) {
-    const Slice& s = b->s[i];
-    BPTask t = bp_task(s, s.sinoCS, sc.p + off);
-    t.nty = bp_tiles_y(s.N, ty);
-    t.tile_begin = tiles;
-    tiles += s.ntx * t.nty;
-    off += (size_t)s.N * s.N;
-    tv.push_back(t);
+    img[&b->s[i]] = sc.p + off;
+    off += (size_t)b->s[i].N * b->s[i].N;
   }
-  DevArray<BPTask> arr;
-  arr.upload(tv, b->ctx->stream);
-  std::vector<float> w;
-  for (int i = 0; i < ns; ++i) bp_tile_work(b->s[i], ty, w);
-  const BPShares sh = bp_xcd_shares(w);
-  auto run = [&] { launch_backproject(arr.d, arr.n, 0, tiles, ty, b->bp_refpos, sh, c->stream); };
+  const BPParts p = bp_parts(b, ns, ty, b->bp_refpos, [](Slice& s) { return s.sinoCS; }, [&](Slice& s) { return img[&s]; });
+  struct Tasks : DevArray<BPTask> { ~Tasks() { release(); } } pair, rest;
+  pair.upload(p.pair, c->stream);
+  rest.upload(p.rest, c->stream);
+  const BPShares shp = bp_xcd_shares(p.pair_work), shr = bp_xcd_shares(p.rest_work);
+  auto run = [&] {
+    launch_backproject_pairs(pair.d, pair.n, shp.b[XCDS], ty, shp, c->stream);
+    launch_backproject(rest.d, rest.n, 0, shr.b[XCDS], ty, b->bp_refpos, shr, c->stream);
+  };
   hipEvent_t e0 = c->ev(), e1 = c->ev();
   run();
   ACU_HIP_CHECK(hipEventRecord(e0, c->stream));
@@ -1223,7 +1312,6 @@ double time_bp(acu_batch* b, int ty, int reps) {
   ACU_HIP_CHECK(hipEventElapsedTime(&ms, e0, e1));
   c->pool.push_back(e0);
   c->pool.push_back(e1);
-  arr.release();
   return (double)ms / reps;
 }
 
@@ -1620,7 +1708,11 @@ int acu_batch_set_theta(acu_batch* b, int slice, const float* theta_deg) {
           std::memcpy(b->s[slice].theta.data(), theta_deg, sizeof(float) * b->s[slice].T);
           acu::upload_theta(b, slice);
           // whether the cells pass is launched depends on the angles
-          try { acu::refresh_fp(b); } catch (...) { b->s[slice].theta_set = false; throw; });
+          // and so does which slices the backprojection takes together
+          try {
+            if (b->s.size() > 1) acu::assign_bp_shares(b), acu::build_op_tasks(b);
+            acu::refresh_fp(b);
+          } catch (...) { b->s[slice].theta_set = false; throw; });
 }
 
 int acu_batch_set_sino(acu_batch* b, int slice, const float* f_host) {

@@ -35,8 +35,21 @@
 //    in both, y1 = floor(yr) and the pair's LDS offset come from v_fract and
 //    full-rate float arithmetic (lds_units) instead of v_cvt and
 //    v_lshl_add: 551 against 575 us per 4 x 1025^2 x 720 launch, 6.23
-//    against 6.34 ms per 8 x 2049^2 x 1500 (0.79 ms a slice; the kernel is
-//    bound by its VALU issue, 1.4-1.5 wave-instructions per CU and clock);
+//    against 6.34 ms per 8 x 2049^2 x 1500;
+//  * REFPOS keeps scalar loads out of the loop over angles: the rows' terms,
+//    the sine and the window's base come from LDS, which answers in order,
+//    so the wait for one half of the rows' taps leaves the other half's and
+//    the next angle's in flight (a scalar load outstanding turns every such
+//    wait into a wait for all).  8 x 2049^2 x 1500 6.33 to 5.75 ms, 2 x
+//    1025^2 x 720 at TY = 16 360 to 260 us;
+//  * a pair of slices of one geometry (G = 2, REFPOS) shares positions,
+//    weights and offsets: 4.5 VALU instructions an update instead of 7.  The
+//    windows are two arrays read by two ds_read_b64 (2.2 clocks each; one
+//    ds_read2st64_b64 takes 8, a b128 of interleaved pairs 5.9 with its bank
+//    conflicts), staged 16 angles at a time so that 5 workgroups fit a CU.
+//    8 x 2049^2 x 1500 5.75 to 5.07 ms (0.63 ms a slice), 4 x 1025^2 x 720
+//    490 to 390 us.  1.25 wave-instructions per CU and clock, LDS 69% busy,
+//    at 1.95 GHz (2.1 with one slice): the power limit is near as well;
 //  * each 32-angle block is summed separately and then added;
 //  * tiles whose mask is identically zero (by 64 x 16 sub-tiles) only store
 //    zeros.
@@ -66,15 +79,22 @@ __device__ __forceinline__ int find_task(const BPTask* tasks, int ntasks, int gt
   return lo;
 }
 
-template <int TY, bool REFPOS>
+template <int TY, bool REFPOS, int G>
 __global__ __launch_bounds__(64 * bp_waves(TY)) void bp_kernel(const BPTask* __restrict__ tasks, int ntasks, int base,
                                                                BPShares sh) {
-  constexpr int NW = bp_waves(TY), NT = 64 * NW, PY = TY / NW, W = bp_window(TY), SUBS = TY / BP_SUB;
-  constexpr int SPA = NT / AB, NST = W / SPA;  // staging threads per angle, pairs per thread
-  static_assert(TY % BP_SUB == 0 && TY % NW == 0 && NT % AB == 0 && W % SPA == 0, "tile shape");
-  __shared__ float2 P[AB * W];
-  __shared__ int lo_s[AB];
-  __shared__ float k_s[AB];    // K of the tile-local position (see above)
+  constexpr int NW = bp_waves(TY), NT = 64 * NW, PY = TY / NW, SUBS = TY / BP_SUB;
+  constexpr int AS = G == 2 ? 16 : AB;  // angles staged at a time (G = 1 with 16: 2% slower)
+  constexpr int W = (G == 2 && TY == 16) ? 80 : bp_window(TY);
+  constexpr int SPA = NT / AS, NST = W / SPA;  // staging threads per angle, pairs per thread
+  static_assert(G == 1 || (G == 2 && REFPOS), "pairs have the reference's positions");
+  static_assert(TY % BP_SUB == 0 && TY % NW == 0 && NT % AS == 0 && W % SPA == 0 && AB % AS == 0, "tile shape");
+  constexpr int P2 = AS * W + 1;  // second slice's window; not a multiple of 512 bytes, which would merge the reads
+  __shared__ float2 P[G == 2 ? P2 + AS * W : AS * W];
+  __shared__ int lo_s[AS];
+  __shared__ float k_s[AS];    // K of the tile-local position (see above)
+  // row terms of the tile
+  __shared__ __attribute__((aligned(16))) float rt_s[REFPOS ? AS * TY : 1];
+  __shared__ float2 ab_s[REFPOS ? AS : 1];  // sine, LDS offset of P[a * W - 1 - lo] (lds_units)
 
   // XCD k (xcd_remap) runs the tiles of its share in order
   const int l = xcd_remap(blockIdx.x, gridDim.x);
@@ -103,7 +123,10 @@ __global__ __launch_bounds__(64 * bp_waves(TY)) void bp_kernel(const BPTask* __r
     if (x < N) {
 #pragma unroll
       for (int r = 0; r < PY; ++r)
-        if (yb + r < N) tk.img[(size_t)(yb + r) * N + x] = 0.0f;
+        if (yb + r < N) {
+          tk.img[(size_t)(yb + r) * N + x] = 0.0f;
+          if (G == 2) tk.img2[(size_t)(yb + r) * N + x] = 0.0f;
+        }
     }
     return;
   }
@@ -119,16 +142,19 @@ __global__ __launch_bounds__(64 * bp_waves(TY)) void bp_kernel(const BPTask* __r
   const float cx0 = (float)(x0 + 1) - m, cx1 = (float)(x0 + TX) - m;
   const float cy0 = (float)(y0 + 1) - m, cy1 = (float)(y0 + TY) - m;
 
-  float acc[PY];
+  float acc[G][PY];
 #pragma unroll
-  for (int r = 0; r < PY; ++r) acc[r] = 0.0f;
+  for (int g = 0; g < G; ++g)
+#pragma unroll
+    for (int r = 0; r < PY; ++r) acc[g][r] = 0.0f;
 
-  const ACU_GLOBAL float* __restrict__ S = as_global(tk.sino);
+  const ACU_GLOBAL float* __restrict__ S[2] = {as_global(tk.sino), as_global(G == 2 ? tk.sino2 : tk.sino)};
   const float2* __restrict__ sc = tk.sc;
   const int sa = tid / SPA, sj = tid % SPA;  // staging: angle of the block, first bin
 
-  for (int a0 = 0; a0 < T; a0 += AB) {
-    const int na = min(AB, T - a0);
+  float blk[G][PY];  // the 32-angle block's sums
+  for (int a0 = 0; a0 < T; a0 += AS) {
+    const int na = min(AS, T - a0);
     // window start per angle: lowest 0-based detector position over the tile, minus one bin
     if (tid < na) {
       const float2 v = const_f2(sc, a0 + tid);
@@ -136,50 +162,89 @@ __global__ __launch_bounds__(64 * bp_waves(TY)) void bp_kernel(const BPTask* __r
       const float ey = fminf(v.y * cy0, v.y * cy1);
       const int lo = (int)floorf(ex + ey + m - 1.0f) - 1;
       lo_s[tid] = lo;
-      k_s[tid] = (float)((double)v.x * (double)cx0 + (double)v.y * (double)cy0 + (double)m - 1.0 -
+      if (!REFPOS)
+        k_s[tid] = (float)((double)v.x * (double)cx0 + (double)v.y * (double)cy0 + (double)m - 1.0 -
                          (double)lo);
+      if (REFPOS) ab_s[tid] = make_float2(v.x, lds_base(8 * (tid * W - 1 - lo)));
+    }
+    if (REFPOS) {
+#pragma unroll
+      for (int i = 0; i < AS * TY; i += NT) {
+        const int a = (i + tid) / TY, r = (i + tid) % TY;
+        rt_s[i + tid] = as_global(tk.rowterm)[(size_t)min(a0 + a, T - 1) * N + y0 + r];
+      }
     }
     __syncthreads();
     if (sa < na) {
       const int lo = lo_s[sa];
-      const ACU_GLOBAL float* row = S + (size_t)(a0 + sa) * N;
-      float2 v[NST];
+      float2 v[G][NST];
 #pragma unroll
-      for (int k = 0; k < NST; ++k) {
-        const int dc = min(max(lo + sj + SPA * k, 1), N - 2);  // N >= 3: row[dc + 1] is in the row
-        v[k] = make_float2(row[dc], row[dc + 1]);
+      for (int g = 0; g < G; ++g) {
+        const ACU_GLOBAL float* row = S[g] + (size_t)(a0 + sa) * N;
+#pragma unroll
+        for (int k = 0; k < NST; ++k) {
+          const int dc = min(max(lo + sj + SPA * k, 1), N - 2);  // N >= 3: row[dc + 1] is in the row
+          v[g][k] = make_float2(row[dc], row[dc + 1]);
+        }
       }
 #pragma unroll
       for (int k = 0; k < NST; ++k) {
         const int d = lo + sj + SPA * k;
-        P[sa * W + sj + SPA * k] = (d >= 1 && d <= N - 2) ? make_float2(v[k].x, v[k].y - v[k].x)
-                                                          : make_float2(0.0f, 0.0f);
+        const bool in = d >= 1 && d <= N - 2;
+#pragma unroll
+        for (int g = 0; g < G; ++g)
+          P[g * P2 + sa * W + sj + SPA * k] = in ? make_float2(v[g][k].x, v[g][k].y - v[g][k].x) : make_float2(0.0f, 0.0f);
       }
     }
     __syncthreads();
-    float blk[PY];
+    if (a0 % AB == 0) {
 #pragma unroll
-    for (int r = 0; r < PY; ++r) blk[r] = 0.0f;
+      for (int g = 0; g < G; ++g)
+#pragma unroll
+        for (int r = 0; r < PY; ++r) blk[g][r] = 0.0f;
+    }
     if (REFPOS) {
-      // the wave's rows of the row-term table: wave-uniform, scalar loads
-      const int ybu = __builtin_amdgcn_readfirstlane(yb);
-      const ACU_CONST float* rt = as_const(tk.rowterm) + (size_t)a0 * N + ybu;
-      for (int a = 0; a < na; ++a, rt += N) {
 #pragma clang fp contract(off)
-        const float sa = const_f2(sc, a0 + a).x;
-        const float A = sa * ux;  // sin(c)*(jx-midpoint), tv_hpc.F90:114
-        // offset of P[a*W - 1 - lo] (wave-uniform): the pair of the 1-based
-        // tap y1 is 8*y1 bytes on
-        const float base = lds_base(__builtin_amdgcn_readfirstlane(8 * (a * W - 1 - lo_s[a])));
+      // the rows in two halves: one half's taps are in flight while the other
+      // half's (of the angle before, at first) are added
+      constexpr int H = PY / 2;
+      float2 q[2][H][G];
+      float fr[2][H];
 #pragma unroll
-        for (int r = 0; r < PY; ++r) {
-          const float yr = (A + rt[r]) + m;  // (sin(c)*(jx-m) + cos(c)*(jy-m)) + m
-          const float fr = __builtin_amdgcn_fractf(yr);  // yr - y1, y1 = floor(yr) = yr - fr, both exact
-          const unsigned o = __float_as_uint(fmaf(yr - fr, lds_units(8), base));
-          const float2 pv = *(const float2*)((const char*)P + o);
-          blk[r] += fmaf(fr, pv.y, pv.x);
+      for (int h = 0; h < H; ++h) {
+        fr[1][h] = 0.0f;
+#pragma unroll
+        for (int g = 0; g < G; ++g) q[1][h][g] = make_float2(0.0f, 0.0f);
+      }
+      const float* rts = rt_s + wave * PY;
+      for (int a = 0; a < na; ++a) {
+        const float2 ab = ab_s[a];
+        float rv[PY];
+#pragma unroll
+        for (int r = 0; r < PY; ++r) rv[r] = rts[a * TY + r];
+        const float A = ab.x * ux;  // sin(c)*(jx-midpoint), tv_hpc.F90:114
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+#pragma unroll
+          for (int h = 0; h < H; ++h) {
+            const float yr = (A + rv[u * H + h]) + m;  // (sin(c)*(jx-m) + cos(c)*(jy-m)) + m
+            // yr - y1; y1 = floor(yr) = yr - fr, both exact
+            fr[u][h] = __builtin_amdgcn_fractf(yr);
+            const unsigned o = __float_as_uint(fmaf(yr - fr[u][h], lds_units(8), ab.y));
+#pragma unroll
+            for (int g = 0; g < G; ++g) q[u][h][g] = *(const float2*)((const char*)(P + g * P2) + o);
+          }
+#pragma unroll
+          for (int h = 0; h < H; ++h)
+#pragma unroll
+            for (int g = 0; g < G; ++g)
+              blk[g][(1 - u) * H + h] += fmaf(fr[1 - u][h], q[1 - u][h][g].y, q[1 - u][h][g].x);
         }
       }
+#pragma unroll
+      for (int h = 0; h < H; ++h)
+#pragma unroll
+        for (int g = 0; g < G; ++g) blk[g][H + h] += fmaf(fr[1][h], q[1][h][g].y, q[1][h][g].x);
     } else {
       for (int a = 0; a < na; ++a) {
         const float2 v = const_f2(sc, a0 + a);
@@ -191,12 +256,16 @@ __global__ __launch_bounds__(64 * bp_waves(TY)) void bp_kernel(const BPTask* __r
           const float fr = __builtin_amdgcn_fractf(yr);
           const unsigned o = __float_as_uint(fmaf(yr - fr, lds_units(8), Pa));
           const float2 pv = *(const float2*)((const char*)P + o);
-          blk[r] += fmaf(fr, pv.y, pv.x);
+          blk[0][r] += fmaf(fr, pv.y, pv.x);
         }
       }
     }
+    if (a0 % AB == AB - AS || a0 + AS >= T) {
 #pragma unroll
-    for (int r = 0; r < PY; ++r) acc[r] += blk[r];
+      for (int g = 0; g < G; ++g)
+#pragma unroll
+        for (int r = 0; r < PY; ++r) acc[g][r] += blk[g][r];
+    }
     __syncthreads();
   }
 
@@ -206,7 +275,9 @@ __global__ __launch_bounds__(64 * bp_waves(TY)) void bp_kernel(const BPTask* __r
       const int y = yb + r;
       if (y < N) {
         const size_t o = (size_t)y * N + x;
-        tk.img[o] = tk.cmask[o] * acc[r];
+        const float cm = tk.cmask[o];
+        tk.img[o] = cm * acc[0][r];
+        if (G == 2) tk.img2[o] = cm * acc[G - 1][r];
       }
     }
   }
@@ -369,23 +440,33 @@ void launch_bp_rowterm(const float2* sc, int N, int T, float mid, float* rowterm
 int bp_tiles_x(int N) { return (N + TX - 1) / TX; }
 int bp_tiles_y(int N, int ty) { return (N + ty - 1) / ty; }
 
-template <bool REFPOS>
+template <bool REFPOS, int G>
 void launch_bp(const BPTask* d_tasks, int ntasks, int base, int ty, const BPShares& sh, hipStream_t s) {
   const dim3 g((unsigned)(XCDS * sh.C));
   switch (ty) {
-    case 16: hipLaunchKernelGGL((bp_kernel<16, REFPOS>), g, dim3(64 * bp_waves(16)), 0, s, d_tasks, ntasks, base, sh); break;
-    case 32: hipLaunchKernelGGL((bp_kernel<32, REFPOS>), g, dim3(64 * bp_waves(32)), 0, s, d_tasks, ntasks, base, sh); break;
-    case 64: hipLaunchKernelGGL((bp_kernel<64, REFPOS>), g, dim3(64 * bp_waves(64)), 0, s, d_tasks, ntasks, base, sh); break;
+    case 16: hipLaunchKernelGGL((bp_kernel<16, REFPOS, G>), g, dim3(64 * bp_waves(16)), 0, s, d_tasks, ntasks, base, sh); break;
+    case 32: hipLaunchKernelGGL((bp_kernel<32, REFPOS, G>), g, dim3(64 * bp_waves(32)), 0, s, d_tasks, ntasks, base, sh); break;
+    case 64: hipLaunchKernelGGL((bp_kernel<64, REFPOS, G>), g, dim3(64 * bp_waves(64)), 0, s, d_tasks, ntasks, base, sh); break;
     default: throw Error("backprojection tile height must be 16, 32 or 64");
   }
+}
+
+void check_bp_launch(int tiles, const BPShares& sh) {
+  if (sh.b[0] != 0 || sh.b[XCDS] != tiles || sh.C < 1) throw Error("backprojection shares do not match the launch");
 }
 
 void launch_backproject(const BPTask* d_tasks, int ntasks, int base, int tiles, int ty, bool refpos,
                         const BPShares& sh, hipStream_t s) {
   if (tiles <= 0) return;
-  if (sh.b[0] != 0 || sh.b[XCDS] != tiles || sh.C < 1) throw Error("backprojection shares do not match the launch");
-  if (refpos) launch_bp<true>(d_tasks, ntasks, base, ty, sh, s);
-  else launch_bp<false>(d_tasks, ntasks, base, ty, sh, s);
+  check_bp_launch(tiles, sh);
+  if (refpos) launch_bp<true, 1>(d_tasks, ntasks, base, ty, sh, s);
+  else launch_bp<false, 1>(d_tasks, ntasks, base, ty, sh, s);
+}
+
+void launch_backproject_pairs(const BPTask* d_tasks, int ntasks, int tiles, int ty, const BPShares& sh, hipStream_t s) {
+  if (tiles <= 0) return;
+  check_bp_launch(tiles, sh);
+  launch_bp<true, 2>(d_tasks, ntasks, 0, ty, sh, s);
 }
 
 // Cut points at k/XCDS of the total estimated work (a tile starts the next
