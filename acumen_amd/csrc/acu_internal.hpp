@@ -235,7 +235,13 @@ void launch_backproject_pairs(const BPTask* d_tasks, int ntasks, int tiles, int 
 // (bp_use_split): small tiles, their angle blocks over the waves of a
 // workgroup.  Counted in 64 x 8 tiles, bp_split_tiles(N) (even) per slice.
 int bp_split_tiles(int N);
-bool bp_use_split(int tiles);
+// tile height of a batch of that many 64 x 8 tiles: ty (its setting) when
+// they fill the GPU several times over, else 16
+int bp_launch_height(int tiles, int ty);
+// whether a launch of that many 64 x 8 tiles takes slices in pairs; rest:
+// some slices have no partner
+bool bp_use_pairs(int tiles, bool rest);
+bool bp_use_split(int tiles, int T);  // T: the launch's most angles
 void launch_backproject_split(const BPTask* d_tasks, int ntasks, int base, int tiles, hipStream_t s);
 void launch_cells(const CellTask* d_tasks, int ntasks, int base, int blocks, hipStream_t s);
 // rowterm[t*N + y] = cos(c_t) * ((y+1) - mid), one FP32 product each (the

@@ -270,11 +270,14 @@ struct acu_batch {
   acu::DevArray<int> fl_ord_all[acu::FL_GROUPS], fl_ord_one[acu::FL_GROUPS];
   bool fpl_order = true;
   int ramp_variant = acu::RAMP_FP64;  // arithmetic of the ramp filter
-  int bp_ty = acu::BP_TY_DEFAULT;     // backprojection tile height (16, 32 or 64)
+  int bp_ty = acu::BP_TY_DEFAULT;     // backprojection tile height (16, 32 or 64) as set
+  int bp_h = acu::BP_TY_DEFAULT;      // the height its launches have (bp_launch_height)
   acu::BPShares bp_sh_all{};          // XCD shares of the backprojection over all slices
   // slices of one geometry (N, T, wpu, angles) in pairs: each slice's partner
   // or -1 (find_pairs), and the XCD shares of the two parts of a launch
   std::vector<int> bp_partner;
+  bool bp_pairs = false;              // whether launches over all slices take them (bp_use_pairs)
+  int maxT = 0;                       // most angles of a slice
   acu::BPShares bp_sh_pair{}, bp_sh_rest{};
   bool bp_refpos = true;              // FBP backprojection positions in the reference's arithmetic
   bool tv_bp_refpos = true;           // the same inside tvopt's iteration
@@ -667,8 +670,8 @@ void build_bpset(acu_batch* b, BPSet& set, InF in, OutF out) {
   build(b, set.all, [&](Slice& s) { return bp_task(s, in(s), out(s)); });
   set.pair.release();
   set.rest.release();
-  const BPParts p = bp_parts(b, (int)b->s.size(), b->bp_ty, true, in, out);
-  if (p.pair.empty()) return;  // the launch is over set.all
+  if (!b->bp_pairs) return;  // the launch is over set.all
+  const BPParts p = bp_parts(b, (int)b->s.size(), b->bp_h, true, in, out);
   set.pair.upload(p.pair, b->ctx->stream);
   set.rest.upload(p.rest, b->ctx->stream);
 }
@@ -678,13 +681,14 @@ void build_bpset(acu_batch* b, BPSet& set, InF in, OutF out) {
 void assign_bp_shares(acu_batch* b) {
   b->bp_partner = find_pairs(b);
   const auto none = [](Slice&) { return (float*)nullptr; };
-  const BPParts p = bp_parts(b, (int)b->s.size(), b->bp_ty, true, none, none);
+  const BPParts p = bp_parts(b, (int)b->s.size(), b->bp_h, true, none, none);
+  b->bp_pairs = !p.pair.empty() && bp_use_pairs(b->bps_total, !p.rest.empty());
   b->bp_sh_pair = bp_xcd_shares(p.pair_work);
   b->bp_sh_rest = bp_xcd_shares(p.rest_work);
   std::vector<float> all, one;
   for (auto& s : b->s) {
     one.clear();
-    bp_tile_work(s, b->bp_ty, one);
+    bp_tile_work(s, b->bp_h, one);
     s.bp_sh = bp_xcd_shares(one);
     all.insert(all.end(), one.begin(), one.end());
   }
@@ -697,9 +701,13 @@ void assign_bp(acu_batch* b) {
   int bp = 0, bps = 0;
   bool tables = true;
   for (auto& s : b->s) {
-    s.nty = bp_tiles_y(s.N, b->bp_ty);
-    s.bp_begin = bp; s.bp_n = s.ntx * s.nty; bp += s.bp_n;
     s.bps_begin = bps; s.bps_n = bp_split_tiles(s.N); bps += s.bps_n;
+    b->maxT = std::max(b->maxT, s.T);
+  }
+  b->bp_h = bp_launch_height(bps, b->bp_ty);
+  for (auto& s : b->s) {
+    s.nty = bp_tiles_y(s.N, b->bp_h);
+    s.bp_begin = bp; s.bp_n = s.ntx * s.nty; bp += s.bp_n;
     tables = tables && !s.tact_h.empty();
   }
   b->bp_total = bp;
@@ -814,8 +822,8 @@ void ramp_seq(acu_batch* b, const RFSet& rf, int sl) {
 void backproject_one(acu_batch* b, const BPTask* d, int n, int sl, bool own, bool refpos) {
   hipStream_t st = b->ctx->stream;
   const Slice& s = b->s[sl];
-  if (refpos && bp_use_split(s.bps_n)) launch_backproject_split(d, n, own ? 0 : s.bps_begin, s.bps_n, st);
-  else launch_backproject(d, n, own ? 0 : s.bp_begin, s.bp_n, b->bp_ty, refpos, s.bp_sh, st);
+  if (refpos && bp_use_split(s.bps_n, s.T)) launch_backproject_split(d, n, own ? 0 : s.bps_begin, s.bps_n, st);
+  else launch_backproject(d, n, own ? 0 : s.bp_begin, s.bp_n, b->bp_h, refpos, s.bp_sh, st);
 }
 
 // Backprojection of all slices (sl < 0) or one.  With the reference's
@@ -823,13 +831,13 @@ void backproject_one(acu_batch* b, const BPTask* d, int n, int sl, bool own, boo
 void backproject(acu_batch* b, const BPSet& bp, int sl, bool refpos) {
   if (sl >= 0) return backproject_one(b, bp.all.d, bp.all.n, sl, false, refpos);
   hipStream_t st = b->ctx->stream;
-  if (refpos && bp_use_split(b->bps_total)) {
+  if (refpos && bp_use_split(b->bps_total, b->maxT)) {
     launch_backproject_split(bp.all.d, bp.all.n, 0, b->bps_total, st);
-  } else if (refpos && bp.pair.n > 0) {
-    launch_backproject_pairs(bp.pair.d, bp.pair.n, b->bp_sh_pair.b[XCDS], b->bp_ty, b->bp_sh_pair, st);
-    launch_backproject(bp.rest.d, bp.rest.n, 0, b->bp_sh_rest.b[XCDS], b->bp_ty, true, b->bp_sh_rest, st);
+  } else if (refpos && b->bp_pairs) {
+    launch_backproject_pairs(bp.pair.d, bp.pair.n, b->bp_sh_pair.b[XCDS], b->bp_h, b->bp_sh_pair, st);
+    launch_backproject(bp.rest.d, bp.rest.n, 0, b->bp_sh_rest.b[XCDS], b->bp_h, true, b->bp_sh_rest, st);
   } else {
-    launch_backproject(bp.all.d, bp.all.n, 0, b->bp_total, b->bp_ty, refpos, b->bp_sh_all, st);
+    launch_backproject(bp.all.d, bp.all.n, 0, b->bp_total, b->bp_h, refpos, b->bp_sh_all, st);
   }
 }
 
@@ -1292,7 +1300,7 @@ double time_bp(acu_batch* b, int ty, int reps) {
     img[&b->s[i]] = sc.p + off;
     off += (size_t)b->s[i].N * b->s[i].N;
   }
-  const BPParts p = bp_parts(b, ns, ty, b->bp_refpos, [](Slice& s) { return s.sinoCS; }, [&](Slice& s) { return img[&s]; });
+  const BPParts p = bp_parts(b, ns, ty, b->bp_refpos && b->bp_pairs, [](Slice& s) { return s.sinoCS; }, [&](Slice& s) { return img[&s]; });
   struct Tasks : DevArray<BPTask> { ~Tasks() { release(); } } pair, rest;
   pair.upload(p.pair, c->stream);
   rest.upload(p.rest, c->stream);

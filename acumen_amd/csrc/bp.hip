@@ -283,42 +283,42 @@ __global__ __launch_bounds__(64 * bp_waves(TY)) void bp_kernel(const BPTask* __r
   }
 }
 
-// Backprojection of small launches, with the reference's positions.  A tile
-// of the kernel above walks its angles serially: 4 waves of 8 rows, so a
-// 257^2 x 180 slice is 45 workgroups on 256 CUs, each a chain of 6 blocks of
-// staging and 32 angles.  Here a workgroup of 8 waves takes a 64 x ROWS tile
-// and every wave another block of 32 angles: each stages its own window in
-// its own part of LDS (BPS_AB angles at a time, no barrier), and the blocks'
-// sums are then added in block order, so the result is the other kernel's
-// bit for bit (but for the sign of the zeros it stores off the mask, as
-// between that kernel's tile heights).  A staged pair serves 8 or 16 rows
-// instead of 32, so a full GPU is better off with the other kernel.
+// Backprojection of the smallest launches, with the reference's positions.  A
+// tile of the kernel above walks its angles serially, so its time grows with
+// T even where most CUs are idle (a 257^2 slice is 85 workgroups of 64 x 16).
+// Here a workgroup of 8 waves takes a 64 x 8 tile and every wave another
+// block of 32 angles: each stages its own window in its own part of LDS
+// (BPS_AB angles at a time, no barrier), and the blocks' sums are then added
+// in block order, so the result is the other kernel's bit for bit (but for
+// the sign of the zeros it stores off the mask, as between that kernel's tile
+// heights).  A staged pair serves 8 rows instead of 16 or more, so a fuller
+// GPU is better off with the other kernel.
 constexpr int BPS_WAVES = 8;  // waves of a workgroup, one angle block each
 constexpr int BPS_AB = 8;     // angles staged at a time, 8 lanes each
-constexpr int BPS_W = 72;     // window of up to 64 x 16 pixels: hypot(63, 15) + 3.01 = 67.8
+constexpr int BPS_ROWS = 8;   // rows of a tile
+constexpr int BPS_W = 72;     // window of 64 x 8 pixels: hypot(63, 7) + 3.01 = 66.4
 
-__device__ __forceinline__ int find_split_task(const BPTask* tasks, int ntasks, int gtile, int per) {
+__device__ __forceinline__ int find_split_task(const BPTask* tasks, int ntasks, int gtile) {
   int lo = 0, hi = ntasks - 1;
   while (lo < hi) {
     int mid = (lo + hi + 1) >> 1;
-    if (tasks[mid].split_begin / per <= gtile) lo = mid; else hi = mid - 1;
+    if (tasks[mid].split_begin <= gtile) lo = mid; else hi = mid - 1;
   }
   return lo;
 }
 
-template <int ROWS>
 __global__ __launch_bounds__(64 * BPS_WAVES) void bp_split_kernel(const BPTask* __restrict__ tasks, int ntasks,
                                                                   int base, int ntiles) {
-  constexpr int W = BPS_W, NST = W / 8, OWN = ROWS / BPS_WAVES;  // OWN: rows whose block sums a wave adds
+  constexpr int ROWS = BPS_ROWS, W = BPS_W, NST = W / 8, OWN = ROWS / BPS_WAVES;  // OWN: rows a wave adds up
   static_assert(AB % BPS_AB == 0 && W % 8 == 0 && ROWS % BPS_WAVES == 0 && ROWS <= BP_SUB, "tile shape");
   static_assert(ROWS * 64 <= 2 * BPS_AB * W, "a wave's block sums fit its pairs' space");
   __shared__ float2 Ps[BPS_WAVES][BPS_AB * W];
   const int l = xcd_remap(blockIdx.x, gridDim.x);
   if (l >= ntiles) return;  // uniform per workgroup
-  const BPTask& tk = tasks[find_split_task(tasks, ntasks, base + l, ROWS / 8)];
+  const BPTask& tk = tasks[find_split_task(tasks, ntasks, base + l)];
   const int N = tk.N, T = tk.T;
   const float m = tk.mid;
-  const int local = base + l - tk.split_begin / (ROWS / 8);
+  const int local = base + l - tk.split_begin;
   const int tx = local % tk.ntx, ty = local / tk.ntx;
   const int x0 = tx * TX, y0 = ty * ROWS;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -406,21 +406,29 @@ __global__ __launch_bounds__(64 * BPS_WAVES) void bp_split_kernel(const BPTask* 
 
 int bp_split_tiles(int N) { return bp_tiles_x(N) * ((N + 15) / 16) * 2; }
 
-// us per launch, MI355X: 64 x 8 and 64 x 16 tiles here | 64 x 32 tiles of
-// bp_kernel, by the launch's 64 x 8 tiles:
-//   180 (257^2 x 180) 17, 22 | 65;      612 (513^2 x 360) 56, 55 | 126;
-//   1300 (769^2 x 600) 133, 129 | 207;  2244 (1025^2 x 720) 244, 218 | 269;
-//   2880 (16 x 257^2 x 180) 73, 68 | 75;  4900 (1537^2 x 900) 613, 520 | 469
-bool bp_use_split(int tiles) { return tiles <= 3200; }
+// us per FBP (host call and ramp included), MI355X: this kernel | 64 x 16 |
+// 64 x 32 tiles of bp_kernel, by the launch's 64 x 8 tiles:
+//   20 (65^2) x 48 21 | 19 | 24, x 100 22 | 26 | 36, x 180 23 | 36 | 53;
+//   68 (129^2) x 64 22 | 21 | 28, x 90 23 | 25 | 34;
+//   170 (257^2) x 60 22 | 21 | 27, x 180 24 | 38 | 54;
+//   594 (513^2) x 360 64 | 66 | 97;      680 (4 x 257^2) x 180 39 | 40 | 56;
+//   1274 (769^2) x 600 148 | 124 | 158;  2720 (16 x 257^2) x 180 82 | 65 | 80
+// and 64 x 16 | 64 x 32 | 64 x 64 tiles of bp_kernel:
+//   2210 (1025^2) x 720 197 | 236 | 250; 4752 (8 x 513^2) x 720 290 | 343 | 382;
+//   4850 (1537^2) x 900 407 | 435 | 433; 6630 (3 x 1025^2) x 720 411 | 416 | 376;
+//   8840 (4 x 1025^2) x 720 454 | 432 | 400; 8514 (2049^2) x 1500 935 | 944 | 955
+bool bp_use_split(int tiles, int T) { return tiles <= 640 && T > 64; }
+int bp_launch_height(int tiles, int ty) { return tiles <= 5200 ? 16 : ty; }
+// us without | with pairs: 4 x 1025^2 x 720 478 | 400; 8 x 2049^2 x 1500 5960 |
+// 5200; 16 x 257^2 x 180 63 | 65.  A slice without a partner is a launch of
+// its own, with a tail of its own: 9 x 513^2 x 720 (5500 tiles) 360 | 397, 3 x
+// 1025^2 (6600) 376 | 463, 9 x 1025^2 (19900) 937 | 931, 3 x 2049^2 (25500)
+// 2421 | 2389, 5 x 2049^2 (42600) 3982 | 3666
+bool bp_use_pairs(int tiles, bool rest) { return !rest || tiles >= 19000; }
 
 void launch_backproject_split(const BPTask* d_tasks, int ntasks, int base, int tiles, hipStream_t s) {
   if (tiles <= 0) return;
-  if (tiles <= 800)
-    hipLaunchKernelGGL(bp_split_kernel<8>, dim3(xcd_grid(tiles)), dim3(64 * BPS_WAVES), 0, s, d_tasks, ntasks, base,
-                       tiles);
-  else
-    hipLaunchKernelGGL(bp_split_kernel<16>, dim3(xcd_grid(tiles / 2)), dim3(64 * BPS_WAVES), 0, s, d_tasks, ntasks,
-                       base / 2, tiles / 2);
+  hipLaunchKernelGGL(bp_split_kernel, dim3(xcd_grid(tiles)), dim3(64 * BPS_WAVES), 0, s, d_tasks, ntasks, base, tiles);
 }
 
 __global__ __launch_bounds__(256) void rowterm_kernel(const float2* __restrict__ sc, int N, int T, float mid,

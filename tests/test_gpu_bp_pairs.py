@@ -3,8 +3,8 @@ of one slice: the same arithmetic in the same order, so the same bits (the
 sign of the zeros off the mask aside).
 
 Launches are of more than 5200 tiles of 64 x 8, past those that smaller tiles
-serve, with odd counts (a slice without a partner), geometries that
-alternate, and angle counts at the edges of the 16 angles staged at a time
+serve (and of more than 19000 where a slice has no partner), with odd counts,
+geometries that alternate, and angle counts at the edges of the 16 angles staged at a time
 and of the 32 summed as a block.
 """
 import numpy as np
@@ -33,14 +33,17 @@ def single(ctx, N, T, k, f):
 
 # (N, T, k): k shifts the angles, so slices of different k are not of one geometry
 CASES = {
-    "128, one block of 16 angles": [(128, 16, 0)] * 165,
-    "65, 17 angles": [(65, 17, 0)] * 263,
-    "257, 33 angles, odd count": [(257, 33, 0)] * 33,
-    "257, two geometries in turn": [(257, 31, i % 2) for i in range(35)],
+    "128, one block of 16 angles": [(128, 16, 0)] * 164,
+    "65, 17 angles": [(65, 17, 0)] * 262,
+    "257, 33 angles": [(257, 33, 0)] * 32,
+    "257, two geometries in turn": [(257, 31, i % 2) for i in range(36)],
     "513, pairs and singles": [(513, 15, 0), (513, 15, 1), (513, 15, 0), (257, 47, 0), (513, 15, 2), (257, 47, 0),
-                               (513, 48, 0), (513, 48, 3), (513, 48, 0), (1025, 9, 0)],
+                               (513, 48, 0), (513, 48, 3), (513, 48, 0), (2049, 9, 0), (2049, 9, 0), (2049, 1, 0)],
     "1025, 1 angle": [(1025, 1, 0)] * 4,
-    "1026, 65 angles": [(1026, 65, 0)] * 3,
+    "1026, 65 angles, odd count": [(1026, 65, 0)] * 9,
+    "1025, too few tiles for an odd count": [(1025, 33, 0)] * 3,
+    "257, few tiles": [(257, 33, 0)] * 5,
+    "257, more than 64 angles, few tiles": [(257, 66, 0)] * 3,
 }
 
 
