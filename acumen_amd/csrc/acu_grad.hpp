@@ -13,6 +13,13 @@ namespace acu {
 
 constexpr int ADJ_T = 16;          // pixel tile side of the adjoint (16 x 16 threads)
 constexpr int ADJ_AB = 32;         // angles per FP32 block sum
+constexpr int ADJ_GROUP = 8;       // most slices of one geometry a workgroup takes together
+// The most in a launch over slices of that many tiles in all: at 8 a launch of
+// few workgroups is one long chain in each.  us by 1 | 2 | 4 | 8 slices
+// together: 16 x 65^2 x 48 (400 tiles) 40 | 38 | 39 | 47, 16 x 129^2 x 90 (1296)
+// 126 | 85 | 76 | 85, 8 x 257^2 x 180 (2312) 345 | 221 | 169 | 175, 16 x 257^2
+// 600 | 363 | 243 | 210, 8 x 513^2 x 360 (8712) 1958 | 1132 | 704 | 570
+inline int adj_group(int tiles) { return tiles < 2048 ? ADJ_GROUP / 2 : ADJ_GROUP; }
 constexpr int GR_THREADS = 256;
 
 // Exact transpose of radon: img(px,py) = (1/N) sum over angles and samples
@@ -23,9 +30,10 @@ struct AdjTask {
   float mid;
   int block_begin;   // first global block of this slice
   int ntx;           // tiles per side: ceil(N / ADJ_T)
-  const float* sino; // (T, N)
+  int n;             // slices of the task, of one geometry (N, T, angles): at most the launch's group
   const float2* sc;  // (sin, cos) of the projector angles
-  float* out;        // (N, N)
+  const float* sino[ADJ_GROUP];  // (T, N); entries past n are read as well: any of the first n
+  float* out[ADJ_GROUP];         // (N, N); entries past n are not written
 };
 
 // One angle row per workgroup: r = shift_s(y) - b, rs = shift_s^T(r),
@@ -66,7 +74,8 @@ struct LossTask {
 inline int adj_tiles(int N) { return (N + ADJ_T - 1) / ADJ_T; }
 inline int tvg_blocks(int N) { return (int)(((size_t)N * N + GR_THREADS - 1) / GR_THREADS); }
 
-void launch_adjoint(const AdjTask* d_tasks, int ntasks, int base, int blocks, hipStream_t s);
+// group: 1, 2, 4 or 8, the slices a workgroup takes together (n of each task at most)
+void launch_adjoint(const AdjTask* d_tasks, int ntasks, int group, int blocks, hipStream_t s);
 void launch_shift_resid(const ResTask* d_tasks, int ntasks, int base, int rows, hipStream_t s);
 void launch_tvgrad(const TVGTask* d_tasks, int ntasks, int base, int blocks, hipStream_t s);
 void launch_loss_finalize(const LossTask* d_tasks, int ntasks, hipStream_t s);

@@ -273,7 +273,8 @@ struct acu_batch {
   int bp_ty = acu::BP_TY_DEFAULT;     // backprojection tile height (16, 32 or 64) as set
   int bp_h = acu::BP_TY_DEFAULT;      // the height its launches have (bp_launch_height)
   acu::BPShares bp_sh_all{};          // XCD shares of the backprojection over all slices
-  // slices of one geometry (N, T, wpu, angles) in pairs: each slice's partner
+  std::vector<int> geo;               // each slice's geometry (find_geometries)
+  // slices of one geometry and window in pairs: each slice's partner
   // or -1 (find_pairs), and the XCD shares of the two parts of a launch
   std::vector<int> bp_partner;
   bool bp_pairs = false;              // whether launches over all slices take them (bp_use_pairs)
@@ -616,22 +617,34 @@ void bp_tile_work(const Slice& s, int ty, std::vector<float>& w) {
     }
 }
 
-// Pairs of slices with one geometry, in slice order.
-std::vector<int> find_pairs(const acu_batch* b) {
-  std::vector<int> partner(b->s.size(), -1);
-  std::map<std::tuple<int, int, int, uint64_t>, int> open;  // a slice that waits for a partner
+// Each slice's geometry: the first slice of its (N, T, angles).
+std::vector<int> find_geometries(const acu_batch* b) {
+  std::vector<int> geo(b->s.size());
+  std::map<std::tuple<int, int, uint64_t>, int> first;
   for (int i = 0; i < (int)b->s.size(); ++i) {
     const Slice& s = b->s[i];
+    geo[i] = i;
     if (!s.theta_set) continue;
-    const auto key = std::make_tuple(s.N, s.T, s.wpu, theta_hash(s.theta));
+    const int j = first.emplace(std::make_tuple(s.N, s.T, theta_hash(s.theta)), i).first->second;
+    if (std::memcmp(b->s[j].theta.data(), s.theta.data(), sizeof(float) * s.T) == 0) geo[i] = j;
+  }
+  return geo;
+}
+
+// Pairs of slices with one geometry and window, in slice order.
+std::vector<int> find_pairs(const acu_batch* b) {
+  std::vector<int> partner(b->s.size(), -1);
+  std::map<std::pair<int, int>, int> open;  // a slice that waits for a partner
+  for (int i = 0; i < (int)b->s.size(); ++i) {
+    const auto key = std::make_pair(b->geo[i], b->s[i].wpu);
     const auto it = open.find(key);
     if (it == open.end()) {
       open.emplace(key, i);
-    } else if (std::memcmp(b->s[it->second].theta.data(), s.theta.data(), sizeof(float) * s.T) == 0) {
-      partner[i] = it->second;
-      partner[it->second] = i;
-      open.erase(it);
+      continue;
     }
+    partner[i] = it->second;
+    partner[it->second] = i;
+    open.erase(it);
   }
   return partner;
 }
@@ -679,6 +692,7 @@ void build_bpset(acu_batch* b, BPSet& set, InF in, OutF out) {
 // Pairs, and the XCD shares of the all-slice and per-slice backprojection
 // launches.
 void assign_bp_shares(acu_batch* b) {
+  b->geo = find_geometries(b);
   b->bp_partner = find_pairs(b);
   const auto none = [](Slice&) { return (float*)nullptr; };
   const BPParts p = bp_parts(b, (int)b->s.size(), b->bp_h, true, none, none);
@@ -1397,7 +1411,33 @@ std::string autotune(acu_batch* b, int reps, unsigned what = TUNE_ALL) {
 // ---- differentiation: exact adjoint and the gradients of
 // L(x, s) = 1/2 |shift_s(radon(x)) - b|^2 + lambda TV_eps(x), b = the slice's f ----
 AdjTask adj_task(const Slice& s, int block_begin, const float* sino, float* out) {
-  return AdjTask{s.N, s.T, s.mid, block_begin, adj_tiles(s.N), sino, s.scfp, out};
+  AdjTask t{s.N, s.T, s.mid, block_begin, adj_tiles(s.N), 1, s.scfp, {}, {}};
+  for (auto& p : t.sino) p = sino;
+  t.out[0] = out;
+  return t;
+}
+
+// Adjoint tasks of all slices, sino(i) -> out(i), slices of one geometry up to
+// ADJ_GROUP to a task (half of it in small launches); their blocks in total.
+template <class InF, class OutF>
+int adj_tasks(const acu_batch* b, std::vector<AdjTask>& t, InF in, OutF out) {
+  std::map<int, int> open;  // geometry -> its last task
+  int blocks = 0, tiles = 0;
+  for (const auto& s : b->s) tiles += adj_tiles(s.N) * adj_tiles(s.N);
+  const int group = adj_group(tiles);
+  for (int i = 0; i < (int)b->s.size(); ++i) {
+    const auto it = open.find(b->geo[i]);
+    if (it != open.end() && t[it->second].n < group) {
+      AdjTask& a = t[it->second];
+      a.sino[a.n] = in(i);
+      a.out[a.n++] = out(i);
+      continue;
+    }
+    open[b->geo[i]] = (int)t.size();
+    t.push_back(adj_task(b->s[i], blocks, in(i), out(i)));
+    blocks += adj_tiles(b->s[i].N) * adj_tiles(b->s[i].N);
+  }
+  return blocks;
 }
 
 void radon_adjoint_dev(acu_batch* b, int sl, float* img, const float* sino) {
@@ -1405,7 +1445,7 @@ void radon_adjoint_dev(acu_batch* b, int sl, float* img, const float* sino) {
   acu_ctx* c = b->ctx;
   AdjTask* d = put_adhoc(b, adj_task(s, 0, sino, img));
   const int nb = adj_tiles(s.N) * adj_tiles(s.N);
-  timed(c, K_ADJ, [&] { launch_adjoint(d, 1, 0, nb, c->stream); });
+  timed(c, K_ADJ, [&] { launch_adjoint(d, 1, 1, nb, c->stream); });
   check_launch();
 }
 
@@ -1460,8 +1500,7 @@ void loss_grad_run(acu_batch* b, const std::vector<const float*>& x, const std::
   std::vector<ResTask> res(n);
   std::vector<TVGTask> tvg(n);
   std::vector<LossTask> lt(n);
-  std::vector<AdjTask> adj;
-  int rows = 0, tvb = 0, adjb = 0;
+  int rows = 0, tvb = 0;
   for (int i = 0; i < n; ++i) {
     Slice& s = b->s[i];
     res[i] = ResTask{s.N, s.T, rows, s.gx_y, s.f, shift[i], s.gx_rs, gs[i], hs[i], s.gx_pd};
@@ -1470,19 +1509,20 @@ void loss_grad_run(acu_batch* b, const std::vector<const float*>& x, const std::
     tvg[i] = TVGTask{s.N, tvb, nb, lambda, eps, x[i], gx.empty() ? nullptr : gx[i], s.gx_pt};
     tvb += nb;
     lt[i] = LossTask{s.T, nb, (double)lambda, s.gx_pd, s.gx_pt, s.gx_loss};
-    if (!gx.empty()) {
-      adj.push_back(adj_task(s, adjb, s.gx_rs, gx[i]));
-      adjb += adj_tiles(s.N) * adj_tiles(s.N);
-    }
   }
   b->res_g.upload(res, b->ctx->stream);
   b->tvg_g.upload(tvg, b->ctx->stream);
   b->loss_g.upload(lt, b->ctx->stream);
   launch_shift_resid(b->res_g.d, n, 0, rows, c->stream);
   check_launch();
-  if (!adj.empty()) {
+  if (!gx.empty()) {
+    std::vector<AdjTask> adj;
+    const int blocks = adj_tasks(b, adj, [&](int i) { return b->s[i].gx_rs; }, [&](int i) { return gx[i]; });
+    int group = 1;
+    for (const auto& t : adj)
+      while (group < t.n) group *= 2;
     b->adj_g.upload(adj, b->ctx->stream);
-    timed(c, K_ADJ, [&] { launch_adjoint(b->adj_g.d, n, 0, adjb, c->stream); });
+    timed(c, K_ADJ, [&] { launch_adjoint(b->adj_g.d, b->adj_g.n, group, blocks, c->stream); });
     check_launch();
   }
   launch_tvgrad(b->tvg_g.d, n, 0, tvb, c->stream);

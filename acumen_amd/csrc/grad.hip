@@ -28,10 +28,12 @@
 // values of a tile (a window of 32 rays per angle, zero off the detector) are
 // staged in LDS for 32 angles at a time.
 //
-// Bound by VALU issue (about 115 instructions per pixel and angle, 90 of them
-// the candidates).  On MI355X 6.7 ms per 16 x 513^2 x 720 launch (9.7 with
-// comparisons per candidate and three global loads per angle), 130 us at
-// 257^2 x 180 (344).
+// Bound by VALU issue: about 115 instructions per pixel and angle, 90 of them
+// the candidates' weights.  Those depend on the geometry alone, so a workgroup
+// takes up to 8 slices of one geometry together (G, side by side in LDS): 3
+// products and a sum more per slice.  On MI355X, 16 x 513^2 x 720: 6.7 ms by
+// single slices (9.7 with comparisons per candidate and three global loads
+// per angle), 2.2 by fours, 1.75 by eights; one 257^2 x 180 130 us (344).
 #include "acu_grad.hpp"
 
 namespace acu {
@@ -75,16 +77,21 @@ constexpr int ADJ_W = 32;  // rays staged per angle and tile: 15 (|c| + |s|) + 4
 struct AdjPixel {
   float X, Y, px, py, xlo, xhi, ylo, yhi, u0, u1;
 };
-template <bool CHECK>
-__device__ __forceinline__ float adj_angle(const AdjPixel& g, float s, float c, float hw, float m, float w,
-                                           const float* P) {
+// one ray of each of G slices, side by side in LDS
+template <int G>
+struct __attribute__((aligned(G < 4 ? 4 * G : 16))) AdjRay {
+  float v[G];
+};
+template <bool CHECK, int G>
+__device__ __forceinline__ void adj_angle(const AdjPixel& g, float s, float c, float hw, float m, float w,
+                                          const float* P, float (&blk)[G]) {
 #pragma clang fp contract(off)
   // first candidate, relative to the midpoint (integer valued): the margin in
   // hw covers the rounding of this estimate and of the exact positions
   const float ua = ceilf(fmaf(c, g.X, fmaf(s, g.Y, -hw)));
   const float wa = ceilf(fmaf(c, g.Y, fmaf(-s, g.X, -hw)));
-  const float* r = (const float*)((const char*)P + __float_as_uint(fmaf(wa, lds_units(4), w)));
-  const float rv[3] = {r[0], r[1], r[2]};
+  const AdjRay<G>* r = (const AdjRay<G>*)((const char*)P + __float_as_uint(fmaf(wa, lds_units(4 * G), w)));
+  const AdjRay<G> rv[3] = {r[0], r[1], r[2]};
   float cu[3], su[3];
   bool uok[3];
 #pragma unroll
@@ -94,7 +101,9 @@ __device__ __forceinline__ float adj_angle(const AdjPixel& g, float s, float c, 
     su[a] = s * u;
     uok[a] = !CHECK || (u >= g.u0 && u <= g.u1);
   }
-  float v = 0.0f;
+  float v[G];
+#pragma unroll
+  for (int k = 0; k < G; ++k) v[k] = 0.0f;
 #pragma unroll
   for (int b = 0; b < 3; ++b) {
     const float wb = b == 0 ? wa : wa + (float)b;
@@ -110,15 +119,20 @@ __device__ __forceinline__ float adj_angle(const AdjPixel& g, float s, float c, 
       sum = a == 0 ? wx * wy : fmaf(wx, wy, sum);
     }
     // CHECK: a ray of infinity or NaN stays out of the pixels it does not cover
-    if (!CHECK) v = b == 0 ? rv[b] * sum : fmaf(rv[b], sum, v);
-    else v = sum > 0.0f ? fmaf(rv[b], sum, v) : v;
+#pragma unroll
+    for (int k = 0; k < G; ++k) {
+      if (!CHECK) v[k] = b == 0 ? rv[b].v[k] * sum : fmaf(rv[b].v[k], sum, v[k]);
+      else v[k] = sum > 0.0f ? fmaf(rv[b].v[k], sum, v[k]) : v[k];
+    }
   }
-  return v;
+#pragma unroll
+  for (int k = 0; k < G; ++k) blk[k] += v[k];
 }
 
+template <int G>
 __global__ __launch_bounds__(ADJ_T * ADJ_T) void adjoint_kernel(const AdjTask* __restrict__ tasks, int ntasks,
                                                                 int base, int nblocks) {
-  __shared__ float P[ADJ_AB * ADJ_W];
+  __shared__ AdjRay<G> P[ADJ_AB * ADJ_W];
   const int lbk = xcd_remap(blockIdx.x, gridDim.x);
   if (lbk >= nblocks) return;  // uniform per workgroup
   const int gb = base + lbk;
@@ -146,9 +160,10 @@ __global__ __launch_bounds__(ADJ_T * ADJ_T) void adjoint_kernel(const AdjTask* _
   const float X0 = (float)(tx * ADJ_T + 1) - m, X1 = X0 + (float)(ADJ_T - 1);
   const float Y0 = (float)(ty * ADJ_T + 1) - m, Y1 = Y0 + (float)(ADJ_T - 1);
   const float margin = 1e-3f + 3e-7f * (float)N;
-  const ACU_GLOBAL float* __restrict__ sino = as_global(tk.sino);
   const ACU_GLOBAL float* __restrict__ sc = as_global((const float*)tk.sc);
-  float acc = 0.0f;
+  float acc[G];
+#pragma unroll
+  for (int k = 0; k < G; ++k) acc[k] = 0.0f;
   for (int t0 = 0; t0 < T; t0 += ADJ_AB) {
     const int na = min(ADJ_AB, T - t0);
     // lane l (mod 32) of every wave holds angle t0 + l: sine, cosine, first
@@ -160,36 +175,51 @@ __global__ __launch_bounds__(ADJ_T * ADJ_T) void adjoint_kernel(const AdjTask* _
     const float xmin = fminf(hc * X0, hc * X1) + fminf(hs * Y0, hs * Y1);
     const float xmax = fmaxf(hc * X0, hc * X1) + fmaxf(hs * Y0, hs * Y1);
     const int lo = (int)floorf((ymin - hh) + m) - 1;
-    const float hb = lds_base(4 * ((lane & (ADJ_AB - 1)) * ADJ_W + (int)m - lo));  // LDS offset of ray jy = m
+    const float hb = lds_base(4 * G * ((lane & (ADJ_AB - 1)) * ADJ_W + (int)m - lo));  // LDS offset of ray jy = m
     unsigned long long chk = rim ? ~0ull : __ballot(xmin - hh < g.u0 + 1.0f || xmax + hh > g.u1 - 1.0f);
     bool bad = false;
     {
       const int q = tid >> 3, j = tid & 7;  // 8 threads per angle
       const int jy0 = __shfl(lo, q) + j;
-      const ACU_GLOBAL float* row = sino + (size_t)min(t0 + q, T - 1) * N;
-      float v[ADJ_W / 8];
+      AdjRay<G> v[ADJ_W / 8];
 #pragma unroll
-      for (int k = 0; k < ADJ_W / 8; ++k) v[k] = row[min(max(jy0 + 8 * k, 1), N) - 1];
+      for (int i = 0; i < G; ++i) {
+        const ACU_GLOBAL float* row = as_global(tk.sino[i]) + (size_t)min(t0 + q, T - 1) * N;
+#pragma unroll
+        for (int k = 0; k < ADJ_W / 8; ++k) v[k].v[i] = row[min(max(jy0 + 8 * k, 1), N) - 1];
+      }
       if (t0 > 0) __syncthreads();  // the last block's rays are read
 #pragma unroll
       for (int k = 0; k < ADJ_W / 8; ++k) {
-        P[q * ADJ_W + j + 8 * k] = jy0 + 8 * k >= 1 && jy0 + 8 * k <= N ? v[k] : 0.0f;
-        bad = bad || !(fabsf(v[k]) <= 3.40282347e38f);
+        const bool on = jy0 + 8 * k >= 1 && jy0 + 8 * k <= N;
+        AdjRay<G> u;
+#pragma unroll
+        for (int i = 0; i < G; ++i) {
+          u.v[i] = on ? v[k].v[i] : 0.0f;
+          bad = bad || !(fabsf(v[k].v[i]) <= 3.40282347e38f);
+        }
+        P[q * ADJ_W + j + 8 * k] = u;
       }
     }
     if (__syncthreads_or(bad)) chk = ~0ull;  // uniform
-    float blk = 0.0f;  // FP32 sum over one block of angles, then into acc
+    float blk[G];  // FP32 sums over one block of angles, then into acc
+#pragma unroll
+    for (int k = 0; k < G; ++k) blk[k] = 0.0f;
     for (int a = 0; a < na; ++a) {
       const float s = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(hs), a));
       const float c = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(hc), a));
       const float hw = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(hh), a));
       const float w = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(hb), a));
-      if ((chk >> a) & 1) blk += adj_angle<true>(g, s, c, hw, m, w, P);
-      else blk += adj_angle<false>(g, s, c, hw, m, w, P);
+      if ((chk >> a) & 1) adj_angle<true, G>(g, s, c, hw, m, w, &P[0].v[0], blk);
+      else adj_angle<false, G>(g, s, c, hw, m, w, &P[0].v[0], blk);
     }
-    acc += blk;
+#pragma unroll
+    for (int k = 0; k < G; ++k) acc[k] += blk[k];
   }
-  if (px <= N && py <= N) tk.out[(size_t)(py - 1) * N + (px - 1)] = acc / (float)N;
+  if (px <= N && py <= N)
+#pragma unroll
+    for (int k = 0; k < G; ++k)
+      if (k < tk.n) tk.out[k][(size_t)(py - 1) * N + (px - 1)] = acc[k] / (float)N;
 }
 
 __device__ __forceinline__ float at(const ACU_GLOBAL float* row, int N, int i) {
@@ -301,10 +331,16 @@ __global__ __launch_bounds__(GR_THREADS) void loss_finalize_kernel(const LossTas
 
 }  // namespace
 
-void launch_adjoint(const AdjTask* d_tasks, int ntasks, int base, int blocks, hipStream_t s) {
+void launch_adjoint(const AdjTask* d_tasks, int ntasks, int group, int blocks, hipStream_t s) {
   if (blocks <= 0) return;
-  hipLaunchKernelGGL(adjoint_kernel, dim3(xcd_grid(blocks)), dim3(ADJ_T * ADJ_T), 0, s, d_tasks, ntasks, base,
-                     blocks);
+  const dim3 grid(xcd_grid(blocks)), wg(ADJ_T * ADJ_T);
+  switch (group) {
+    case 1: hipLaunchKernelGGL(adjoint_kernel<1>, grid, wg, 0, s, d_tasks, ntasks, 0, blocks); break;
+    case 2: hipLaunchKernelGGL(adjoint_kernel<2>, grid, wg, 0, s, d_tasks, ntasks, 0, blocks); break;
+    case 4: hipLaunchKernelGGL(adjoint_kernel<4>, grid, wg, 0, s, d_tasks, ntasks, 0, blocks); break;
+    case 8: hipLaunchKernelGGL(adjoint_kernel<8>, grid, wg, 0, s, d_tasks, ntasks, 0, blocks); break;
+    default: throw Error("the adjoint takes 1, 2, 4 or 8 slices together");
+  }
 }
 
 void launch_shift_resid(const ResTask* d_tasks, int ntasks, int base, int rows, hipStream_t s) {
