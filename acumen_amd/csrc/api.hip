@@ -718,7 +718,8 @@ void assign_bp(acu_batch* b) {
     s.bps_begin = bps; s.bps_n = bp_split_tiles(s.N); bps += s.bps_n;
     b->maxT = std::max(b->maxT, s.T);
   }
-  b->bp_h = bp_launch_height(bps, b->bp_ty);
+  // tile-relative positions round by the tile's height: the height is as set
+  b->bp_h = b->bp_refpos && b->tv_bp_refpos ? bp_launch_height(bps, b->bp_ty) : b->bp_ty;
   for (auto& s : b->s) {
     s.nty = bp_tiles_y(s.N, b->bp_h);
     s.bp_begin = bp; s.bp_n = s.ntx * s.nty; bp += s.bp_n;
@@ -1839,7 +1840,7 @@ int acu_batch_set_bp_positions(acu_batch* b, int fbp, int tv) {
   if (!ok(fbp) || !ok(tv)) return fail(ACU_ERR_ARG, "acu_batch_set_bp_positions: unknown positions");
   // the TV task table points at s.fbp or s.ftv: tvopt rebuilds it
   ACU_TRY(hipSetDevice(b->ctx->device); b->ctx->sync(); b->bp_refpos = fbp == ACU_BP_POS_REFERENCE;
-          b->tv_bp_refpos = tv == ACU_BP_POS_REFERENCE; b->tv.release(); b->drop_graphs();
+          b->tv_bp_refpos = tv == ACU_BP_POS_REFERENCE; b->tv.release(); acu::set_bp_tile(b, b->bp_ty);
           for (auto& s : b->s) { s.fbp_valid = false; s.tv_valid = false; });
 }
 

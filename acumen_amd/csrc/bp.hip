@@ -459,21 +459,21 @@ void launch_bp(const BPTask* d_tasks, int ntasks, int base, int ty, const BPShar
   }
 }
 
-void check_bp_launch(int tiles, const BPShares& sh) {
-  if (sh.b[0] != 0 || sh.b[XCDS] != tiles || sh.C < 1) throw Error("backprojection shares do not match the launch");
+void check_bp_launch(const BPTask* d_tasks, int ntasks, int tiles, const BPShares& sh) {
+  if (!d_tasks || ntasks < 1 || sh.b[0] != 0 || sh.b[XCDS] != tiles || sh.C < 1) throw Error("backprojection tasks or shares do not match the launch");
 }
 
 void launch_backproject(const BPTask* d_tasks, int ntasks, int base, int tiles, int ty, bool refpos,
                         const BPShares& sh, hipStream_t s) {
   if (tiles <= 0) return;
-  check_bp_launch(tiles, sh);
+  check_bp_launch(d_tasks, ntasks, tiles, sh);
   if (refpos) launch_bp<true, 1>(d_tasks, ntasks, base, ty, sh, s);
   else launch_bp<false, 1>(d_tasks, ntasks, base, ty, sh, s);
 }
 
 void launch_backproject_pairs(const BPTask* d_tasks, int ntasks, int tiles, int ty, const BPShares& sh, hipStream_t s) {
   if (tiles <= 0) return;
-  check_bp_launch(tiles, sh);
+  check_bp_launch(d_tasks, ntasks, tiles, sh);
   launch_bp<true, 2>(d_tasks, ntasks, 0, ty, sh, s);
 }
 

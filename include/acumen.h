@@ -222,8 +222,10 @@ int acu_batch_set_fp_variant(acu_batch *b, int slice, int variant);
  * The angle blocks (32 angles, each block summed separately) are the same
  * at every height; with the reference's positions the heights give the
  * same FP32 result, with tile-relative positions they differ by FP32
- * rounding only.  The initial value comes from ACUMEN_BP_TILE.  The getter
- * returns the rows or -ACU_ERR_ARG. */
+ * rounding only.  With the reference's positions, batches of few tiles (up
+ * to about one 1537^2 slice) run at 16 rows or fewer whatever is set, for
+ * more workgroups (the same bits).  The initial value comes from
+ * ACUMEN_BP_TILE.  The getter returns the rows set or -ACU_ERR_ARG. */
 int acu_batch_set_bp_tile(acu_batch *b, int rows);
 int acu_batch_bp_tile(const acu_batch *b);
 
@@ -232,7 +234,7 @@ int acu_batch_bp_tile(const acu_batch *b);
  * rounded once in FP32, so every floor, weight and mask decision is the
  * reference's; ACU_BP_POS_TILE forms it relative to the tile origin with
  * one FMA per update (rounded at magnitude < 140 instead of N: closer to
- * FP64, about 25% faster).  fbp: the positions of FBP images, acu_iradon*
+ * FP64).  fbp: the positions of FBP images, acu_iradon*
  * and acu_backproject_dev (from ACUMEN_BP_POSITIONS = reference | tile);
  * tv: those of the backprojections inside tvopt's iteration, whose warm
  * start is the FBP image (from ACUMEN_TV_BP_POSITIONS).  Both default to

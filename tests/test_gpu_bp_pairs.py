@@ -10,7 +10,7 @@ and of the 32 summed as a block.
 import numpy as np
 import pytest
 
-from acumen_amd import ACU_IMG_FBP, ACU_IMG_TV, ACU_TV_GRAPH, Batch, synth
+from acumen_amd import ACU_IMG_FBP, ACU_IMG_TV, ACU_TV_GRAPH, Batch, _lib, synth
 
 pytestmark = pytest.mark.gpu
 
@@ -83,3 +83,22 @@ def test_new_angles_part_a_pair(ctx):
                     p.tvopt(0.05, 0.1, 2, 1, 2, ACU_TV_GRAPH)
                     assert np.array_equal(b.get_image(i, ACU_IMG_FBP), p.get_image(0, ACU_IMG_FBP)), (k, i)
                     assert np.array_equal(b.get_image(i, ACU_IMG_TV), p.get_image(0, ACU_IMG_TV)), (k, i)
+
+
+def test_tile_positions_keep_the_set_height(ctx):
+    """Tile-relative positions round by the tile's height, so a small batch
+    and a large one of the same slice agree at the height that is set."""
+    N, T = 129, 40
+    f = sinos([(N, T, 0)])[0]
+    big = (1537, 1, synth.default_wpu(1537), synth.angles(1))
+    print("[case] bp tile positions", flush=True)
+    for ty in (16, 32):
+        out = []
+        for extra in ([], [big] * 2):
+            with Batch(ctx, [(N, T, synth.default_wpu(N), synth.angles(T))] + extra) as b:
+                b.set_bp_positions(_lib.ACU_BP_POS_TILE, _lib.ACU_BP_POS_TILE)
+                b.set_bp_tile(ty)
+                b.set_sino(0, f)
+                b.fbp()
+                out.append(b.get_image(0, ACU_IMG_FBP))
+        assert np.array_equal(out[0], out[1])
