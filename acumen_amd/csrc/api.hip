@@ -173,6 +173,7 @@ struct Slice {
   float mid = 0.f;
   std::vector<float> theta;
   bool theta_set = false;
+  uint64_t theta_key = 0;  // theta_hash of the angles the tables are of
   int ntx = 0, nty = 0, nsub = 0;  // backprojection tiles along x, y; 16-row sub-tiles along y
   std::vector<uint8_t> tact_h;     // host copy of the sub-tile activity (tact)
   BPShares bp_sh{};                // XCD shares of this slice's own backprojection launch
@@ -277,6 +278,7 @@ struct acu_batch {
   // slices of one geometry and window in pairs: each slice's partner
   // or -1 (find_pairs), and the XCD shares of the two parts of a launch
   std::vector<int> bp_partner;
+  bool bp_built = true;               // false: a change of angles failed before the tasks were rebuilt
   bool bp_pairs = false;              // whether launches over all slices take them (bp_use_pairs)
   int maxT = 0;                       // most angles of a slice
   acu::BPShares bp_sh_pair{}, bp_sh_rest{};
@@ -475,6 +477,7 @@ void upload_theta(acu_batch* b, int i) {
   launch_bp_rowterm(s.scbp, s.N, s.T, s.mid, s.rowterm, st);
   ACU_HIP_CHECK(hipGetLastError());
   ACU_HIP_CHECK(hipStreamSynchronize(st));  // bp and fp end here
+  s.theta_key = theta_hash(s.theta);
   s.theta_set = true;
 }
 
@@ -625,7 +628,7 @@ std::vector<int> find_geometries(const acu_batch* b) {
     const Slice& s = b->s[i];
     geo[i] = i;
     if (!s.theta_set) continue;
-    const int j = first.emplace(std::make_tuple(s.N, s.T, theta_hash(s.theta)), i).first->second;
+    const int j = first.emplace(std::make_tuple(s.N, s.T, s.theta_key), i).first->second;
     if (std::memcmp(b->s[j].theta.data(), s.theta.data(), sizeof(float) * s.T) == 0) geo[i] = j;
   }
   return geo;
@@ -1756,10 +1759,17 @@ int acu_batch_set_theta(acu_batch* b, int slice, const float* theta_deg) {
   ACU_TRY(hipSetDevice(b->ctx->device); b->ctx->sync();
           std::memcpy(b->s[slice].theta.data(), theta_deg, sizeof(float) * b->s[slice].T);
           acu::upload_theta(b, slice);
-          // whether the cells pass is launched depends on the angles
-          // and so does which slices the backprojection takes together
+          // whether the cells pass is launched depends on the angles, and so
+          // does which slices the backprojection takes together
           try {
-            if (b->s.size() > 1) acu::assign_bp_shares(b), acu::build_op_tasks(b);
+            if (b->s.size() > 1) {
+              const auto partner = b->bp_partner;
+              const bool pairs = b->bp_pairs, built = b->bp_built;
+              b->bp_built = false;
+              acu::assign_bp_shares(b);
+              if (!built || partner != b->bp_partner || pairs != b->bp_pairs) acu::build_op_tasks(b);
+              b->bp_built = true;
+            }
             acu::refresh_fp(b);
           } catch (...) { b->s[slice].theta_set = false; throw; });
 }
