@@ -214,15 +214,16 @@ struct Slice {
   double2* fftW = nullptr;
   int ff_begin = 0, ff_n = 0;
   float ff_edge = 0.0f;    // FFT ramp: the tap at distance N-1 (h(2N-1), 0-based)
-  int rf_begin = 0, rf_n = 0, bp_begin = 0, bp_n = 0, bps_begin = 0, bps_n = 0, cl_begin = 0, cl_n = 0,
+  int rf_begin = 0, rf_n = 0, rfp_begin = 0, bp_begin = 0, bp_n = 0, bps_begin = 0, bps_n = 0, cl_begin = 0, cl_n = 0,
       fp_begin = 0, fp_n = 0, fs_begin = 0, fs_n = 0, fl_begin = 0, fl_n = 0, ew_begin = 0, ew_n = 0, sw_begin = 0, sw_n = 0;
 };
 
-// Ramp-filter task arrays of one operand pair: the Toeplitz GEMM and the FFT form.
+// Ramp-filter task arrays of one operand pair: the Toeplitz GEMM, the FFT form,
+// and the GEMM for the slices past the FFT's limit alone.
 struct RFSet {
-  DevArray<RFTask> rf;
+  DevArray<RFTask> rf, past;
   DevArray<FFTTask> ff;
-  void release() { rf.release(); ff.release(); }
+  void release() { rf.release(); past.release(); ff.release(); }
 };
 
 // Backprojection tasks of one operand pair: of every slice, and, where slices
@@ -262,7 +263,7 @@ struct acu_batch {
   void* tv_mem = nullptr;
   int tv_delta_cap = 0;
   int ff_total = 0, ff_threads = 64;  // FFT ramp blocks (slices within its limit) and threads per workgroup
-  int rf_total = 0, bp_total = 0, bps_total = 0, cl_total = 0, fp_total = 0, fs_total = 0, ew_total = 0,
+  int rf_total = 0, rfp_total = 0, bp_total = 0, bps_total = 0, cl_total = 0, fp_total = 0, fs_total = 0, ew_total = 0,
       sw_total = 0;
   int fl_total[acu::FL_GROUPS] = {0, 0, 0, 0};  // LDS projector blocks per variant group (lds1, lds2, lds4, cell16)
   // dispatch orders of the LDS projector (fpl_dispatch_order) per variant
@@ -586,13 +587,19 @@ void build_tv_tasks(acu_batch* b);
 
 template <class InF, class OutF>
 void build_rfset(acu_batch* b, RFSet& set, InF in, OutF out) {
-  std::vector<RFTask> rf;
+  std::vector<RFTask> rf, past;
   std::vector<FFTTask> ff;
   for (auto& s : b->s) {
     rf.push_back(rf_task(s, in(s), out(s)));
-    if (s.fftG) ff.push_back(ff_task(s, in(s), out(s)));
+    if (s.fftG) {
+      ff.push_back(ff_task(s, in(s), out(s)));
+    } else {
+      past.push_back(rf.back());
+      past.back().tile_begin = s.rfp_begin;
+    }
   }
   set.rf.upload(rf, b->ctx->stream);
+  set.past.upload(past, b->ctx->stream);
   set.ff.upload(ff, b->ctx->stream);
 }
 
@@ -816,15 +823,17 @@ Range sw_range(acu_batch* b, int sl) { return sl < 0 ? Range{0, b->sw_total} : R
 // points fit LDS twice over) and by the Toeplitz product on the FP64 matrix
 // cores beyond.  The FFT is faster at every size within it: ms by FFT and as
 // a product, 0.008 and 0.033 at 257^2 x 180, 0.032 and 0.27 at 2049^2 x 1500.
+// The slices beyond share a launch: 8 x 4500^2 x 60 are 71 workgroups each
+// for 256 CUs, and FBP of them takes 1.66 ms so, 6.1 with a launch for each.
 void launch_ramp_any(acu_batch* b, const RFSet& rf, int sl, int variant) {
   hipStream_t st = b->ctx->stream;
   const bool all = sl < 0;
   if (variant == RAMP_FFT || variant == RAMP_FP64) {
     launch_ramp_fft(rf.ff.d, rf.ff.n, all ? 0 : b->s[sl].ff_begin, all ? b->ff_total : b->s[sl].ff_n, b->ff_threads,
                     st);
-    if (variant == RAMP_FP64)
-      for (int i = all ? 0 : sl; i < (all ? (int)b->s.size() : sl + 1); ++i)
-        if (!b->s[i].fftG) launch_ramp(rf.rf.d, rf.rf.n, b->s[i].rf_begin, b->s[i].rf_n, variant, st);
+    if (variant == RAMP_FP64 && all) launch_ramp(rf.past.d, rf.past.n, 0, b->rfp_total, variant, st);
+    else if (variant == RAMP_FP64 && !b->s[sl].fftG)
+      launch_ramp(rf.past.d, rf.past.n, b->s[sl].rfp_begin, b->s[sl].rf_n, variant, st);
     return;
   }
   const Range r = rf_range(b, sl);
@@ -1688,6 +1697,8 @@ int acu_batch_create(acu_ctx* ctx, int nslices, const int* nimage, const int* nt
     for (auto& s : b->s)
       if (acu::fft_supported(s.N)) {
         s.ff_begin = b->ff_total; s.ff_n = acu::fft_blocks(s.N, s.T, b->ff_threads); b->ff_total += s.ff_n;
+      } else {
+        s.rfp_begin = b->rfp_total; b->rfp_total += s.rf_n;
       }
     acu::assign_bp(b.get());
     b->ew_total = ew; b->sw_total = sw;

@@ -1,10 +1,11 @@
 """The FP64 ramp filter by FFT on rows that are not ordinary: mixtures of
 infinities and NaN against the plain FP64 sum, one or a few values that
-dominate the row, and the time that infinities cost."""
+dominate the row, the time that infinities cost, and batches with slices past
+its length limit."""
 import numpy as np
 import pytest
 
-from acumen_amd import Batch, _lib, synth
+from acumen_amd import ACU_IMG_FBP, Batch, _lib, synth
 from helpers import HipBuffers
 
 pytestmark = pytest.mark.gpu
@@ -102,3 +103,34 @@ def test_infinities_cost_no_plain_sum(ctx):
     column = ramp(ctx, s, 5)
     print("ms:", finite, column, flush=True)
     assert column < 4 * finite
+
+
+def fbp_images(ctx, spec, fs):
+    with Batch(ctx, spec) as b:
+        for i, f in enumerate(fs):
+            b.set_sino(i, f)
+        best = np.inf
+        for _ in range(4):
+            ctx.set_timing(True)
+            b.fbp()
+            best = min(best, ctx.kernel_time(_lib.KIND_RAMP)[0])
+        ctx.set_timing(False)
+        return [b.get_image(i, ACU_IMG_FBP) for i in range(len(fs))], best
+
+
+def test_slices_past_the_fft_limit_share_a_launch(ctx):
+    """Slices of N > 4097 (the FP64 matrix product) between slices within the
+    limit equal single plans, and six of few angles take one launch's time: 71
+    workgroups each, where the GPU runs several hundred at once."""
+    print("[case] ramp past the FFT limit", flush=True)
+    sizes = [(4099, 3), (65, 20), (4098, 70), (4500, 16), (33, 1), (4099, 3)]
+    fs = [np.random.default_rng(i).random((T, N), np.float32) for i, (N, T) in enumerate(sizes)]
+    spec = [(N, T, 4, synth.angles(T)) for N, T in sizes]
+    got, _ = fbp_images(ctx, spec, fs)
+    for i, f in enumerate(fs):
+        want, _ = fbp_images(ctx, spec[i:i + 1], [f])
+        assert np.array_equal(got[i], want[0]), i
+    _, one = fbp_images(ctx, spec[3:4], fs[3:4])
+    _, six = fbp_images(ctx, spec[3:4] * 6, fs[3:4] * 6)
+    print("ms:", one, six, flush=True)
+    assert six < 3 * one
