@@ -9,6 +9,8 @@
 
 #include "acu_internal.hpp"
 
+#include <vector>
+
 namespace acu {
 
 constexpr int ADJ_T = 16;          // pixel tile side of the adjoint (16 x 16 threads)
@@ -20,6 +22,8 @@ constexpr int ADJ_GROUP = 8;       // most slices of one geometry a workgroup ta
 // 126 | 85 | 76 | 85, 8 x 257^2 x 180 (2312) 345 | 221 | 169 | 175, 16 x 257^2
 // 600 | 363 | 243 | 210, 8 x 513^2 x 360 (8712) 1958 | 1132 | 704 | 570
 inline int adj_group(int tiles) { return tiles < 2048 ? ADJ_GROUP / 2 : ADJ_GROUP; }
+// The width of a task of n slices: rays that lie side by side in LDS.
+__host__ __device__ inline int adj_width(int n) { return n <= 2 ? n : n <= 4 ? 4 : 8; }
 constexpr int GR_THREADS = 256;
 
 // Exact transpose of radon: img(px,py) = (1/N) sum over angles and samples
@@ -30,7 +34,7 @@ struct AdjTask {
   float mid;
   int block_begin;   // first global block of this slice
   int ntx;           // tiles per side: ceil(N / ADJ_T)
-  int n;             // slices of the task, of one geometry (N, T, angles): at most the launch's group
+  int n;             // slices of the task, of one geometry (N, T, angles): at most ADJ_GROUP
   const float2* sc;  // (sin, cos) of the projector angles
   const float* sino[ADJ_GROUP];  // (T, N); entries past n are read as well: any of the first n
   float* out[ADJ_GROUP];         // (N, N); entries past n are not written
@@ -74,8 +78,11 @@ struct LossTask {
 inline int adj_tiles(int N) { return (N + ADJ_T - 1) / ADJ_T; }
 inline int tvg_blocks(int N) { return (int)(((size_t)N * N + GR_THREADS - 1) / GR_THREADS); }
 
-// group: 1, 2, 4 or 8, the slices a workgroup takes together (n of each task at most)
-void launch_adjoint(const AdjTask* d_tasks, int ntasks, int group, int blocks, hipStream_t s);
+// Slices by geometry (equal numbers in geo are of one) and angle count, up to
+// `most` to a group, the groups whose tiles take longest first.
+std::vector<std::vector<int>> adj_groups(const std::vector<int>& geo, const std::vector<int>& T, int most);
+// tasks: the host copy of d_tasks, their blocks numbered in order from 0
+void launch_adjoint(const AdjTask* d_tasks, const std::vector<AdjTask>& tasks, hipStream_t s);
 void launch_shift_resid(const ResTask* d_tasks, int ntasks, int base, int rows, hipStream_t s);
 void launch_tvgrad(const TVGTask* d_tasks, int ntasks, int base, int blocks, hipStream_t s);
 void launch_loss_finalize(const LossTask* d_tasks, int ntasks, hipStream_t s);

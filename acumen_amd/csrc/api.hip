@@ -1431,34 +1431,35 @@ AdjTask adj_task(const Slice& s, int block_begin, const float* sino, float* out)
 }
 
 // Adjoint tasks of all slices, sino(i) -> out(i), slices of one geometry up to
-// ADJ_GROUP to a task (half of it in small launches); their blocks in total.
+// ADJ_GROUP to a task (half of it in small launches).
 template <class InF, class OutF>
-int adj_tasks(const acu_batch* b, std::vector<AdjTask>& t, InF in, OutF out) {
-  std::map<int, int> open;  // geometry -> its last task
+std::vector<AdjTask> adj_tasks(const acu_batch* b, InF in, OutF out) {
   int blocks = 0, tiles = 0;
-  for (const auto& s : b->s) tiles += adj_tiles(s.N) * adj_tiles(s.N);
-  const int group = adj_group(tiles);
-  for (int i = 0; i < (int)b->s.size(); ++i) {
-    const auto it = open.find(b->geo[i]);
-    if (it != open.end() && t[it->second].n < group) {
-      AdjTask& a = t[it->second];
-      a.sino[a.n] = in(i);
-      a.out[a.n++] = out(i);
-      continue;
-    }
-    open[b->geo[i]] = (int)t.size();
-    t.push_back(adj_task(b->s[i], blocks, in(i), out(i)));
-    blocks += adj_tiles(b->s[i].N) * adj_tiles(b->s[i].N);
+  std::vector<int> T;
+  for (const auto& s : b->s) {
+    tiles += adj_tiles(s.N) * adj_tiles(s.N);
+    T.push_back(s.T);
   }
-  return blocks;
+  std::vector<AdjTask> t;
+  for (const auto& g : adj_groups(b->geo, T, adj_group(tiles))) {
+    const Slice& s = b->s[g[0]];
+    t.push_back(adj_task(s, blocks, in(g[0]), out(g[0])));
+    AdjTask& a = t.back();
+    for (a.n = 1; a.n < (int)g.size(); ++a.n) {
+      a.sino[a.n] = in(g[a.n]);
+      a.out[a.n] = out(g[a.n]);
+    }
+    blocks += adj_tiles(s.N) * adj_tiles(s.N);
+  }
+  return t;
 }
 
 void radon_adjoint_dev(acu_batch* b, int sl, float* img, const float* sino) {
   Slice& s = slice_of(b, sl);
   acu_ctx* c = b->ctx;
-  AdjTask* d = put_adhoc(b, adj_task(s, 0, sino, img));
-  const int nb = adj_tiles(s.N) * adj_tiles(s.N);
-  timed(c, K_ADJ, [&] { launch_adjoint(d, 1, 1, nb, c->stream); });
+  const AdjTask t = adj_task(s, 0, sino, img);
+  AdjTask* d = put_adhoc(b, t);
+  timed(c, K_ADJ, [&] { launch_adjoint(d, {t}, c->stream); });
   check_launch();
 }
 
@@ -1529,13 +1530,10 @@ void loss_grad_run(acu_batch* b, const std::vector<const float*>& x, const std::
   launch_shift_resid(b->res_g.d, n, 0, rows, c->stream);
   check_launch();
   if (!gx.empty()) {
-    std::vector<AdjTask> adj;
-    const int blocks = adj_tasks(b, adj, [&](int i) { return b->s[i].gx_rs; }, [&](int i) { return gx[i]; });
-    int group = 1;
-    for (const auto& t : adj)
-      while (group < t.n) group *= 2;
+    const std::vector<AdjTask> adj =
+        adj_tasks(b, [&](int i) { return b->s[i].gx_rs; }, [&](int i) { return gx[i]; });
     b->adj_g.upload(adj, b->ctx->stream);
-    timed(c, K_ADJ, [&] { launch_adjoint(b->adj_g.d, b->adj_g.n, group, blocks, c->stream); });
+    timed(c, K_ADJ, [&] { launch_adjoint(b->adj_g.d, adj, c->stream); });
     check_launch();
   }
   launch_tvgrad(b->tvg_g.d, n, 0, tvb, c->stream);

@@ -36,6 +36,9 @@
 // per angle), 2.2 by fours, 1.75 by eights; one 257^2 x 180 130 us (344).
 #include "acu_grad.hpp"
 
+#include <algorithm>
+#include <map>
+
 namespace acu {
 namespace {
 
@@ -129,17 +132,11 @@ __device__ __forceinline__ void adj_angle(const AdjPixel& g, float s, float c, f
   for (int k = 0; k < G; ++k) blk[k] += v[k];
 }
 
+// One 16 x 16 tile of a task, its n <= G slices together.
 template <int G>
-__global__ __launch_bounds__(ADJ_T * ADJ_T) void adjoint_kernel(const AdjTask* __restrict__ tasks, int ntasks,
-                                                                int base, int nblocks) {
-  __shared__ AdjRay<G> P[ADJ_AB * ADJ_W];
-  const int lbk = xcd_remap(blockIdx.x, gridDim.x);
-  if (lbk >= nblocks) return;  // uniform per workgroup
-  const int gb = base + lbk;
-  const AdjTask& tk = tasks[find_by<AdjTask, &AdjTask::block_begin>(tasks, ntasks, gb)];
+__device__ __forceinline__ void adjoint_tile(const AdjTask& tk, int local, AdjRay<G>* __restrict__ P) {
   const int N = tk.N, T = tk.T;
   const float m = tk.mid;
-  const int local = gb - tk.block_begin;
   const int ty = local / tk.ntx, tx = local - ty * tk.ntx;
   const int tid = (int)threadIdx.x, lane = tid & 63;
   const int px = tx * ADJ_T + tid % ADJ_T + 1;  // 1-based pixel; past the image in the last tiles (not stored)
@@ -220,6 +217,28 @@ __global__ __launch_bounds__(ADJ_T * ADJ_T) void adjoint_kernel(const AdjTask* _
 #pragma unroll
     for (int k = 0; k < G; ++k)
       if (k < tk.n) tk.out[k][(size_t)(py - 1) * N + (px - 1)] = acc[k] / (float)N;
+}
+
+// W: the most slices of a task.  Each task runs at its own width, so a slice
+// without a partner costs what it would in a launch of single slices: 5 equal
+// and 20 different slices of 513^2 x 360 (loss and gradients) take 6.5 ms, 25
+// different ones 6.95, with every task at the width of the widest 7.85.  Blocks
+// go round-robin over the XCDs, the tasks of the longest first: with
+// contiguous shares of the blocks the XCD of the wide tasks was the last (9
+// equal slices 1.65 ms instead of 1.47, eight sizes from 65^2 x 1000 to
+// 600^2 x 90 1.44 instead of 1.16), and sharing an L2 gains nothing here (25
+// different slices the same).
+template <int W>
+__global__ __launch_bounds__(ADJ_T * ADJ_T) void adjoint_kernel(const AdjTask* __restrict__ tasks, int ntasks) {
+  __shared__ AdjRay<W> P[ADJ_AB * ADJ_W];
+  const int gb = (int)blockIdx.x;
+  const AdjTask& tk = tasks[find_by<AdjTask, &AdjTask::block_begin>(tasks, ntasks, gb)];
+  const int local = gb - tk.block_begin;
+  const int width = adj_width(tk.n);
+  if (W == 1 || width == 1) return adjoint_tile<1>(tk, local, (AdjRay<1>*)P);
+  if constexpr (W >= 2) if (width == 2) return adjoint_tile<2>(tk, local, (AdjRay<2>*)P);
+  if constexpr (W >= 4) if (width == 4) return adjoint_tile<4>(tk, local, (AdjRay<4>*)P);
+  if constexpr (W >= 8) adjoint_tile<8>(tk, local, (AdjRay<8>*)P);
 }
 
 __device__ __forceinline__ float at(const ACU_GLOBAL float* row, int N, int i) {
@@ -331,15 +350,42 @@ __global__ __launch_bounds__(GR_THREADS) void loss_finalize_kernel(const LossTas
 
 }  // namespace
 
-void launch_adjoint(const AdjTask* d_tasks, int ntasks, int group, int blocks, hipStream_t s) {
+std::vector<std::vector<int>> adj_groups(const std::vector<int>& geo, const std::vector<int>& T, int most) {
+  std::vector<std::vector<int>> g;
+  std::map<int, size_t> open;  // geometry -> its last group
+  for (int i = 0; i < (int)geo.size(); ++i) {
+    const auto it = open.find(geo[i]);
+    if (it != open.end() && (int)g[it->second].size() < most) {
+      g[it->second].push_back(i);
+      continue;
+    }
+    open[geo[i]] = g.size();
+    g.push_back({i});
+  }
+  // a tile's time: us per tile and angle at widths 1, 2, 4 and 8 as 245, 283, 352 and 570
+  auto time = [&](const std::vector<int>& v) {
+    const int w = adj_width((int)v.size());
+    return (double)T[v[0]] * (w == 1 ? 245 : w == 2 ? 283 : w == 4 ? 352 : 570);
+  };
+  std::stable_sort(g.begin(), g.end(), [&](const auto& a, const auto& b) { return time(a) > time(b); });
+  return g;
+}
+
+void launch_adjoint(const AdjTask* d_tasks, const std::vector<AdjTask>& tasks, hipStream_t s) {
+  int most = 1, blocks = 0;
+  for (const AdjTask& t : tasks) {
+    if (t.n < 1 || t.n > ADJ_GROUP || t.block_begin != blocks) throw Error("adjoint tasks do not match the launch");
+    most = std::max(most, adj_width(t.n));
+    blocks += t.ntx * t.ntx;
+  }
   if (blocks <= 0) return;
-  const dim3 grid(xcd_grid(blocks)), wg(ADJ_T * ADJ_T);
-  switch (group) {
-    case 1: hipLaunchKernelGGL(adjoint_kernel<1>, grid, wg, 0, s, d_tasks, ntasks, 0, blocks); break;
-    case 2: hipLaunchKernelGGL(adjoint_kernel<2>, grid, wg, 0, s, d_tasks, ntasks, 0, blocks); break;
-    case 4: hipLaunchKernelGGL(adjoint_kernel<4>, grid, wg, 0, s, d_tasks, ntasks, 0, blocks); break;
-    case 8: hipLaunchKernelGGL(adjoint_kernel<8>, grid, wg, 0, s, d_tasks, ntasks, 0, blocks); break;
-    default: throw Error("the adjoint takes 1, 2, 4 or 8 slices together");
+  const dim3 grid(blocks), wg(ADJ_T * ADJ_T);
+  const int n = (int)tasks.size();
+  switch (most) {
+    case 1: hipLaunchKernelGGL(adjoint_kernel<1>, grid, wg, 0, s, d_tasks, n); break;
+    case 2: hipLaunchKernelGGL(adjoint_kernel<2>, grid, wg, 0, s, d_tasks, n); break;
+    case 4: hipLaunchKernelGGL(adjoint_kernel<4>, grid, wg, 0, s, d_tasks, n); break;
+    default: hipLaunchKernelGGL(adjoint_kernel<8>, grid, wg, 0, s, d_tasks, n); break;
   }
 }
 
