@@ -228,9 +228,11 @@ struct BPShares { int b[XCDS + 1]; int C; };
 BPShares bp_xcd_shares(const std::vector<float>& w);
 void launch_backproject(const BPTask* d_tasks, int ntasks, int base, int tiles, int ty, bool refpos,
                         const BPShares& sh, hipStream_t s);
-// The same, with the reference's positions, for tasks of two slices each
-// (sino2, img2): the positions are computed once for both.
-void launch_backproject_pairs(const BPTask* d_tasks, int ntasks, int tiles, int ty, const BPShares& sh, hipStream_t s);
+// The same, with the reference's positions, where some tasks are of two slices
+// (sino2, img2), whose positions are computed once for both.
+// share: see bp_pad.
+void launch_backproject_pairs(const BPTask* d_tasks, int ntasks, int tiles, int share, int ty, const BPShares& sh,
+                              hipStream_t s);
 // The same, with the reference's positions, for launches of few tiles
 // (bp_use_split): small tiles, their angle blocks over the waves of a
 // workgroup.  Counted in 64 x 8 tiles, bp_split_tiles(N) (even) per slice.
@@ -238,9 +240,12 @@ int bp_split_tiles(int N);
 // tile height of a batch of that many 64 x 8 tiles: ty (its setting) when
 // they fill the GPU several times over, else 16
 int bp_launch_height(int tiles, int ty);
-// whether a launch of that many 64 x 8 tiles takes slices in pairs; rest:
-// some slices have no partner
-bool bp_use_pairs(int tiles, bool rest);
+// whether a launch of that many 64 x 8 tiles, `paired` of them of slices with a
+// partner, takes slices in pairs
+bool bp_use_pairs(int tiles, int paired);
+// LDS bytes that a launch asks for on top of its kernel's own; share: the
+// workgroups of the fullest XCD that do not only store zeros (0: none are asked for)
+int bp_pad(int share, int own);
 bool bp_use_split(int tiles, int T);  // T: the launch's most angles
 void launch_backproject_split(const BPTask* d_tasks, int ntasks, int base, int tiles, hipStream_t s);
 void launch_cells(const CellTask* d_tasks, int ntasks, int base, int blocks, hipStream_t s);

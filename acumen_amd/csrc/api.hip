@@ -227,11 +227,10 @@ struct RFSet {
 };
 
 // Backprojection tasks of one operand pair: of every slice, and, where slices
-// share their geometry, of a launch over all slices in two parts: pairs of
-// slices (pair) and the slices without a partner (rest).
+// share their geometry, of a launch over all slices with those in pairs.
 struct BPSet {
-  DevArray<BPTask> all, pair, rest;
-  void release() { all.release(); pair.release(); rest.release(); }
+  DevArray<BPTask> all, pairs;
+  void release() { all.release(); pairs.release(); }
 };
 
 // Task arrays of one radon operand pair, one array per variant group; a
@@ -277,12 +276,13 @@ struct acu_batch {
   acu::BPShares bp_sh_all{};          // XCD shares of the backprojection over all slices
   std::vector<int> geo;               // each slice's geometry (find_geometries)
   // slices of one geometry and window in pairs: each slice's partner
-  // or -1 (find_pairs), and the XCD shares of the two parts of a launch
+  // or -1 (find_pairs)
   std::vector<int> bp_partner;
   bool bp_built = true;               // false: a change of angles failed before the tasks were rebuilt
   bool bp_pairs = false;              // whether launches over all slices take them (bp_use_pairs)
   int maxT = 0;                       // most angles of a slice
-  acu::BPShares bp_sh_pair{}, bp_sh_rest{};
+  acu::BPShares bp_sh_pairs{};        // their XCD shares
+  int bp_share = 0;                   // and BPPlan::share
   bool bp_refpos = true;              // FBP backprojection positions in the reference's arithmetic
   bool tv_bp_refpos = true;           // the same inside tvopt's iteration
   // task sets for the fixed operand combinations of FBP / TV
@@ -659,31 +659,50 @@ std::vector<int> find_pairs(const acu_batch* b) {
   return partner;
 }
 
-// The two parts of a backprojection launch over the first ns slices at tile
-// height ty (one part if not pairs): their tasks and the estimated work of
-// their tiles.
-struct BPParts {
-  std::vector<BPTask> pair, rest;
-  std::vector<float> pair_work, rest_work;
+// The tasks of a backprojection launch over the first ns slices at tile height
+// ty, partners in one task if pairs, and the estimated work of their tiles (a
+// pair's is 1.54 of a slice's: 4.67 and 6.04 ms per 8 x 2049^2 x 1500).
+struct BPPlan {
+  std::vector<BPTask> tasks;
+  std::vector<float> work;
+  std::vector<uint8_t> active;  // 1 for a tile with a mask pixel, 0 for one that only stores zeros
+  // For a launch at shares sh: the active tiles of the fullest share, or 0
+  // where the dispatch of the other tiles counts beside the chains (fewer than
+  // 64 angles a tile, those counted as none): 700 x 65^2 x 48 66 us with room
+  // for 5 workgroups a CU, 73 with 3; 256 x 129^2 x 90 86 with 5, 96 with 4; but
+  // 2 x 1025^2 x 100 54 with 6 and 45 with 4.
+  int share(const BPShares& sh) const {
+    int most = 0;
+    for (int k = 0; k < XCDS; ++k) {
+      int c = 0;
+      for (int i = sh.b[k]; i < sh.b[k + 1]; ++i) c += active[i];
+      most = std::max(most, c);
+    }
+    double angles = 0.0;
+    for (size_t t = 0, i = 0; t < tasks.size(); ++t)
+      for (const size_t end = i + (size_t)tasks[t].ntx * tasks[t].nty; i < end; ++i) angles += active[i] * tasks[t].T;
+    return angles >= 64.0 * active.size() ? most : 0;
+  }
 };
 template <class InF, class OutF>
-BPParts bp_parts(acu_batch* b, int ns, int ty, bool pairs, InF in, OutF out) {
-  BPParts p;
+BPPlan bp_plan(acu_batch* b, int ns, int ty, bool pairs, InF in, OutF out) {
+  BPPlan p;
   for (int i = 0; i < ns; ++i) {
     Slice& s = b->s[i];
     const int j = b->bp_partner[i];
     const bool two = pairs && j >= 0 && j < ns;
     if (two && j < i) continue;  // with its partner's task
-    std::vector<float>& w = two ? p.pair_work : p.rest_work;
     BPTask t = bp_task(s, in(s), out(s));
     t.nty = bp_tiles_y(s.N, ty);
-    t.tile_begin = (int)w.size();
+    t.tile_begin = (int)p.work.size();
+    bp_tile_work(s, ty, p.work);
+    for (size_t k = t.tile_begin; k < p.work.size(); ++k) p.active.push_back(p.work[k] == (float)s.T);
     if (two) {
       t.sino2 = in(b->s[j]);
       t.img2 = out(b->s[j]);
+      for (size_t k = t.tile_begin; k < p.work.size(); ++k) p.work[k] *= 1.54f;
     }
-    bp_tile_work(s, ty, w);
-    (two ? p.pair : p.rest).push_back(t);
+    p.tasks.push_back(t);
   }
   return p;
 }
@@ -691,12 +710,9 @@ BPParts bp_parts(acu_batch* b, int ns, int ty, bool pairs, InF in, OutF out) {
 template <class InF, class OutF>
 void build_bpset(acu_batch* b, BPSet& set, InF in, OutF out) {
   build(b, set.all, [&](Slice& s) { return bp_task(s, in(s), out(s)); });
-  set.pair.release();
-  set.rest.release();
-  if (!b->bp_pairs) return;  // the launch is over set.all
-  const BPParts p = bp_parts(b, (int)b->s.size(), b->bp_h, true, in, out);
-  set.pair.upload(p.pair, b->ctx->stream);
-  set.rest.upload(p.rest, b->ctx->stream);
+  set.pairs.release();
+  if (b->bp_pairs)  // else the launch is over set.all
+    set.pairs.upload(bp_plan(b, (int)b->s.size(), b->bp_h, true, in, out).tasks, b->ctx->stream);
 }
 
 // Pairs, and the XCD shares of the all-slice and per-slice backprojection
@@ -705,10 +721,12 @@ void assign_bp_shares(acu_batch* b) {
   b->geo = find_geometries(b);
   b->bp_partner = find_pairs(b);
   const auto none = [](Slice&) { return (float*)nullptr; };
-  const BPParts p = bp_parts(b, (int)b->s.size(), b->bp_h, true, none, none);
-  b->bp_pairs = !p.pair.empty() && bp_use_pairs(b->bps_total, !p.rest.empty());
-  b->bp_sh_pair = bp_xcd_shares(p.pair_work);
-  b->bp_sh_rest = bp_xcd_shares(p.rest_work);
+  const BPPlan p = bp_plan(b, (int)b->s.size(), b->bp_h, true, none, none);
+  int paired = 0;
+  for (size_t i = 0; i < b->s.size(); ++i) paired += b->bp_partner[i] >= 0 ? b->s[i].bps_n : 0;
+  b->bp_pairs = bp_use_pairs(b->bps_total, paired);
+  b->bp_sh_pairs = bp_xcd_shares(p.work);
+  b->bp_share = p.share(b->bp_sh_pairs);
   std::vector<float> all, one;
   for (auto& s : b->s) {
     one.clear();
@@ -861,8 +879,7 @@ void backproject(acu_batch* b, const BPSet& bp, int sl, bool refpos) {
   if (refpos && bp_use_split(b->bps_total, b->maxT)) {
     launch_backproject_split(bp.all.d, bp.all.n, 0, b->bps_total, st);
   } else if (refpos && b->bp_pairs) {
-    launch_backproject_pairs(bp.pair.d, bp.pair.n, b->bp_sh_pair.b[XCDS], b->bp_h, b->bp_sh_pair, st);
-    launch_backproject(bp.rest.d, bp.rest.n, 0, b->bp_sh_rest.b[XCDS], b->bp_h, true, b->bp_sh_rest, st);
+    launch_backproject_pairs(bp.pairs.d, bp.pairs.n, b->bp_sh_pairs.b[XCDS], b->bp_share, b->bp_h, b->bp_sh_pairs, st);
   } else {
     launch_backproject(bp.all.d, bp.all.n, 0, b->bp_total, b->bp_h, refpos, b->bp_sh_all, st);
   }
@@ -1327,14 +1344,14 @@ double time_bp(acu_batch* b, int ty, int reps) {
     img[&b->s[i]] = sc.p + off;
     off += (size_t)b->s[i].N * b->s[i].N;
   }
-  const BPParts p = bp_parts(b, ns, ty, b->bp_refpos && b->bp_pairs, [](Slice& s) { return s.sinoCS; }, [&](Slice& s) { return img[&s]; });
-  struct Tasks : DevArray<BPTask> { ~Tasks() { release(); } } pair, rest;
-  pair.upload(p.pair, c->stream);
-  rest.upload(p.rest, c->stream);
-  const BPShares shp = bp_xcd_shares(p.pair_work), shr = bp_xcd_shares(p.rest_work);
+  const bool pairs = b->bp_refpos && b->bp_pairs;
+  const BPPlan p = bp_plan(b, ns, ty, pairs, [](Slice& s) { return s.sinoCS; }, [&](Slice& s) { return img[&s]; });
+  struct Tasks : DevArray<BPTask> { ~Tasks() { release(); } } tasks;
+  tasks.upload(p.tasks, c->stream);
+  const BPShares sh = bp_xcd_shares(p.work);
   auto run = [&] {
-    launch_backproject_pairs(pair.d, pair.n, shp.b[XCDS], ty, shp, c->stream);
-    launch_backproject(rest.d, rest.n, 0, shr.b[XCDS], ty, b->bp_refpos, shr, c->stream);
+    if (pairs) launch_backproject_pairs(tasks.d, tasks.n, sh.b[XCDS], p.share(sh), ty, sh, c->stream);
+    else launch_backproject(tasks.d, tasks.n, 0, sh.b[XCDS], ty, b->bp_refpos, sh, c->stream);
   };
   hipEvent_t e0 = c->ev(), e1 = c->ev();
   run();

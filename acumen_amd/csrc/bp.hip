@@ -48,8 +48,7 @@
 //    ds_read2st64_b64 takes 8, a b128 of interleaved pairs 5.9 with its bank
 //    conflicts), staged 16 angles at a time so that 5 workgroups fit a CU.
 //    8 x 2049^2 x 1500 5.75 to 5.07 ms (0.63 ms a slice), 4 x 1025^2 x 720
-//    490 to 390 us.  1.25 wave-instructions per CU and clock, LDS 69% busy,
-//    at 1.95 GHz (2.1 with one slice): the power limit is near as well;
+//    490 to 390 us, and 4.79 with five waves per SIMD instead of four;
 //  * each 32-angle block is summed separately and then added;
 //  * tiles whose mask is identically zero (by 64 x 16 sub-tiles) only store
 //    zeros.
@@ -79,33 +78,37 @@ __device__ __forceinline__ int find_task(const BPTask* tasks, int ntasks, int gt
   return lo;
 }
 
+// LDS of a workgroup: AS angles' pairs (of two slices if G = 2), window starts,
+// constants and row terms.
 template <int TY, bool REFPOS, int G>
-__global__ __launch_bounds__(64 * bp_waves(TY)) void bp_kernel(const BPTask* __restrict__ tasks, int ntasks, int base,
-                                                               BPShares sh) {
+struct BPLds {
+  static constexpr int AS = G == 2 ? 16 : AB;  // angles staged at a time (G = 1 with 16: 2% slower)
+  static constexpr int W = (G == 2 && TY == 16) ? 80 : bp_window(TY);
+  // second slice's window; not a multiple of 512 bytes, which would merge the reads
+  static constexpr int P2 = AS * W + 1;
+  float2 P[G == 2 ? P2 + AS * W : AS * W];
+  float2 ab[REFPOS ? AS : 1];  // sine, LDS offset of P[a * W - 1 - lo] (lds_units)
+  __attribute__((aligned(16))) float rt[REFPOS ? AS * TY : 1];  // row terms of the tile
+  int lo[AS];
+  float k[AS];  // K of the tile-local position (see above)
+};
+
+// Tile `local` of a task, its G slices together.
+template <int TY, bool REFPOS, int G>
+__device__ __forceinline__ void bp_tile(const BPTask& tk, int local, BPLds<TY, REFPOS, G>& lds) {
+  typedef BPLds<TY, REFPOS, G> L;
   constexpr int NW = bp_waves(TY), NT = 64 * NW, PY = TY / NW, SUBS = TY / BP_SUB;
-  constexpr int AS = G == 2 ? 16 : AB;  // angles staged at a time (G = 1 with 16: 2% slower)
-  constexpr int W = (G == 2 && TY == 16) ? 80 : bp_window(TY);
+  constexpr int AS = L::AS, W = L::W, P2 = L::P2;
   constexpr int SPA = NT / AS, NST = W / SPA;  // staging threads per angle, pairs per thread
   static_assert(G == 1 || (G == 2 && REFPOS), "pairs have the reference's positions");
   static_assert(TY % BP_SUB == 0 && TY % NW == 0 && NT % AS == 0 && W % SPA == 0 && AB % AS == 0, "tile shape");
-  constexpr int P2 = AS * W + 1;  // second slice's window; not a multiple of 512 bytes, which would merge the reads
-  __shared__ float2 P[G == 2 ? P2 + AS * W : AS * W];
-  __shared__ int lo_s[AS];
-  __shared__ float k_s[AS];    // K of the tile-local position (see above)
-  // row terms of the tile
-  __shared__ __attribute__((aligned(16))) float rt_s[REFPOS ? AS * TY : 1];
-  __shared__ float2 ab_s[REFPOS ? AS : 1];  // sine, LDS offset of P[a * W - 1 - lo] (lds_units)
-
-  // XCD k (xcd_remap) runs the tiles of its share in order
-  const int l = xcd_remap(blockIdx.x, gridDim.x);
-  const int k = l / sh.C;
-  const int lt = sh.b[k] + (l - k * sh.C);
-  if (lt >= sh.b[k + 1]) return;
-  const int gtile = base + lt;
-  const BPTask& tk = tasks[find_task(tasks, ntasks, gtile)];
+  float2* const P = lds.P;
+  int* const lo_s = lds.lo;
+  float* const k_s = lds.k;
+  float* const rt_s = lds.rt;
+  float2* const ab_s = lds.ab;
   const int N = tk.N, T = tk.T;
   const float m = tk.mid;
-  const int local = gtile - tk.tile_begin;
   const int tx = local % tk.ntx, tyi = local / tk.ntx;
   const int x0 = tx * TX, y0 = tyi * TY;
   const int tid = threadIdx.x;
@@ -283,6 +286,32 @@ __global__ __launch_bounds__(64 * bp_waves(TY)) void bp_kernel(const BPTask* __r
   }
 }
 
+template <int TY, bool REFPOS, bool PAIRS>
+constexpr int bp_lds() {
+  const int a = sizeof(BPLds<TY, REFPOS, 1>), b = sizeof(BPLds<TY, REFPOS, PAIRS ? 2 : 1>);
+  return a > b ? a : b;
+}
+
+// PAIRS: tasks of two slices (sino2) beside tasks of one, each at its own
+// width.  Five waves per SIMD (96 registers instead of 101) for those.
+template <int TY, bool REFPOS, bool PAIRS>
+__global__ __launch_bounds__(64 * bp_waves(TY), PAIRS ? 5 : 1) void bp_kernel(const BPTask* __restrict__ tasks,
+                                                                              int ntasks, int base, BPShares sh) {
+  typedef BPLds<TY, REFPOS, 1> L1;
+  typedef BPLds<TY, REFPOS, PAIRS ? 2 : 1> L2;
+  __shared__ __attribute__((aligned(16))) char lds[bp_lds<TY, REFPOS, PAIRS>()];
+  // XCD k (xcd_remap) runs the tiles of its share in order
+  const int l = xcd_remap(blockIdx.x, gridDim.x);
+  const int k = l / sh.C;
+  const int lt = sh.b[k] + (l - k * sh.C);
+  if (lt >= sh.b[k + 1]) return;
+  const int gtile = base + lt;
+  const BPTask& tk = tasks[find_task(tasks, ntasks, gtile)];
+  const int local = gtile - tk.tile_begin;
+  if constexpr (PAIRS) if (tk.sino2) return bp_tile<TY, REFPOS, 2>(tk, local, *(L2*)lds);
+  bp_tile<TY, REFPOS, 1>(tk, local, *(L1*)lds);
+}
+
 // Backprojection of the smallest launches, with the reference's positions.  A
 // tile of the kernel above walks its angles serially, so its time grows with
 // T even where most CUs are idle (a 257^2 slice is 85 workgroups of 64 x 16).
@@ -419,12 +448,22 @@ int bp_split_tiles(int N) { return bp_tiles_x(N) * ((N + 15) / 16) * 2; }
 //   8840 (4 x 1025^2) x 720 454 | 432 | 400; 8514 (2049^2) x 1500 935 | 944 | 955
 bool bp_use_split(int tiles, int T) { return tiles <= 640 && T > 64; }
 int bp_launch_height(int tiles, int ty) { return tiles <= 5200 ? 16 : ty; }
-// us without | with pairs: 4 x 1025^2 x 720 478 | 400; 8 x 2049^2 x 1500 5960 |
-// 5200; 16 x 257^2 x 180 63 | 65.  A slice without a partner is a launch of
-// its own, with a tail of its own: 9 x 513^2 x 720 (5500 tiles) 360 | 397, 3 x
-// 1025^2 (6600) 376 | 463, 9 x 1025^2 (19900) 937 | 931, 3 x 2049^2 (25500)
-// 2421 | 2389, 5 x 2049^2 (42600) 3982 | 3666
-bool bp_use_pairs(int tiles, bool rest) { return !rest || tiles >= 19000; }
+// us per FBP without | with pairs, by the launch's 64 x 8 tiles (heights 16 up
+// to 5200, then 32): 1188 (2 x 513^2) x 360 70 | 90; 1360 (8 x 257^2) x 180 40 |
+// 51; 2376 (4 x 513^2) x 360 95 | 104; 2548 (2 x 769^2) x 600 153 | 152; 3456 (64 x
+// 129^2) x 90 35 | 37; 4080 (24 x 257^2) x 180 69 | 63; 5096 (4 x 769^2) x 600
+// 251 | 215; 8840 (4 x 1025^2) x 720 478 | 393; 68112 (8 x 2049^2) x 1500 6250 |
+// 4790.  A pair's tile takes 1.54 times as long, so a few pairs among single
+// slices lengthen the launch's end more than they shorten the rest: by share
+// of the tiles in pairs 0.2% (2 x 65^2 x 1500 + 3 x 2049^2 x 300) 475 | 552, 10%
+// (2 equal of 20 x 1025^2 x 720) 1891 | 1890, 20% (2 equal of 10 x 513^2 x 720) 376
+// | 386, 57% (4 equal of 7 x 1025^2 x 720) 713 | 663, 80% (16 of 20) 1890 | 1607;
+// and where a slice is left over in launches of few tiles: 6370 (5 x 769^2 x 600)
+// 318 | 331, 6534 (11 x 513^2 x 360) 197 | 204, 8918 (7 x 769^2 x 600) 411 | 389,
+// 25542 (3 x 2049^2 x 1500) 2299 | 2005.  Pairs and singles share a launch: in one
+// of each kind, the first's end waits for nobody (990 for the 0.2%, 5 x 2049^2 x
+// 1500 3450 instead of 3190).
+bool bp_use_pairs(int tiles, int paired) { return tiles >= (paired < tiles ? 8500 : 3500) && 2 * (long)paired >= tiles; }
 
 void launch_backproject_split(const BPTask* d_tasks, int ntasks, int base, int tiles, hipStream_t s) {
   if (tiles <= 0) return;
@@ -448,13 +487,34 @@ void launch_bp_rowterm(const float2* sc, int N, int T, float mid, float* rowterm
 int bp_tiles_x(int N) { return (N + TX - 1) / TX; }
 int bp_tiles_y(int N, int ty) { return (N + ty - 1) / ty; }
 
-template <bool REFPOS, int G>
-void launch_bp(const BPTask* d_tasks, int ntasks, int base, int ty, const BPShares& sh, hipStream_t s) {
-  const dim3 g((unsigned)(XCDS * sh.C));
+// LDS to ask for on top of a kernel's `own`, so that an XCD whose `share` of
+// workgroups (of those that do not only store zeros) fits its 32 CUs at once
+// spreads them evenly: no CU has room for more than its part.  Without it some
+// CUs fill up and the launch waits for those: us per FBP without | with, 4 x
+// 1025^2 x 720 444 | 393, 8 x 769^2 x 600 396 | 355, 16 x 513^2 x 360 238 | 210, 4
+// x 769^2 x 600 (16 rows) 244 | 215.  No fewer than 3 to a CU (64 x 129^2 x 90 37
+// with more, 52 with 2).
+int bp_pad(int share, int own) {
+  constexpr int CUS = 32, LDS = 160 << 10, GRAIN = 1280;
+  if (share <= 0) return 0;
+  const int k = std::max(3, (share + CUS - 1) / CUS);
+  const int total = LDS / k - GRAIN;  // k fit, k + 1 do not
+  return total > own ? total - own : 0;
+}
+
+template <int TY, bool REFPOS, bool PAIRS>
+void launch_bp_ty(const BPTask* d_tasks, int ntasks, int base, const BPShares& sh, int share, hipStream_t s) {
+  int pad = 0;
+  if (PAIRS) pad = bp_pad(share, bp_lds<TY, REFPOS, PAIRS>());
+  hipLaunchKernelGGL((bp_kernel<TY, REFPOS, PAIRS>), dim3((unsigned)(XCDS * sh.C)), dim3(64 * bp_waves(TY)), pad, s, d_tasks,
+                     ntasks, base, sh);
+}
+template <bool REFPOS, bool PAIRS>
+void launch_bp(const BPTask* d_tasks, int ntasks, int base, int ty, const BPShares& sh, int share, hipStream_t s) {
   switch (ty) {
-    case 16: hipLaunchKernelGGL((bp_kernel<16, REFPOS, G>), g, dim3(64 * bp_waves(16)), 0, s, d_tasks, ntasks, base, sh); break;
-    case 32: hipLaunchKernelGGL((bp_kernel<32, REFPOS, G>), g, dim3(64 * bp_waves(32)), 0, s, d_tasks, ntasks, base, sh); break;
-    case 64: hipLaunchKernelGGL((bp_kernel<64, REFPOS, G>), g, dim3(64 * bp_waves(64)), 0, s, d_tasks, ntasks, base, sh); break;
+    case 16: launch_bp_ty<16, REFPOS, PAIRS>(d_tasks, ntasks, base, sh, share, s); break;
+    case 32: launch_bp_ty<32, REFPOS, PAIRS>(d_tasks, ntasks, base, sh, share, s); break;
+    case 64: launch_bp_ty<64, REFPOS, PAIRS>(d_tasks, ntasks, base, sh, share, s); break;
     default: throw Error("backprojection tile height must be 16, 32 or 64");
   }
 }
@@ -467,14 +527,15 @@ void launch_backproject(const BPTask* d_tasks, int ntasks, int base, int tiles, 
                         const BPShares& sh, hipStream_t s) {
   if (tiles <= 0) return;
   check_bp_launch(d_tasks, ntasks, tiles, sh);
-  if (refpos) launch_bp<true, 1>(d_tasks, ntasks, base, ty, sh, s);
-  else launch_bp<false, 1>(d_tasks, ntasks, base, ty, sh, s);
+  if (refpos) launch_bp<true, false>(d_tasks, ntasks, base, ty, sh, 0, s);
+  else launch_bp<false, false>(d_tasks, ntasks, base, ty, sh, 0, s);
 }
 
-void launch_backproject_pairs(const BPTask* d_tasks, int ntasks, int tiles, int ty, const BPShares& sh, hipStream_t s) {
+void launch_backproject_pairs(const BPTask* d_tasks, int ntasks, int tiles, int share, int ty, const BPShares& sh,
+                              hipStream_t s) {
   if (tiles <= 0) return;
   check_bp_launch(d_tasks, ntasks, tiles, sh);
-  launch_bp<true, 2>(d_tasks, ntasks, 0, ty, sh, s);
+  launch_bp<true, true>(d_tasks, ntasks, 0, ty, sh, share, s);
 }
 
 // Cut points at k/XCDS of the total estimated work (a tile starts the next
