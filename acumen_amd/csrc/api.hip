@@ -226,11 +226,15 @@ struct RFSet {
   void release() { rf.release(); past.release(); ff.release(); }
 };
 
-// Backprojection tasks of one operand pair: of every slice, and, where slices
-// share their geometry, of a launch over all slices with those in pairs.
+// Backprojection tasks of one operand pair: of every slice, and after those,
+// where slices share their geometry, of a launch over all slices with those in
+// pairs.
 struct BPSet {
-  DevArray<BPTask> all, pairs;
-  void release() { all.release(); pairs.release(); }
+  DevArray<BPTask> tasks;
+  int n = 0;  // tasks of single slices
+  const BPTask* pairs() const { return tasks.d + n; }
+  int npairs() const { return tasks.n - n; }
+  void release() { tasks.release(); }
 };
 
 // Task arrays of one radon operand pair, one array per variant group; a
@@ -278,7 +282,8 @@ struct acu_batch {
   // slices of one geometry and window in pairs: each slice's partner
   // or -1 (find_pairs)
   std::vector<int> bp_partner;
-  bool bp_built = true;               // false: a change of angles failed before the tasks were rebuilt
+  bool geo_stale = false;             // angles changed since (settle_geometries)
+  bool bp_built = true;               // false: rebuilding the tasks for new pairs failed
   bool bp_pairs = false;              // whether launches over all slices take them (bp_use_pairs)
   int maxT = 0;                       // most angles of a slice
   acu::BPShares bp_sh_pairs{};        // their XCD shares
@@ -709,24 +714,30 @@ BPPlan bp_plan(acu_batch* b, int ns, int ty, bool pairs, InF in, OutF out) {
 
 template <class InF, class OutF>
 void build_bpset(acu_batch* b, BPSet& set, InF in, OutF out) {
-  build(b, set.all, [&](Slice& s) { return bp_task(s, in(s), out(s)); });
-  set.pairs.release();
-  if (b->bp_pairs)  // else the launch is over set.all
-    set.pairs.upload(bp_plan(b, (int)b->s.size(), b->bp_h, true, in, out).tasks, b->ctx->stream);
+  std::vector<BPTask> v;
+  for (auto& s : b->s) v.push_back(bp_task(s, in(s), out(s)));
+  set.n = (int)v.size();
+  if (b->bp_pairs) {
+    const BPPlan p = bp_plan(b, set.n, b->bp_h, true, in, out);
+    v.insert(v.end(), p.tasks.begin(), p.tasks.end());
+  }
+  set.tasks.upload(v, b->ctx->stream);
 }
 
-// Pairs, and the XCD shares of the all-slice and per-slice backprojection
-// launches.
-void assign_bp_shares(acu_batch* b) {
-  b->geo = find_geometries(b);
-  b->bp_partner = find_pairs(b);
-  const auto none = [](Slice&) { return (float*)nullptr; };
-  const BPPlan p = bp_plan(b, (int)b->s.size(), b->bp_h, true, none, none);
+// Whether launches over all slices take pairs, and then their XCD shares.
+void assign_bp_pairs(acu_batch* b) {
   int paired = 0;
   for (size_t i = 0; i < b->s.size(); ++i) paired += b->bp_partner[i] >= 0 ? b->s[i].bps_n : 0;
   b->bp_pairs = bp_use_pairs(b->bps_total, paired);
+  if (!b->bp_pairs) return;
+  const auto none = [](Slice&) { return (float*)nullptr; };
+  const BPPlan p = bp_plan(b, (int)b->s.size(), b->bp_h, true, none, none);
   b->bp_sh_pairs = bp_xcd_shares(p.work);
   b->bp_share = p.share(b->bp_sh_pairs);
+}
+
+// XCD shares of the all-slice and per-slice backprojection launches.
+void assign_bp_shares(acu_batch* b) {
   std::vector<float> all, one;
   for (auto& s : b->s) {
     one.clear();
@@ -735,6 +746,7 @@ void assign_bp_shares(acu_batch* b) {
     all.insert(all.end(), one.begin(), one.end());
   }
   b->bp_sh_all = bp_xcd_shares(all);
+  assign_bp_pairs(b);
 }
 
 // Backprojection tile ranges at the batch's tile height (and their XCD
@@ -759,6 +771,27 @@ void assign_bp(acu_batch* b) {
 }
 
 void build_op_tasks(acu_batch* b);
+
+// Geometries and pairs after changes of angles, and the tasks if the pairs
+// changed.  Done once before the next launch over all slices, not in each
+// change: a program that gives n slices new angles one by one parts and joins
+// pairs on the way (ms for the n changes and an FBP, settled in each and once:
+// 16 x 1025^2 x 360 8.3, 6.3; 16 x 257^2 x 180 3.2, 2.3).
+void settle_geometries(acu_batch* b) {
+  if (!b->geo_stale) return;
+  b->geo = find_geometries(b);
+  std::vector<int> partner = find_pairs(b);
+  if (!b->bp_built || partner != b->bp_partner) {
+    b->bp_built = false;
+    b->bp_partner = std::move(partner);
+    assign_bp_pairs(b);
+    build_op_tasks(b);
+    if (b->tv_mem) build_tv_tasks(b);
+    b->drop_graphs();
+    b->bp_built = true;
+  }
+  b->geo_stale = false;
+}
 
 // A new backprojection tile height: new ranges and task arrays, and a
 // captured outer iteration is rebuilt on the next tvopt.
@@ -825,9 +858,11 @@ void ensure_tv(acu_batch* b, int delta_cap) {
   b->tv.release();
 }
 
+// Every slice's angles are set; the batch is ready for work on all slices.
 void require_theta(acu_batch* b) {
   for (size_t i = 0; i < b->s.size(); ++i)
     if (!b->s[i].theta_set) throw Error("theta of slice " + std::to_string(i) + " was never set");
+  settle_geometries(b);
 }
 
 // ---- operator sequences (all slices at once, or one slice: sl >= 0) ----
@@ -874,14 +909,14 @@ void backproject_one(acu_batch* b, const BPTask* d, int n, int sl, bool own, boo
 // Backprojection of all slices (sl < 0) or one.  With the reference's
 // positions slices of one geometry go two to a workgroup (the same bits).
 void backproject(acu_batch* b, const BPSet& bp, int sl, bool refpos) {
-  if (sl >= 0) return backproject_one(b, bp.all.d, bp.all.n, sl, false, refpos);
+  if (sl >= 0) return backproject_one(b, bp.tasks.d, bp.n, sl, false, refpos);
   hipStream_t st = b->ctx->stream;
   if (refpos && bp_use_split(b->bps_total, b->maxT)) {
-    launch_backproject_split(bp.all.d, bp.all.n, 0, b->bps_total, st);
+    launch_backproject_split(bp.tasks.d, bp.n, 0, b->bps_total, st);
   } else if (refpos && b->bp_pairs) {
-    launch_backproject_pairs(bp.pairs.d, bp.pairs.n, b->bp_sh_pairs.b[XCDS], b->bp_share, b->bp_h, b->bp_sh_pairs, st);
+    launch_backproject_pairs(bp.pairs(), bp.npairs(), b->bp_sh_pairs.b[XCDS], b->bp_share, b->bp_h, b->bp_sh_pairs, st);
   } else {
-    launch_backproject(bp.all.d, bp.all.n, 0, b->bp_total, b->bp_h, refpos, b->bp_sh_all, st);
+    launch_backproject(bp.tasks.d, bp.n, 0, b->bp_total, b->bp_h, refpos, b->bp_sh_all, st);
   }
 }
 
@@ -1738,6 +1773,8 @@ int acu_batch_create(acu_ctx* ctx, int nslices, const int* nimage, const int* nt
         acu::upload_theta(b.get(), i);
       }
     }
+    b->geo = acu::find_geometries(b.get());
+    b->bp_partner = acu::find_pairs(b.get());
     acu::assign_bp_shares(b.get());
     if (b->ramp_variant == acu::RAMP_FFT)
       for (auto& s : b->s)
@@ -1787,17 +1824,8 @@ int acu_batch_set_theta(acu_batch* b, int slice, const float* theta_deg) {
           acu::upload_theta(b, slice);
           // whether the cells pass is launched depends on the angles, and so
           // does which slices the backprojection takes together
-          try {
-            if (b->s.size() > 1) {
-              const auto partner = b->bp_partner;
-              const bool pairs = b->bp_pairs, built = b->bp_built;
-              b->bp_built = false;
-              acu::assign_bp_shares(b);
-              if (!built || partner != b->bp_partner || pairs != b->bp_pairs) acu::build_op_tasks(b);
-              b->bp_built = true;
-            }
-            acu::refresh_fp(b);
-          } catch (...) { b->s[slice].theta_set = false; throw; });
+          b->geo_stale = true;
+          try { acu::refresh_fp(b); } catch (...) { b->s[slice].theta_set = false; throw; });
 }
 
 int acu_batch_set_sino(acu_batch* b, int slice, const float* f_host) {
@@ -2270,6 +2298,7 @@ void volume_run(acu_ctx* ctx, int nslices, int N, int T, int wpu, const float* t
     if (tv) {
       acu::tvopt_run(bt, mu, lambda, nouter, ninner, ncg, ACU_TV_GRAPH);
     } else {
+      acu::require_theta(bt);
       acu::fbp_all(bt, -1);
       for (auto& s : bt->s) s.fbp_valid = true;
     }
