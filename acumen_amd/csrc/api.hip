@@ -1364,8 +1364,15 @@ int bp_timing_slices(const acu_batch* b) {
   return n;
 }
 
+// Whether the batch's launches have one height, or the split kernel, whatever
+// tile height is set (bp_launch_height).
+bool bp_height_fixed(const acu_batch* b) {
+  return b->bp_refpos && b->tv_bp_refpos && bp_launch_height(b->bps_total, 32) == bp_launch_height(b->bps_total, 64);
+}
+
 // Average ms of one batched backprojection of those slices (sinoCS ->
-// scratch images, contents irrelevant to the timing) at tile height ty.
+// scratch images, contents irrelevant to the timing) at tile height ty, by the
+// kernel that the batch's launches take.
 double time_bp(acu_batch* b, int ty, int reps) {
   acu_ctx* c = b->ctx;
   const int ns = bp_timing_slices(b);
@@ -1385,7 +1392,10 @@ double time_bp(acu_batch* b, int ty, int reps) {
   tasks.upload(p.tasks, c->stream);
   const BPShares sh = bp_xcd_shares(p.work);
   auto run = [&] {
-    if (pairs) launch_backproject_pairs(tasks.d, tasks.n, sh.b[XCDS], p.share(sh), ty, sh, c->stream);
+    // of at most 640 tiles, so these are all of the batch's slices
+    if (b->bp_refpos && bp_use_split(b->bps_total, b->maxT))
+      launch_backproject_split(tasks.d, tasks.n, 0, b->bps_total, c->stream);
+    else if (pairs) launch_backproject_pairs(tasks.d, tasks.n, sh.b[XCDS], p.share(sh), ty, sh, c->stream);
     else launch_backproject(tasks.d, tasks.n, 0, sh.b[XCDS], ty, b->bp_refpos, sh, c->stream);
   };
   hipEvent_t e0 = c->ev(), e1 = c->ev();
@@ -1444,9 +1454,13 @@ std::string autotune(acu_batch* b, int reps, unsigned what = TUNE_ALL) {
     double best_ms = 0.0;
     js << ",\"ramp\":{\"ms\":{";
     bool first = true;
+    double fp64_ms = 0.0;
     for (int k = 0; k < 4; ++k) {
       if (rc[k] == RAMP_FFT && !fft_ok) continue;
-      const double ms = time_ramp(b, rc[k], reps);
+      // FFT is FP64's own launch where it is allowed: timed once, so that FP64,
+      // which takes slices of any size, is the choice between them
+      const double ms = rc[k] == RAMP_FFT ? fp64_ms : time_ramp(b, rc[k], reps);
+      if (rc[k] == RAMP_FP64) fp64_ms = ms;
       js << (first ? "" : ",") << "\"" << ramp_name(rc[k]) << "\":" << ms;
       first = false;
       if (best < 0 || ms < best_ms) { best = rc[k]; best_ms = ms; }
@@ -1457,16 +1471,20 @@ std::string autotune(acu_batch* b, int reps, unsigned what = TUNE_ALL) {
   // backprojection tile height: the fastest over the batch's first slices
   if (what & TUNE_BP) {
     static const int tys[3] = {16, 32, 64};
+    // (timed once where the launches do not depend on it)
+    const bool fixed = bp_height_fixed(b);
+    const double fixed_ms = fixed ? time_bp(b, b->bp_h, reps) : 0.0;
     int best = b->bp_ty;
     double best_ms = -1.0;
     js << ",\"bp\":{\"ms\":{";
     for (int k = 0; k < 3; ++k) {
-      const double ms = time_bp(b, tys[k], reps);
+      const double ms = fixed ? fixed_ms : time_bp(b, tys[k], reps);
       js << (k ? "," : "") << "\"" << tys[k] << "\":" << ms;
       if (best_ms < 0.0 || ms < best_ms) { best = tys[k]; best_ms = ms; }
     }
     js << "},\"choice\":" << best << "}";
-    if (best != b->bp_ty) set_bp_tile(b, best);
+    if (fixed) b->bp_ty = best;
+    else if (best != b->bp_ty) set_bp_tile(b, best);
   }
   js << "}";
   refresh_fp(b);
