@@ -166,7 +166,10 @@ __device__ __forceinline__ void adjoint_tile(const AdjTask& tk, int local, AdjRa
     // lane l (mod 32) of every wave holds angle t0 + l: sine, cosine, first
     // ray of the tile's window, and whether a sample can leave 1 <= jx <= N
     const int t = min(t0 + (lane & (ADJ_AB - 1)), T - 1);
-    const float hs = sc[2 * t], hc = sc[2 * t + 1];
+    const float vs = sc[2 * t], vc = sc[2 * t + 1];
+    // an angle that is not finite covers no pixel: its window holds no ray of the detector
+    const bool fin = fabsf(vs) <= 1.0f && fabsf(vc) <= 1.0f;
+    const float hs = fin ? vs : 0.0f, hc = fin ? vc : 0.0f;
     const float hh = fabsf(hc) + fabsf(hs) + margin;
     const float ymin = fminf(hc * Y0, hc * Y1) + fminf(-hs * X0, -hs * X1);
     const float xmin = fminf(hc * X0, hc * X1) + fminf(hs * Y0, hs * Y1);
@@ -177,7 +180,7 @@ __device__ __forceinline__ void adjoint_tile(const AdjTask& tk, int local, AdjRa
     bool bad = false;
     {
       const int q = tid >> 3, j = tid & 7;  // 8 threads per angle
-      const int jy0 = __shfl(lo, q) + j;
+      const int jy0 = __shfl(fin ? lo : N + 1, q) + j;
       AdjRay<G> v[ADJ_W / 8];
 #pragma unroll
       for (int i = 0; i < G; ++i) {
