@@ -174,7 +174,8 @@ __device__ __forceinline__ void bp_tile(const BPTask& tk, int local, BPLds<TY, R
 #pragma unroll
       for (int i = 0; i < AS * TY; i += NT) {
         const int a = (i + tid) / TY, r = (i + tid) % TY;
-        rt_s[i + tid] = as_global(tk.rowterm)[(size_t)min(a0 + a, T - 1) * N + y0 + r];
+        // rows past the image (not stored) as its last: positions in the window
+        rt_s[i + tid] = as_global(tk.rowterm)[(size_t)min(a0 + a, T - 1) * N + min(y0 + r, N - 1)];
       }
     }
     __syncthreads();
@@ -379,7 +380,7 @@ __global__ __launch_bounds__(64 * BPS_WAVES) void bp_split_kernel(const BPTask* 
     for (int r = 0; r < ROWS; ++r) blk[r] = 0.0f;
     for (int a0 = b * AB; a0 < min(T, (b + 1) * AB); a0 += BPS_AB) {
       const int na = min(BPS_AB, T - a0);
-      // lane l (mod 16) holds angle a0 + l: sine, cosine and window start
+      // lane l (mod BPS_AB) holds angle a0 + l: sine, cosine and window start
       const int t = min(a0 + (lane & (BPS_AB - 1)), T - 1);
       const float hs = sc[2 * t], hc = sc[2 * t + 1];
       const int hlo = (int)floorf(fminf(hs * cx0, hs * cx1) + fminf(hc * cy0, hc * cy1) + m - 1.0f) - 1;

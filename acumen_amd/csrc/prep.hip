@@ -256,14 +256,15 @@ __global__ __launch_bounds__(256) void sum_kernel(const double* __restrict__ par
 
 }  // namespace
 
-constexpr int MED_MIN = 512;  // workgroups of strips of 8 rows: two per CU
+constexpr int MED_MIN = 512;  // workgroups of strips of 8 rows, two per CU: 1000^2 pixels
 
 void launch_median27(int n, const float* l, const float* c, const float* r, float* out, hipStream_t s) {
   const int tx = (n + MED_X - 1) / MED_X;
   auto rows = [&](int k) { return (n + 4 * k - 1) / (4 * k); };
   // strips of 8 rows sort 10 rows for 8 pixels, of 2 rows 4 for 2, but keep
-  // the GPU busier on small images: us per image with 8 and with 2 rows, 6.5
-  // and 6.8 at 1024^2, 4.2 and 4.3 at 700^2, 4.1 and 4.0 at 512^2
+  // the GPU busier on small images: us of the kernel with 8 and with 2 rows, 3.6
+  // and 2.6 at 65^2, 3.9 and 2.8 at 257^2, 4.0 and 3.2 at 512^2, 4.9 and 4.5 at
+  // 700^2, 5.3 and 5.2 at 850^2, 6.5 and 6.5 at 1024^2, 18.9 and 21.0 at 2048^2
   if (tx * rows(8) >= MED_MIN)
     hipLaunchKernelGGL(median27_kernel<8>, dim3(tx * rows(8)), dim3(256), 0, s, n, l, c, r, out, tx);
   else
