@@ -72,6 +72,7 @@ __device__ double block_sum(double v, double* wsum) {
   return r;
 }
 
+static_assert(ADJ_AB == 32, "a bit of a mask per angle");
 constexpr int ADJ_W = 32;  // rays staged per angle and tile: 15 (|c| + |s|) + 4 <= 25.3, and one of margin on each side
 
 // One angle's contribution to one pixel.  (X, Y): the pixel relative to the
@@ -166,10 +167,7 @@ __device__ __forceinline__ void adjoint_tile(const AdjTask& tk, int local, AdjRa
     // lane l (mod 32) of every wave holds angle t0 + l: sine, cosine, first
     // ray of the tile's window, and whether a sample can leave 1 <= jx <= N
     const int t = min(t0 + (lane & (ADJ_AB - 1)), T - 1);
-    const float vs = sc[2 * t], vc = sc[2 * t + 1];
-    // an angle that is not finite covers no pixel: its window holds no ray of the detector
-    const bool fin = fabsf(vs) <= 1.0f && fabsf(vc) <= 1.0f;
-    const float hs = fin ? vs : 0.0f, hc = fin ? vc : 0.0f;
+    const float hs = sc[2 * t], hc = sc[2 * t + 1];
     const float hh = fabsf(hc) + fabsf(hs) + margin;
     const float ymin = fminf(hc * Y0, hc * Y1) + fminf(-hs * X0, -hs * X1);
     const float xmin = fminf(hc * X0, hc * X1) + fminf(hs * Y0, hs * Y1);
@@ -180,7 +178,7 @@ __device__ __forceinline__ void adjoint_tile(const AdjTask& tk, int local, AdjRa
     bool bad = false;
     {
       const int q = tid >> 3, j = tid & 7;  // 8 threads per angle
-      const int jy0 = __shfl(fin ? lo : N + 1, q) + j;
+      const int jy0 = __shfl(lo, q) + j;
       AdjRay<G> v[ADJ_W / 8];
 #pragma unroll
       for (int i = 0; i < G; ++i) {
@@ -205,7 +203,9 @@ __device__ __forceinline__ void adjoint_tile(const AdjTask& tk, int local, AdjRa
     float blk[G];  // FP32 sums over one block of angles, then into acc
 #pragma unroll
     for (int k = 0; k < G; ++k) blk[k] = 0.0f;
-    for (int a = 0; a < na; ++a) {
+    // an angle that is not finite covers no pixel (and has no window in LDS)
+    for (unsigned live = (unsigned)__ballot(hh <= 4.0f) & (~0u >> (ADJ_AB - na)); live != 0; live &= live - 1) {
+      const int a = __builtin_ctz(live);
       const float s = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(hs), a));
       const float c = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(hc), a));
       const float hw = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(hh), a));
