@@ -225,16 +225,19 @@ __device__ __forceinline__ void adjoint_tile(const AdjTask& tk, int local, AdjRa
 // W: the most slices of a task.  Each task runs at its own width, so a slice
 // without a partner costs what it would in a launch of single slices: 5 equal
 // and 20 different slices of 513^2 x 360 (loss and gradients) take 6.5 ms, 25
-// different ones 6.95, with every task at the width of the widest 7.85.  Blocks
-// go round-robin over the XCDs, the tasks of the longest first: with
-// contiguous shares of the blocks the XCD of the wide tasks was the last (9
-// equal slices 1.65 ms instead of 1.47, eight sizes from 65^2 x 1000 to
-// 600^2 x 90 1.44 instead of 1.16), and sharing an L2 gains nothing here (25
-// different slices the same).
+// different ones 6.95, with every task at the width of the widest 7.85.
+// mixed: tasks whose tiles take unequal times, the longest first, go
+// round-robin over the XCDs: with contiguous shares of the blocks the XCD of
+// the wide tasks is the last (9 equal slices 1.62 ms instead of 1.50, eight
+// sizes from 65^2 x 1000 to 600^2 x 90 1.48 instead of 1.19, the 25 slices
+// above 6.9).  Others keep neighbouring tiles on one XCD (360^2 x 360 255 us,
+// 286 round-robin; 16 different 65^2 x 48 400, 418; 513^2 x 360 397, 393).
 template <int W>
-__global__ __launch_bounds__(ADJ_T * ADJ_T) void adjoint_kernel(const AdjTask* __restrict__ tasks, int ntasks) {
+__global__ __launch_bounds__(ADJ_T * ADJ_T) void adjoint_kernel(const AdjTask* __restrict__ tasks, int ntasks,
+                                                                int nblocks, bool mixed) {
   __shared__ AdjRay<W> P[ADJ_AB * ADJ_W];
-  const int gb = (int)blockIdx.x;
+  const int gb = mixed ? (int)blockIdx.x : xcd_remap(blockIdx.x, gridDim.x);
+  if (gb >= nblocks) return;  // uniform per workgroup
   const AdjTask& tk = tasks[find_by<AdjTask, &AdjTask::block_begin>(tasks, ntasks, gb)];
   const int local = gb - tk.block_begin;
   const int width = adj_width(tk.n);
@@ -376,19 +379,21 @@ std::vector<std::vector<int>> adj_groups(const std::vector<int>& geo, const std:
 
 void launch_adjoint(const AdjTask* d_tasks, const std::vector<AdjTask>& tasks, hipStream_t s) {
   int most = 1, blocks = 0;
+  bool mixed = false;
   for (const AdjTask& t : tasks) {
     if (t.n < 1 || t.n > ADJ_GROUP || t.block_begin != blocks) throw Error("adjoint tasks do not match the launch");
     most = std::max(most, adj_width(t.n));
+    mixed = mixed || t.T != tasks[0].T || adj_width(t.n) != adj_width(tasks[0].n);
     blocks += t.ntx * t.ntx;
   }
   if (blocks <= 0) return;
-  const dim3 grid(blocks), wg(ADJ_T * ADJ_T);
+  const dim3 grid(xcd_grid(blocks)), wg(ADJ_T * ADJ_T);
   const int n = (int)tasks.size();
   switch (most) {
-    case 1: hipLaunchKernelGGL(adjoint_kernel<1>, grid, wg, 0, s, d_tasks, n); break;
-    case 2: hipLaunchKernelGGL(adjoint_kernel<2>, grid, wg, 0, s, d_tasks, n); break;
-    case 4: hipLaunchKernelGGL(adjoint_kernel<4>, grid, wg, 0, s, d_tasks, n); break;
-    default: hipLaunchKernelGGL(adjoint_kernel<8>, grid, wg, 0, s, d_tasks, n); break;
+    case 1: hipLaunchKernelGGL(adjoint_kernel<1>, grid, wg, 0, s, d_tasks, n, blocks, mixed); break;
+    case 2: hipLaunchKernelGGL(adjoint_kernel<2>, grid, wg, 0, s, d_tasks, n, blocks, mixed); break;
+    case 4: hipLaunchKernelGGL(adjoint_kernel<4>, grid, wg, 0, s, d_tasks, n, blocks, mixed); break;
+    default: hipLaunchKernelGGL(adjoint_kernel<8>, grid, wg, 0, s, d_tasks, n, blocks, mixed); break;
   }
 }
 
