@@ -874,8 +874,8 @@ Range sw_range(acu_batch* b, int sl) { return sl < 0 ? Range{0, b->sw_total} : R
 // The ramp filter of all slices (sl < 0) or one, in one arithmetic.  FP64
 // goes by FFT for every slice within its length limit (N <= 4097: a row's
 // points fit LDS twice over) and by the Toeplitz product on the FP64 matrix
-// cores beyond.  The FFT is faster at every size within it: ms by FFT and as
-// a product, 0.008 and 0.033 at 257^2 x 180, 0.032 and 0.27 at 2049^2 x 1500.
+// cores beyond.  The FFT is faster at every size within it: us by FFT and as
+// a product, 7 and 23 at 257^2 x 180, 230 and 2285 at 8 x 2049^2 x 1500.
 // The slices beyond share a launch: 8 x 4500^2 x 60 are 71 workgroups each
 // for 256 CUs, and FBP of them takes 1.66 ms so, 6.1 with a launch for each.
 void launch_ramp_any(acu_batch* b, const RFSet& rf, int sl, int variant) {

@@ -43,12 +43,13 @@
 //    wait into a wait for all).  8 x 2049^2 x 1500 6.33 to 5.75 ms, 2 x
 //    1025^2 x 720 at TY = 16 360 to 260 us;
 //  * a pair of slices of one geometry (G = 2, REFPOS) shares positions,
-//    weights and offsets: 4.5 VALU instructions an update instead of 7.  The
+//    weights and offsets: 4.2 VALU instructions an update instead of 7.  The
 //    windows are two arrays read by two ds_read_b64 (2.2 clocks each; one
 //    ds_read2st64_b64 takes 8, a b128 of interleaved pairs 5.9 with its bank
 //    conflicts), staged 16 angles at a time so that 5 workgroups fit a CU.
-//    8 x 2049^2 x 1500 5.75 to 5.07 ms (0.63 ms a slice), 4 x 1025^2 x 720
-//    490 to 390 us, and 4.79 with five waves per SIMD instead of four;
+//    8 x 2049^2 x 1500 5.75 to 5.0 ms, and 4.6 with five waves per SIMD instead
+//    of four: 1.45 wave-instructions per CU and clock, LDS active 75% of the
+//    cycles, at 1.83 GHz: the power limit is near as well;
 //  * each 32-angle block is summed separately and then added;
 //  * tiles whose mask is identically zero (by 64 x 16 sub-tiles) only store
 //    zeros.

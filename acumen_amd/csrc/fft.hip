@@ -31,13 +31,12 @@
 // barriers.  A 2049^2 x 1500 slice is 12.6 GFLOP as a Toeplitz product and
 // 0.45 GFLOP this way.  The result is the exact one but for its rounding to
 // FP32, as the Toeplitz product's on the FP64 matrix cores is (filter.hip):
-// both are 2.5e-8 from FP64 on noise at N = 6..4097.  Measured on MI355X, ms
-// per launch: 8 x 2049^2 x 1500 0.207 (product 2.18; the radix-2 FP32
-// transform of row pairs this replaces 0.406), 4 x 1025^2 x 720 0.030
-// (product 0.21), 257^2 x 180 0.008 (product 0.033).  The same passes in
-// FP32 took 0.144 with products of FP32 twiddles, but 1.2x the error of that
-// radix-2 transform; without the extra error they took 0.202, so there is no
-// FP32 form.
+// both are 2.5e-8 from FP64 on noise at N = 6..4097.  Kernel times on MI355X,
+// us, this | the radix-2 FP32 transform of row pairs that it replaces | the
+// product: 8 x 2049^2 x 1500 230 | 437 | 2285, 4 x 1025^2 x 720 35 | 54 | 208, 257^2 x
+// 180 7 | 7 | 23.  The same passes in FP32 took 164 at 8 x 2049^2 x 1500 with
+// products of FP32 twiddles, but 1.2x the error of that radix-2 transform;
+// without the extra error they took 202, so there is no FP32 form.
 #include "acu_internal.hpp"
 
 #include <algorithm>
@@ -142,7 +141,7 @@ __device__ void direct_row(const float* __restrict__ h, const float* __restrict_
 
 // A row that holds infinities or NaN: the plain sum's result follows from
 // those values alone, as the finite terms cannot overflow FP64.  The tap at
-// distance 0 is positive, every other one negative (tv_hpc.F90:49-54), and
+// distance 0 is positive, every other one negative (tv_hpc.F90:53-56), and
 // none is zero: a NaN makes every output NaN, and an infinity is an infinity
 // of its own sign at its place and of the other sign everywhere else.  Each
 // wave looks through the row itself (its rt threads, if fewer than 64 have

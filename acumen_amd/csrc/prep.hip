@@ -67,9 +67,10 @@ struct Float3Ops {
 // pixel (and 27 for each of the rows above and below its K) instead of the
 // 306 of the network for 27 loose values.  That network stays for waves whose
 // values hold a NaN, where the result depends on the order of comparisons.
-// Bound by its traffic (three images in, one out: 67 MB, 3.5 TB/s) beside
-// about 80 instructions a pixel. us per 2048^2 image: 19, 21 with the rows
-// staged in LDS, 57 with the network in every pixel.
+// Bound by its traffic (three images in, one out: 67 MB, 12 us at the ingest
+// kernels' rate) and its sorting (about 10 us of half-rate min, med and max
+// issue), which a wave does one after the other. us per 2048^2 image: 19, 21
+// with the rows staged in LDS, 57 with the network in every pixel.
 constexpr int MED_X = 62;
 
 __device__ __forceinline__ float lane_prev(float v) {  // wave_shr:1: lane i reads lane i - 1

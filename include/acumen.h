@@ -165,7 +165,9 @@ int acu_ramp_dev(acu_batch *b, int slice, float *out_dev, const float *sino_dev)
 int acu_backproject_dev(acu_batch *b, int slice, float *img_dev, const float *filtered_dev);
 
 /* Host-memory forms of the reference subroutines on a single-slice plan
- * (slice 0).  Synchronous. */
+ * (slice 0).  Synchronous.  The first call of acu_radon, acu_iradon or
+ * acu_radon_adjoint allocates an image and a sinogram of that slice on the
+ * device, 4 (N^2 + N*T) bytes, which the batch keeps until it is destroyed. */
 int acu_radon(acu_batch *b, float *sino_host, const float *img_host);
 int acu_iradon(acu_batch *b, float *img_host, const float *sino_host);
 int acu_get_slice(acu_batch *b, const float *f_host, float *img_fbp_host);
@@ -187,13 +189,15 @@ int acu_tvopt(acu_batch *b, const float *f_host, float mu, float lambda, int nou
  * calls.  It also times the ramp-filter arithmetics that meet the FBP and
  * TV accuracy bar (ACU_RAMP_FP64, _FP32, _BF16X6, _FFT; not _BF16X3) on the
  * whole batch and keeps the fastest, and the backprojection tile height
- * (below) on the whole batch.  report (may be NULL) receives a JSON summary
- * of the timings and choices, truncated to cap bytes including the
- * terminating NUL.  The choices follow measured times, so two runs may
- * choose differently; projector variants 4 and 8 agree bit for bit where
- * their boxes fit, while the ramp arithmetics and the tile heights differ
- * at FP32 rounding level.  A caller that needs identical bits from run to
- * run stores the choices and reapplies them with the setters.  The
+ * (below) on the whole batch.  Candidates that are the same launch (_FFT is
+ * _FP64's; the heights of batches of few tiles) are timed once and reported
+ * with one time, of which the first is the choice.  report (may be NULL)
+ * receives a JSON summary of the timings and choices, truncated to cap bytes
+ * including the terminating NUL.  The choices follow measured times, so two
+ * runs may choose differently; projector variants 4 and 8 agree bit for bit
+ * where their boxes fit, while the ramp arithmetics and the tile heights
+ * differ at FP32 rounding level.  A caller that needs identical bits from run
+ * to run stores the choices and reapplies them with the setters.  The
  * getter returns the variant, or -ACU_ERR_ARG for a bad slice; the setter
  * lets a caller reapply a stored choice. */
 int acu_batch_autotune(acu_batch *b, int reps, char *report, int cap);

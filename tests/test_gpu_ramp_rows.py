@@ -12,7 +12,7 @@ pytestmark = pytest.mark.gpu
 
 
 def taps(N):
-    """The reference's FP32 taps at distances -(N-1)..N-1 (tv_hpc.F90:49-56), one rounding per operation."""
+    """The reference's FP32 taps at distances -(N-1)..N-1 (tv_hpc.F90:53-56), one rounding per operation."""
     k = np.arange(-(N - 1), N)
     q = (4 * k * k - 1).astype(np.float32)
     pi = np.float32(np.pi)
