@@ -782,6 +782,7 @@ void settle_geometries(acu_batch* b) {
   b->geo = find_geometries(b);
   std::vector<int> partner = find_pairs(b);
   if (!b->bp_built || partner != b->bp_partner) {
+    b->ctx->sync();  // launches since the change may still read the arrays that are replaced
     b->bp_built = false;
     b->bp_partner = std::move(partner);
     assign_bp_pairs(b);
