@@ -439,15 +439,17 @@ int bp_split_tiles(int N) { return bp_tiles_x(N) * ((N + 15) / 16) * 2; }
 
 // us per FBP (host call and ramp included), MI355X: this kernel | 64 x 16 |
 // 64 x 32 tiles of bp_kernel, by the launch's 64 x 8 tiles:
-//   20 (65^2) x 48 21 | 19 | 24, x 100 22 | 26 | 36, x 180 23 | 36 | 53;
-//   68 (129^2) x 64 22 | 21 | 28, x 90 23 | 25 | 34;
-//   170 (257^2) x 60 22 | 21 | 27, x 180 24 | 38 | 54;
-//   594 (513^2) x 360 64 | 66 | 97;      680 (4 x 257^2) x 180 39 | 40 | 56;
-//   1274 (769^2) x 600 148 | 124 | 158;  2720 (16 x 257^2) x 180 82 | 65 | 80
+//   20 (65^2) x 48 19 | 16 | 21, x 100 19 | 24 | 33, x 180 21 | 34 | 50;
+//   54 (129^2) x 64 20 | 19 | 25, x 90 20 | 23 | 31;
+//   170 (257^2) x 60 19 | 18 | 24, x 180 21 | 35 | 51;
+//   594 (513^2) x 360 58 | 61 | 93;      680 (4 x 257^2) x 180 34 | 35 | 51;
+//   1274 (769^2) x 600 133 | 111 | 150;  2720 (16 x 257^2) x 180 74 | 54 | 66
 // and 64 x 16 | 64 x 32 | 64 x 64 tiles of bp_kernel:
-//   2210 (1025^2) x 720 197 | 236 | 250; 4752 (8 x 513^2) x 720 290 | 343 | 382;
-//   4850 (1537^2) x 900 407 | 435 | 433; 6630 (3 x 1025^2) x 720 411 | 416 | 376;
-//   8840 (4 x 1025^2) x 720 454 | 432 | 400; 8514 (2049^2) x 1500 935 | 944 | 955
+//   2210 (1025^2) x 720 176 | 223 | 245; 4752 (8 x 513^2) x 720 251 | 330 | 371;
+//   4850 (1537^2) x 900 344 | 394 | 418; 5096 (4 x 769^2) x 600 215 | 287 | 316.
+// From about there on taller tiles win in part, so the height is as set (the
+// autotuner's to choose): 6630 (3 x 1025^2) x 720 335 | 372 | 344; 8514 (2049^2) x
+// 1500 832 | 892 | 927; 8840 (4 x 1025^2) x 720 414 | 396 | 373
 bool bp_use_split(int tiles, int T) { return tiles <= 640 && T > 64; }
 int bp_launch_height(int tiles, int ty) { return tiles <= 5200 ? 16 : ty; }
 // us per FBP without | with pairs, by the launch's 64 x 8 tiles (heights 16 up
